@@ -84,6 +84,57 @@ struct gfsx_ctx {
         return events[events_used++].data();
     }
 
+    // Workspace of the point calls (gfsx_g2p*, gfsx_advect*), which take no
+    // other: calls from several threads enqueue one after the other, and a
+    // call on another stream waits for the last one's work.
+    struct PointWork {
+        std::mutex mu;
+        void *buf = nullptr;
+        size_t bytes = 0;
+        hipEvent_t done = nullptr;   // after the last call that used buf
+    } points;
+
+    // order 0: out = the MAC sample at pos; 1..4: a Runge-Kutta step from pos
+    void point_call(const float *pos, int64_t n, const gfsx::MacGrid &g, int order, double dt,
+                    int stencil, float *out) {
+        auto direct = [&] {
+            if (order == 0) gfsx::g2p(pos, n, g, stencil, out, stream);
+            else gfsx::advect(pos, n, g, order, dt, stencil, out, stream);
+        };
+        if (!gfsx::points_by_brick(n, g.ni, g.nj, g.nk, order, stencil)) return direct();
+        // a captured call must not depend on memory that a later call may
+        // replace: it takes the direct kernels
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return direct();
+        }
+        std::lock_guard<std::mutex> lock(points.mu);
+        const size_t need = gfsx::points_workspace(n, g.ni, g.nj, g.nk);
+        if (points.bytes < need) {
+            // (another thread's capture is left alone by this allocation)
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (!points.done) (void)hipEventCreateWithFlags(&points.done, hipEventDisableTiming);
+            else (void)hipEventSynchronize(points.done);
+            if (points.buf) (void)hipFree(points.buf);
+            points.buf = nullptr;
+            points.bytes = 0;
+            const bool got = points.done && hipMalloc(&points.buf, need) == hipSuccess;
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (!got) {   // no memory for it: the direct kernels need none
+                points.buf = nullptr;
+                (void)hipGetLastError();
+                return direct();
+            }
+            points.bytes = need;
+        } else {
+            GFSX_HIP(hipStreamWaitEvent(stream, points.done, 0));
+        }
+        gfsx::points_run(points.buf, pos, n, g, order, dt, stencil, out, stream);
+        GFSX_HIP(hipEventRecord(points.done, stream));
+    }
+
     // Device workspace, grown on demand and kept until gfsx_destroy.
     void *get(int slot, size_t nbytes) {
         nbytes = std::max<size_t>(nbytes, 256);
@@ -217,6 +268,8 @@ struct gfsx_ctx {
             for (auto &x : e) (void)hipEventDestroy(x);
         for (auto &t : tables)
             if (t.dev) (void)hipFree(t.dev);
+        if (points.buf) (void)hipFree(points.buf);
+        if (points.done) (void)hipEventDestroy(points.done);
         if (own_stream) (void)hipStreamDestroy(own_stream);
     }
 };
@@ -904,7 +957,7 @@ void gfsx_g2p_device(gfsx_ctx *ctx, const float *pos, int64_t n,
         require(stencil == GFSX_TRILINEAR || stencil == GFSX_TRICUBIC, "gfsx: unknown stencil");
         require(u && v && w, "gfsx: null velocity grid");
         require(n == 0 || out, "gfsx: null output");
-        gfsx::g2p(pos, n, mac_grid(u, v, w, ni, nj, nk, dx), stencil, out, ctx->stream);
+        ctx->point_call(pos, n, mac_grid(u, v, w, ni, nj, nk, dx), 0, 0.0, stencil, out);
     });
 }
 
@@ -929,7 +982,7 @@ void gfsx_g2p(gfsx_ctx *ctx, const float *pos, int64_t n, const float *u,
             copy_in(dg[c], hg[c], sizeof(float) * m, s);
         }
         copy_in(dpos, pos, sizeof(float) * 3 * n, s);
-        gfsx::g2p(dpos, n, mac_grid(dg[0], dg[1], dg[2], ni, nj, nk, dx), stencil, dout, s);
+        ctx->point_call(dpos, n, mac_grid(dg[0], dg[1], dg[2], ni, nj, nk, dx), 0, 0.0, stencil, dout);
         copy_out(out, dout, sizeof(float) * 3 * n, s);
         GFSX_HIP(hipStreamSynchronize(s));
     });
@@ -949,8 +1002,7 @@ void gfsx_advect_device(gfsx_ctx *ctx, int order, const float *pos, int64_t n,
         require(std::isfinite(dt), "gfsx: dt must be finite");
         require(u && v && w, "gfsx: null velocity grid");
         require(n == 0 || out, "gfsx: null output");
-        gfsx::advect(pos, n, mac_grid(u, v, w, ni, nj, nk, dx), order, dt, stencil, out,
-                     ctx->stream);
+        ctx->point_call(pos, n, mac_grid(u, v, w, ni, nj, nk, dx), order, dt, stencil, out);
     });
 }
 
@@ -978,8 +1030,8 @@ void gfsx_advect(gfsx_ctx *ctx, int order, const float *pos, int64_t n,
             copy_in(dg[c], hg[c], sizeof(float) * m, s);
         }
         copy_in(dpos, pos, sizeof(float) * 3 * n, s);
-        gfsx::advect(dpos, n, mac_grid(dg[0], dg[1], dg[2], ni, nj, nk, dx), order, dt,
-                     stencil, dout, s);
+        ctx->point_call(dpos, n, mac_grid(dg[0], dg[1], dg[2], ni, nj, nk, dx), order, dt, stencil,
+                        dout);
         copy_out(out, dout, sizeof(float) * 3 * n, s);
         GFSX_HIP(hipStreamSynchronize(s));
     });

@@ -128,6 +128,16 @@ struct RkConsts {
     float half, three_q, full, sixth, ninth;
 };
 
+inline RkConsts rk_consts(double dt) {
+    RkConsts c;
+    c.half = (float)(0.5 * dt);
+    c.three_q = (float)(0.75 * dt);
+    c.full = (float)dt;
+    c.sixth = (float)(dt / 6.0f);
+    c.ninth = (float)(dt / 9.0f);
+    return c;
+}
+
 // ParticleAdvector::_RK1.._RK4 (particleadvector.cpp:1045-1078) in FP32
 // vec3 arithmetic; the step sizes are the reference's FP32 casts.
 template <int ST>

@@ -407,6 +407,29 @@ void g2p(const float *pos, int64_t n, const MacGrid &g, int stencil,
 void advect(const float *pos, int64_t n, const MacGrid &g, int order,
             double dt, int stencil, float *out, hipStream_t s);
 
+// The same over bricks of points staged in LDS (gfsx_points.hip; the same
+// bits).  points_by_brick: whether a call of n points takes that path; work
+// holds points_workspace bytes of device memory; order 0 is the sample,
+// 1..4 the Runge-Kutta step.
+//
+// Where the line lies (us per call, direct / bricked, particles 8 per cell in
+// cell order, and shuffled): tricubic RK4 268k points 122 / 95 and 216 / 105
+// (131k: 74 / 83 and 85 / 89); tricubic sample 1M 69 / 74 and 204 / 87
+// (268k: 30 / 50 and 59 / 56); trilinear RK4 1M 58 / 73 and 196 / 85 (268k:
+// 20 / 52 and 54 / 60); a trilinear sample or a one- or two-sample step gains
+// only when shuffled (8M: 104 / 241 and 1260 / 458) and stays direct.  Below
+// about a hundred points per brick of the grid the histograms and the boxes
+// cost more than they save (256^3, 1M points spread over it, tricubic RK4:
+// 734 / 989).
+constexpr int64_t kPointsPerBrick = 96;
+constexpr int64_t kPointsMinLinear = (int64_t)1 << 20;
+constexpr int64_t kPointsMinCubicRk = 200000;
+constexpr int64_t kPointsMinCubic = (int64_t)1 << 19;
+bool points_by_brick(int64_t n, int ni, int nj, int nk, int order, int stencil);
+size_t points_workspace(int64_t n, int ni, int nj, int nk);
+void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int order, double dt,
+                int stencil, float *out, hipStream_t s);
+
 // Face rows along x that one wave of the combine takes in turn: enough for
 // about 256 faces, so that short rows share a wave's set-up.
 __host__ __device__ inline int combine_rows(int nx) { return nx < 256 ? 256 / nx : 1; }

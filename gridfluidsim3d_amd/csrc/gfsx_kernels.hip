@@ -775,16 +775,6 @@ __global__ __launch_bounds__(kBlock) void k_advect(const float *pos, int64_t n,
     out[3 * p + 2] = x1[2];
 }
 
-static RkConsts rk_consts(double dt) {
-    RkConsts c;
-    c.half = (float)(0.5 * dt);
-    c.three_q = (float)(0.75 * dt);
-    c.full = (float)dt;
-    c.sixth = (float)(dt / 6.0f);
-    c.ninth = (float)(dt / 9.0f);
-    return c;
-}
-
 void advect(const float *pos, int64_t n, const MacGrid &g, int order,
             double dt, int stencil, float *out, hipStream_t s) {
     if (n <= 0) return;

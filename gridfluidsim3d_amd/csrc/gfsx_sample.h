@@ -173,6 +173,42 @@ __device__ __forceinline__ float sample_comp(const float *__restrict__ f,
     return tricubic(f, w, h, d, i, j, k, tx, ty, tz);
 }
 
+// sample_comp, the same bits, for kernels that sample straight from memory:
+// a stencil that lies inside the array reads each row along x with one load
+// (2 or 4 floats from any 4-byte address) and no clamps, a quarter of the
+// loads; any other stencil takes sample_comp.
+template <int ST>
+__device__ __forceinline__ float sample_comp_rows(const float *__restrict__ f, int w, int h, int d,
+                                                  int i, int j, int k, float tx, float ty,
+                                                  float tz) {
+    constexpr int S = ST;
+    if (i >= S && j >= S && k >= S && i + 1 + S < w && j + 1 + S < h && k + 1 + S < d) {
+        const float *b = f + ((uint32_t)(i - S) +
+                              (uint32_t)w * ((uint32_t)(j - S) + (uint32_t)h * (uint32_t)(k - S)));
+        const uint32_t sj = (uint32_t)w, sk = (uint32_t)w * (uint32_t)h;
+        if (ST == 0) {
+            typedef float Row __attribute__((ext_vector_type(2), aligned(4)));
+            typedef const __attribute__((address_space(1))) Row GRow;
+            const Row r00 = *(GRow *)b, r10 = *(GRow *)(b + sj);
+            const Row r01 = *(GRow *)(b + sk), r11 = *(GRow *)(b + sk + sj);
+            const float c00 = fmaf(tx, r00[1] - r00[0], r00[0]);
+            const float c10 = fmaf(tx, r10[1] - r10[0], r10[0]);
+            const float c01 = fmaf(tx, r01[1] - r01[0], r01[0]);
+            const float c11 = fmaf(tx, r11[1] - r11[0], r11[0]);
+            const float c0 = fmaf(ty, c10 - c00, c00);
+            const float c1 = fmaf(ty, c11 - c01, c01);
+            return fmaf(tz, c1 - c0, c0);
+        }
+        typedef float Row __attribute__((ext_vector_type(4), aligned(4)));
+        typedef const __attribute__((address_space(1))) Row GRow;
+        Row r[16];
+#pragma unroll
+        for (int m = 0; m < 16; m++) r[m] = *(GRow *)(b + sj * (uint32_t)(m & 3) + sk * (uint32_t)(m >> 2));
+        return tricubic_sum([&](int mi, int mj, int mk) { return r[4 * mk + mj][mi]; }, tx, ty, tz);
+    }
+    return sample_comp<ST>(f, w, h, d, i, j, k, tx, ty, tz);
+}
+
 // Velocity of grid g (and, when OLD, of the same-shaped grid o0,o1,o2) at
 // (x,y,z): MACVelocityField::evaluateVelocityAtPosition
 // {,Linear} (macvelocityfield.cpp:549-575), (0,0,0) outside the grid.
@@ -191,13 +227,13 @@ __device__ __forceinline__ void sample_mac(const MacGrid &g, const float *o0,
     const AxisCoords cy = axis_coords(y, g.inv_dx);
     const AxisCoords cz = axis_coords(z, g.inv_dx);
     const int ni = g.ni, nj = g.nj, nk = g.nk;
-    out[0] = sample_comp<ST>(g.f[0], ni + 1, nj, nk, cx.ia, cy.ib, cz.ib, cx.ta, cy.tb, cz.tb);
-    out[1] = sample_comp<ST>(g.f[1], ni, nj + 1, nk, cx.ib, cy.ia, cz.ib, cx.tb, cy.ta, cz.tb);
-    out[2] = sample_comp<ST>(g.f[2], ni, nj, nk + 1, cx.ib, cy.ib, cz.ia, cx.tb, cy.tb, cz.ta);
+    out[0] = sample_comp_rows<ST>(g.f[0], ni + 1, nj, nk, cx.ia, cy.ib, cz.ib, cx.ta, cy.tb, cz.tb);
+    out[1] = sample_comp_rows<ST>(g.f[1], ni, nj + 1, nk, cx.ib, cy.ia, cz.ib, cx.tb, cy.ta, cz.tb);
+    out[2] = sample_comp_rows<ST>(g.f[2], ni, nj, nk + 1, cx.ib, cy.ib, cz.ia, cx.tb, cy.tb, cz.ta);
     if (OLD) {
-        out_old[0] = sample_comp<ST>(o0, ni + 1, nj, nk, cx.ia, cy.ib, cz.ib, cx.ta, cy.tb, cz.tb);
-        out_old[1] = sample_comp<ST>(o1, ni, nj + 1, nk, cx.ib, cy.ia, cz.ib, cx.tb, cy.ta, cz.tb);
-        out_old[2] = sample_comp<ST>(o2, ni, nj, nk + 1, cx.ib, cy.ib, cz.ia, cx.tb, cy.tb, cz.ta);
+        out_old[0] = sample_comp_rows<ST>(o0, ni + 1, nj, nk, cx.ia, cy.ib, cz.ib, cx.ta, cy.tb, cz.tb);
+        out_old[1] = sample_comp_rows<ST>(o1, ni, nj + 1, nk, cx.ib, cy.ia, cz.ib, cx.tb, cy.ta, cz.tb);
+        out_old[2] = sample_comp_rows<ST>(o2, ni, nj, nk + 1, cx.ib, cy.ib, cz.ia, cx.tb, cy.tb, cz.ta);
     }
 }
 
