@@ -47,7 +47,7 @@ enum Slot {
     S_P_TILE, S_P_TFLAG,
     S_K_COUNT, S_K_START, S_K_PSTART, S_K_RSTART, S_K_RUNREC, S_K_NRUNS, S_K_LIST, S_K_LIST2,
     S_K_RUNBASE, S_K_MID, S_K_HUGE, S_K_LCOUNT, S_K_SCAN, S_K_FLUID, S_K_SSLOT,
-    S_K_SCOUNT, S_K_JR, S_K_RLEN, S_K_NCHUNK,
+    S_K_SCOUNT, S_SPLAT, S_K_JR, S_K_RLEN, S_K_NCHUNK,
     NSLOT
 };
 
@@ -416,6 +416,11 @@ void p2g_device_impl(gfsx_ctx *c, const float *pos, const float *val,
     bg.inv_dx = 1.0 / dx;
     bg.nbin = (uint32_t)nbin;
     ng.dx_f = (float)dx;
+    if (gfsx::splat_by_brick(n, bg, r)) {
+        gfsx::splat_run(c->get(S_SPLAT, gfsx::splat_workspace(n, bg)), pos, val, n, bg, ng, radius,
+                        dx, S, W, c->stream);
+        return;
+    }
     std::vector<gfsx::SceneDesc> t(1);
     std::memset(t.data(), 0, sizeof(gfsx::SceneDesc));
     t[0].aos = pos;

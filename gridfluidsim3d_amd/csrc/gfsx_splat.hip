@@ -1,0 +1,407 @@
+// gfsx_splat.hip -- P2G of point arrays onto a node grid for any radius
+// (CLScalarField::addPointValues / addPoints, clscalarfield.cpp:68-301) on
+// gfx950: a stable sort of the points by cell whose records the gather reads
+// in sequence.
+//
+// The bin cells (gfsx_internal.h, BinGrid) are grouped in bricks of 8^3; the
+// sort places brick after brick, cell after cell inside a brick (i fastest)
+// and point index order inside a cell:
+//
+//   1. k_sp_count / k_sp_starts / k_sp_place: every point's record (x, y, z,
+//      value; 16 bytes) and index into its brick's range, by histograms of
+//      the bricks in LDS (the order inside a brick is not fixed yet).
+//   2. k_sp_cells: one work-group per brick counts its cells in LDS, and
+//      writes each record to its cell at the rank of its index there; the
+//      512 cell starts go to a table (brick * 512 + cell, so a cell's end is
+//      the next entry).
+//   3. k_sp_gather: every node sums the records of its candidate cells, rows
+//      in (k, j) order, then cell order, then index order: a fixed order, so
+//      results are bit-identical run to run.
+//
+// Bound: the gather by L2 reads (a lane's records are 16 bytes apart, a
+// wave's spread over a cache line per cell), the passes before it by
+// scattered memory.  The gather through a permutation of unsorted AoS points
+// read 16 bytes from a random place per candidate (64-odd per node at 8
+// points per cell).  3.85M shuffled points with values on 131x97x113, R = dx,
+// with weights, per component: 1.44 -> 0.33 ms (gather 1.14 -> 0.10, sort
+// 0.30 -> 0.20); 0.73M points on 160x121x144, R = 2.5 dx: 0.94 -> 0.41 ms.
+
+#include "gfsx_internal.h"
+#include "gfsx_device.h"
+
+#include <algorithm>
+
+namespace gfsx {
+
+namespace {
+
+constexpr int SNT = 1024;             // threads of the count and place kernels
+constexpr int SITEMS = 16;            // most points per thread there
+constexpr uint32_t kMaxBricks = 40000;   // histogram words that fit a CU's 160 KB of LDS
+constexpr uint32_t CAP = 6144;        // points of a brick ordered in LDS
+constexpr int CELLS = 512;            // cells of a brick
+
+struct SplatGrid {
+    BinGrid bg;
+    int gb[3];          // bricks per axis
+    uint32_t nbrick;    // their number; also the bin of the points outside the bins
+};
+
+// A point's brick and its cell there; bin_of's arithmetic.
+__device__ __forceinline__ uint32_t brick_of(const SplatGrid &g, float x, float y, float z,
+                                             uint32_t &cell) {
+    const float px = x - g.bg.off[0], py = y - g.bg.off[1], pz = z - g.bg.off[2];
+    const double fi = floor((double)px * g.bg.inv_dx) + g.bg.pad[0];
+    const double fj = floor((double)py * g.bg.inv_dx) + g.bg.pad[1];
+    const double fk = floor((double)pz * g.bg.inv_dx) + g.bg.pad[2];
+    cell = 0;
+    if (!(fi >= 0.0 && fj >= 0.0 && fk >= 0.0 && fi < (double)g.bg.b[0] &&
+          fj < (double)g.bg.b[1] && fk < (double)g.bg.b[2]))
+        return g.nbrick;
+    const uint32_t i = (uint32_t)fi, j = (uint32_t)fj, k = (uint32_t)fk;
+    cell = (i & 7u) | ((j & 7u) << 3) | ((k & 7u) << 6);
+    return (i >> 3) + (uint32_t)g.gb[0] * ((j >> 3) + (uint32_t)g.gb[1] * (k >> 3));
+}
+
+__global__ __launch_bounds__(SNT) void k_sp_count(SplatGrid g, const float *__restrict__ pos,
+                                                  int64_t n, int items,
+                                                  uint32_t *__restrict__ count) {
+    extern __shared__ uint32_t s_hist[];
+    for (uint32_t b = threadIdx.x; b <= g.nbrick; b += SNT) s_hist[b] = 0u;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * items * SNT + threadIdx.x;
+    for (int m = 0; m < items; m++) {
+        const int64_t p = base + (int64_t)m * SNT;
+        uint32_t cell;
+        if (p < n)
+            atomicAdd(&s_hist[brick_of(g, gld(pos, 3 * p), gld(pos, 3 * p + 1), gld(pos, 3 * p + 2),
+                                       cell)], 1u);
+    }
+    __syncthreads();
+    for (uint32_t b = threadIdx.x; b <= g.nbrick; b += SNT) {
+        const uint32_t c = s_hist[b];
+        if (c) atomicAdd(&count[b], c);
+    }
+}
+
+// One work-group: first[b] (b = 0..nbrick+1) and the placing cursors.
+__global__ __launch_bounds__(SNT) void k_sp_starts(uint32_t nbrick, const uint32_t *__restrict__ count,
+                                                   uint32_t *__restrict__ first,
+                                                   uint32_t *__restrict__ cursor) {
+    __shared__ uint32_t s_w[SNT / 64];
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    uint32_t at = 0;
+    for (uint32_t b0 = 0; b0 <= nbrick; b0 += SNT) {
+        const uint32_t b = b0 + (uint32_t)t;
+        const uint32_t c = b <= nbrick ? count[b] : 0u;
+        const uint32_t inc = wave_inclusive_sum(c);
+        if (lane == 63) s_w[wid] = inc;
+        __syncthreads();
+        uint32_t s = at + inc - c;
+        for (int w = 0; w < SNT / 64; w++) {
+            const uint32_t v = s_w[w];
+            if (w < wid) s += v;
+            at += v;
+        }
+        if (b <= nbrick) {
+            first[b] = s;
+            cursor[b] = s;
+        }
+        __syncthreads();
+    }
+    if (t == 0) first[nbrick + 1] = at;
+}
+
+__global__ __launch_bounds__(SNT) void k_sp_place(SplatGrid g, const float *__restrict__ pos,
+                                                  const float *__restrict__ val, int64_t n,
+                                                  int items, uint32_t *__restrict__ cursor,
+                                                  float4 *__restrict__ rec,
+                                                  uint32_t *__restrict__ idx) {
+    extern __shared__ uint32_t s_hist[];
+    for (uint32_t b = threadIdx.x; b <= g.nbrick; b += SNT) s_hist[b] = 0u;
+    __syncthreads();
+    const int64_t base = (int64_t)blockIdx.x * items * SNT + threadIdx.x;
+    uint32_t bin[SITEMS], rank[SITEMS];
+#pragma unroll
+    for (int m = 0; m < SITEMS; m++) {
+        const int64_t p = base + (int64_t)m * SNT;
+        if (m < items && p < n) {
+            uint32_t cell;
+            bin[m] = brick_of(g, gld(pos, 3 * p), gld(pos, 3 * p + 1), gld(pos, 3 * p + 2), cell);
+            rank[m] = atomicAdd(&s_hist[bin[m]], 1u);
+        }
+    }
+    __syncthreads();
+    // each brick's count becomes the first slot of this work-group's range
+    for (uint32_t b = threadIdx.x; b <= g.nbrick; b += SNT) {
+        const uint32_t c = s_hist[b];
+        if (c) s_hist[b] = atomicAdd(&cursor[b], c);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < SITEMS; m++) {
+        const int64_t p = base + (int64_t)m * SNT;
+        if (m < items && p < n) {
+            const uint32_t q = s_hist[bin[m]] + rank[m];
+            rec[q] = make_float4(gld(pos, 3 * p), gld(pos, 3 * p + 1), gld(pos, 3 * p + 2),
+                                 val ? gld(val, p) : 1.0f);
+            idx[q] = (uint32_t)p;
+        }
+    }
+}
+
+// One work-group per brick: its records from rec (any order) to out (by
+// cell, then point index), and its cells' starts.  Ranks inside a cell come
+// from counting the cell's smaller indices, 8 at 8 points per cell.
+__global__ __launch_bounds__(CELLS) void k_sp_cells(SplatGrid g, const uint32_t *__restrict__ first,
+                                                     const float4 *__restrict__ rec,
+                                                     const uint32_t *__restrict__ idx,
+                                                     uint2 *__restrict__ spill,
+                                                     float4 *__restrict__ out,
+                                                     uint32_t *__restrict__ start) {
+    __shared__ uint32_t s_cell[CELLS + 1];    // points per cell, then the cell's first place
+    __shared__ uint32_t s_cur[CELLS];
+    __shared__ uint32_t s_idx[CAP];           // point indices, grouped by cell
+    __shared__ uint32_t s_src[CAP];           // cell << 16 | place in rec
+    __shared__ uint32_t s_wsum[CELLS / 64];
+    const int t = threadIdx.x;
+    const uint32_t b = blockIdx.x;
+    const uint32_t q0 = first[b], N = first[b + 1] - q0;
+    uint32_t *st = start + (size_t)b * CELLS;
+    if (b == g.nbrick - 1 && t == 0) start[(size_t)g.nbrick * CELLS] = q0 + N;
+    if (N == 0) {
+        st[t] = q0;
+        return;
+    }
+    s_cell[t] = 0u;
+    __syncthreads();
+    for (uint32_t e = t; e < N; e += CELLS) {
+        const float4 r = rec[q0 + e];
+        uint32_t cell;
+        brick_of(g, r.x, r.y, r.z, cell);
+        atomicAdd(&s_cell[cell], 1u);
+    }
+    __syncthreads();
+    {
+        // one cell per thread
+        const int lane = t & 63, wid = t >> 6;
+        const uint32_t n = s_cell[t], inc = wave_inclusive_sum(n);
+        if (lane == 63) s_wsum[wid] = inc;
+        __syncthreads();
+        uint32_t at = inc - n;
+        for (int w = 0; w < wid; w++) at += s_wsum[w];
+        s_cell[t] = s_cur[t] = at;
+        st[t] = q0 + at;
+        if (t == 0) s_cell[CELLS] = N;
+    }
+    __syncthreads();
+    if (N <= CAP) {
+        for (uint32_t e = t; e < N; e += CELLS) {
+            const float4 r = rec[q0 + e];
+            uint32_t cell;
+            brick_of(g, r.x, r.y, r.z, cell);
+            const uint32_t at = atomicAdd(&s_cur[cell], 1u);
+            s_idx[at] = idx[q0 + e];
+            s_src[at] = (cell << 16) | e;
+        }
+        __syncthreads();
+        for (uint32_t e = t; e < N; e += CELLS) {
+            const uint32_t sc = s_src[e], mine = s_idx[e];
+            const uint32_t c0 = s_cell[sc >> 16], c1 = s_cell[(sc >> 16) + 1];
+            uint32_t rank = 0;
+            for (uint32_t k = c0; k < c1; k++) rank += s_idx[k] < mine;
+            out[q0 + c0 + rank] = rec[q0 + (sc & 0xFFFFu)];
+        }
+        return;
+    }
+    // a crowded brick: the same with the groups in memory
+    for (uint32_t e = t; e < N; e += CELLS) {
+        const float4 r = rec[q0 + e];
+        uint32_t cell;
+        brick_of(g, r.x, r.y, r.z, cell);
+        spill[q0 + atomicAdd(&s_cur[cell], 1u)] = make_uint2(idx[q0 + e], e);
+    }
+    __syncthreads();   // (the groups are read back below)
+    for (uint32_t e = t; e < N; e += CELLS) {
+        const uint2 me = spill[q0 + e];
+        const float4 r = rec[q0 + me.y];
+        uint32_t cell;
+        brick_of(g, r.x, r.y, r.z, cell);
+        const uint32_t c0 = s_cell[cell], c1 = s_cell[cell + 1];
+        uint32_t rank = 0;
+        for (uint32_t k = c0; k < c1; k++) rank += spill[q0 + k].x < me.x;
+        out[q0 + c0 + rank] = r;
+    }
+}
+
+// One thread per column of kseg nodes along z.  A node's candidate cells
+// along an axis are D consecutive ones (dhi - dlo + 1), so the cells of one
+// plane reach D nodes of the column: the thread walks the planes upwards,
+// reads each candidate record once for all of them (its x and y distances
+// are shared) and keeps their sums in registers, slot m for node
+// plane - dhi + m.  A node's own terms still come plane by plane, row by row
+// and in cell order.  A row's cells are one range per brick they lie in; two
+// records are loaded ahead of the sums, and one past the range adds K = 0.
+template <bool HAS_VAL, int D>
+__global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, double dx,
+                                                      float inv_r2, int kseg,
+                                                      const uint32_t *__restrict__ start,
+                                                      const float4 *__restrict__ rec,
+                                                      float *__restrict__ S, float *__restrict__ W) {
+    constexpr int AHEAD = 2;
+    const int64_t col = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    const int64_t ncol = (int64_t)ng.n[0] * ng.n[1];
+    if (col >= ncol) return;
+    const int i = (int)(col % ng.n[0]), j = (int)(col / ng.n[0]);
+    const int k0 = (int)blockIdx.y * kseg, k1 = min(k0 + kseg, ng.n[2]);
+    // node position in the shifted frame, rounded as
+    // Grid3d::GridIndexToPosition does (grid3d.h:79-81)
+    const float gx = (float)((float)i * dx);
+    const float gy = (float)((float)j * dx);
+    const int ilo = max(i + ng.dlo[0], 0), ihi = min(i + ng.dhi[0], g.bg.b[0] - 1);
+    const int jlo = max(j + ng.dlo[1], 0), jhi = min(j + ng.dhi[1], g.bg.b[1] - 1);
+    const size_t stride = (size_t)ng.n[0] * ng.n[1];
+    float s[D], w[D], gz[D];
+#pragma unroll
+    for (int m = 0; m < D; m++) s[m] = w[m] = 0.0f;
+    for (int bk = k0 + ng.dlo[2]; bk <= k1 - 1 + ng.dhi[2]; bk++) {
+        const int kk = bk - ng.dhi[2];   // the node of slot 0
+        if (bk >= 0 && bk < g.bg.b[2]) {
+#pragma unroll
+            for (int m = 0; m < D; m++) gz[m] = (float)((float)(kk + m) * dx);
+            for (int bj = jlo; bj <= jhi; bj++) {
+                const uint32_t row = (uint32_t)g.gb[0] *
+                                     ((uint32_t)(bj >> 3) + (uint32_t)g.gb[1] * (uint32_t)(bk >> 3));
+                const uint32_t cjk = (uint32_t)((bj & 7) << 3) | (uint32_t)((bk & 7) << 6);
+                for (int a = ilo; a <= ihi;) {
+                    const int e = min(ihi, a | 7);
+                    const uint32_t id = ((row + (uint32_t)(a >> 3)) << 9) | cjk | (uint32_t)(a & 7);
+                    const uint32_t q0 = start[id], q1 = start[id + (uint32_t)(e - a) + 1u];
+                    for (uint32_t q = q0; q < q1; q += AHEAD) {
+                        float4 r[AHEAD];
+#pragma unroll
+                        for (int u = 0; u < AHEAD; u++) r[u] = rec[min(q + (uint32_t)u, q1 - 1u)];
+#pragma unroll
+                        for (int u = 0; u < AHEAD; u++) {
+                            // p -= offset, then v = gpos - p (scalarfield.cpp:168,186-188)
+                            const float vx = gx - (r[u].x - ng.off[0]);
+                            const float vy = gy - (r[u].y - ng.off[1]);
+                            const float pz = r[u].z - ng.off[2];
+                            const float dxy = vx * vx + vy * vy;
+                            const bool in = q + (uint32_t)u < q1;
+#pragma unroll
+                            for (int m = 0; m < D; m++) {
+                                // (the same for all lanes)
+                                if (kk + m < k0 || kk + m >= k1) continue;
+                                const float vz = gz[m] - pz;
+                                const float d2 = dxy + vz * vz;
+                                const float t = in ? d2 * inv_r2 : 1.0f;
+                                const float K = wyvill(t);
+                                // only inside the radius (scalarfield.cpp:191-196):
+                                // a value that is not finite must not reach the
+                                // nodes beyond it
+                                if (HAS_VAL) s[m] = fmaf(K, t < 1.0f ? r[u].w : 0.0f, s[m]);
+                                else s[m] += K;
+                                w[m] += K;
+                            }
+                        }
+                    }
+                    a = e + 1;
+                }
+            }
+        }
+        // the node of slot 0 has all its planes: accumulate into the caller's
+        // arrays (clscalarfield.cpp:1448-1449)
+        if (kk >= k0) {
+            const size_t f = (size_t)col + stride * (size_t)kk;
+            S[f] += s[0];
+            if (W) W[f] += w[0];
+        }
+#pragma unroll
+        for (int m = 0; m + 1 < D; m++) {
+            s[m] = s[m + 1];
+            w[m] = w[m + 1];
+        }
+        s[D - 1] = w[D - 1] = 0.0f;
+    }
+}
+
+int64_t bricks(const BinGrid &bg) {
+    int64_t b = 1;
+    for (int a = 0; a < 3; a++) b *= (bg.b[a] + 7) / 8;
+    return b;
+}
+
+}  // namespace
+
+bool splat_by_brick(int64_t n, const BinGrid &bg, double reach) {
+    return reach <= 4.0 && n < ((int64_t)1 << 31) && bricks(bg) < (int64_t)kMaxBricks;
+}
+
+size_t splat_workspace(int64_t n, const BinGrid &bg) {
+    const size_t nb = (size_t)bricks(bg);
+    // records twice, indices, crowded bricks' groups; counts, starts, cursors, cell starts
+    return (16 + 16 + 8 + 4) * (size_t)n + 3 * 4 * (nb + 2) + 4 * (nb * CELLS + 1) + 8 * 256;
+}
+
+void splat_run(void *work, const float *pos, const float *val, int64_t n, const BinGrid &bins,
+               const NodeGrid &nodes, double radius, double dx, float *S, float *W, hipStream_t st) {
+    const int64_t nnode = (int64_t)nodes.n[0] * nodes.n[1] * nodes.n[2];
+    if (nnode <= 0) return;
+    SplatGrid g;
+    g.bg = bins;
+    for (int a = 0; a < 3; a++) g.gb[a] = (bins.b[a] + 7) / 8;
+    g.nbrick = (uint32_t)bricks(bins);
+    char *at = static_cast<char *>(work);
+    auto take = [&](size_t bytes) {
+        char *p = at;
+        at += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    const size_t nn = (size_t)n;
+    float4 *rec = (float4 *)take(16 * nn), *out = (float4 *)take(16 * nn);
+    uint2 *spill = (uint2 *)take(8 * nn);
+    uint32_t *idx = (uint32_t *)take(4 * nn);
+    uint32_t *count = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
+    uint32_t *first = (uint32_t *)take(4 * (size_t)(g.nbrick + 2));
+    uint32_t *cursor = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
+    uint32_t *start = (uint32_t *)take(4 * ((size_t)g.nbrick * CELLS + 1));
+    fill_u32(count, 0u, (int64_t)g.nbrick + 1, st);
+    // about 512 work-groups, each of 1 to SITEMS points per thread, and of
+    // half as many points as histogram words (which each clears and reads)
+    const int items = (int)std::min<int64_t>(
+        std::max<int64_t>({n / ((int64_t)512 * SNT), (int64_t)g.nbrick / (2 * SNT), 1}), SITEMS);
+    const unsigned nblk = grid_for(n, (int64_t)items * SNT);
+    const size_t lds = 4 * ((size_t)g.nbrick + 1);
+    hipLaunchKernelGGL(k_sp_count, dim3(nblk), dim3(SNT), lds, st, g, pos, n, items, count);
+    GFSX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_sp_starts, dim3(1), dim3(SNT), 0, st, g.nbrick, (const uint32_t *)count,
+                       first, cursor);
+    GFSX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_sp_place, dim3(nblk), dim3(SNT), lds, st, g, pos, val, n, items, cursor,
+                       rec, idx);
+    GFSX_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_sp_cells, dim3(g.nbrick), dim3(CELLS), 0, st, g, (const uint32_t *)first,
+                       (const float4 *)rec, (const uint32_t *)idx, spill, out, start);
+    GFSX_LAUNCH_CHECK();
+    const float inv_r2 = (float)(1.0 / (radius * radius));
+    const int D = nodes.dhi[2] - nodes.dlo[2] + 1;
+    auto *kern = D == 2   ? (val ? k_sp_gather<true, 2> : k_sp_gather<false, 2>)
+                 : D == 4 ? (val ? k_sp_gather<true, 4> : k_sp_gather<false, 4>)
+                 : D == 6 ? (val ? k_sp_gather<true, 6> : k_sp_gather<false, 6>)
+                          : (val ? k_sp_gather<true, 8> : k_sp_gather<false, 8>);
+    // Columns of 1 to 16 nodes, about 8192 waves of them (and no more
+    // segments than a grid's y extent holds): longer columns read less,
+    // shorter ones fill the chip.  0.27M nodes, columns of 1 / 4: 22 / 52 us
+    // of gather; 2.8M nodes at R = 2.5 dx, the whole call with columns of
+    // 1 / 3 / 5 / 8: 644 / 442 / 410 / 427 us.
+    const int kseg = (int)std::max<int64_t>(
+        std::min<int64_t>(std::max<int64_t>(nnode / (64 * 8192), 1), 16), nodes.n[2] / 65535 + 1);
+    hipLaunchKernelGGL(kern, dim3(grid_for((int64_t)nodes.n[0] * nodes.n[1], kBlock),
+                                  grid_for(nodes.n[2], kseg)),
+                       dim3(kBlock), 0, st, g, nodes, dx, inv_r2, kseg, (const uint32_t *)start,
+                       (const float4 *)out, S, W);
+    GFSX_LAUNCH_CHECK();
+}
+
+}  // namespace gfsx
