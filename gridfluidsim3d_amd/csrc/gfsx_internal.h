@@ -327,8 +327,11 @@ struct RemoveArgs {
     const uint8_t *solid;
     int max_per_cell;
     uint64_t seed;
-    uint32_t *keep, *dst;
-    uint32_t *full, *nfull;   // over-full cells: list (capacity nbin) and count
+    uint8_t *keep;            // per particle
+    uint32_t *count, *dst;    // kept particles per block of the compaction; their scan
+    uint32_t *full;           // the cells that lose particles: small ones from the front,
+    uint32_t full_cap;        // large ones from the back (nfull[0] and nfull[1] of them)
+    uint32_t *nfull;
 };
 
 // ---- launches (implemented in gfsx_kernels.hip) ------------------------
@@ -340,6 +343,7 @@ void fill_u8(uint8_t *p, uint8_t value, int64_t count, hipStream_t s);
 void fs_epilogue(const FsEpilogue &e, hipStream_t s);
 void fs_collide(const FsEpilogue &e, hipStream_t s);
 // gfsx_remove.hip
+int64_t remove_blocks(int64_t n);   // entries of count (dst has one more)
 void remove_mark(const RemoveArgs &r, hipStream_t s);
 void remove_compact(const RemoveArgs &r, hipStream_t s);
 // gfsx_adjoint.hip
@@ -390,8 +394,10 @@ int64_t sort_blocks(int64_t n);
 // contiguous run), hrank[q] receives the rank of perm[q] inside its
 // half-cell run and soct[q] its octant.  With mark_bricks, brick_flag
 // receives the P2G bricks with a particle within reach.
+// With grouped_only, perm_tmp holds the particles grouped by bin in no order
+// inside one, and perm is not written.
 void cell_sort(const SortBuffers &sb, int64_t n, hipStream_t s, bool octant_order,
-               bool mark_bricks = false);
+               bool mark_bricks = false, bool grouped_only = false);
 
 // Generic P2G gather for one component (ScalarField semantics).
 void p2g_gather(const float *aos, const float *val, int64_t n,

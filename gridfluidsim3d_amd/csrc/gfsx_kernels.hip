@@ -566,7 +566,7 @@ __global__ __launch_bounds__(64) void k_order_big(
 }
 
 void cell_sort(const SortBuffers &sb, int64_t n, hipStream_t s, bool octant_order,
-               bool mark_bricks) {
+               bool mark_bricks, bool grouped_only) {
     fill_u32(sb.count, 0u, (int64_t)sb.nbin_total, s);
     if (n <= 0) {
         fill_u32(sb.start, 0u, (int64_t)sb.nbin_total + 1, s);
@@ -588,6 +588,7 @@ void cell_sort(const SortBuffers &sb, int64_t n, hipStream_t s, bool octant_orde
                        (const uint32_t *)sb.start, (const uint32_t *)sb.block_out_scan,
                        sb.perm_tmp, (const uint8_t *)oct, poct);
     GFSX_LAUNCH_CHECK();
+    if (grouped_only) return;
     fill_u32(sb.big_count, 0u, 2, s);
     OrderOut out;
     out.perm = sb.perm;
