@@ -1046,8 +1046,10 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
 // Combine: every face from the tiles that hold it
 // ---------------------------------------------------------------------------
 //
-// One wave per combine_rows(nx) consecutive face rows along x (component
-// c, node rows j, k), each row 64 faces at a time in array order.  Node
+// Where the rows along x fill a wave's lanes (ROWS; combine_by_rows): one wave
+// per combine_rows consecutive rows (component c, node rows j, k), each row 64
+// faces at a time, its bricks and masks scalar work.  Otherwise (33 of 64
+// lanes, 129 of 192) array order across row ends, fpw faces per wave.  Node
 // 4b+r of an axis lies in the tile of brick b at position r (own axis:
 // nodes 4b .. 4b+4) or r+1 (across: 4b-1 .. 4b+4); also in brick b-1's tile
 // (r = 0: position 4 along the own axis, 5 across) or, across, in brick
@@ -1101,6 +1103,7 @@ __device__ __forceinline__ bool cell_fluid(const SceneDesc &sd,
     return (gld(fluid, bin) >> ((i & 3) + 4 * (j & 3) + 16 * (k & 3))) & 1ull;
 }
 
+template <bool ROWS>
 __global__ __launch_bounds__(kBlock) void k_p2g_bcombine(
     const SceneDesc *__restrict__ scenes, const int64_t *__restrict__ r0s, int nsc, int64_t nwave,
     const float2 *__restrict__ tiles, const unsigned long long *__restrict__ tile_rows,
@@ -1130,25 +1133,127 @@ __global__ __launch_bounds__(kBlock) void k_p2g_bcombine(
     if (c > 0) lw -= sd.cw[c - 1];
     const int ni = sd.ni, nj = sd.nj, nk = sd.nk;
     const int nxc = ni + (c == 0), nyc = nj + (c == 1), nzc = nk + (c == 2);
-    // this wave's rows, in turn: [r, r + rpw) of the component's nyc * nzc;
-    // every index below is the same for all lanes
-    const int rpw = combine_rows(nxc);
-    const uint32_t nrows = (uint32_t)nyc * (uint32_t)nzc;
-    const uint32_t r0 = (uint32_t)lw * (uint32_t)rpw;
-    const uint32_t r1 = min(r0 + (uint32_t)rpw, nrows);
-    int J = (int)(r0 % (uint32_t)nyc), K = (int)(r0 / (uint32_t)nyc);
     const TileGrid tg = tile_grid(sd, c);
     const int sx = tsx(c), sy = tsy(c), sz = tsz(c);
     const FaceOut fo = face_out(sd.p2g, c);
     const unsigned long long *te = reinterpret_cast<const unsigned long long *>(tiles);
-    for (uint32_t r = r0; r < r1; r++) {
-        const AxisTiles ay = axis_tiles(J, sd.nby, c == 1), az = axis_tiles(K, sd.nbz, c == 2);
-        // per (z, y) brick row of the face row: the tile row it reads, and
-        // that row's occupied-brick mask (one word, loaded once for the
-        // wave, when the grid has at most 64 bricks along x)
+    if (ROWS) {
+        // this wave's rows, in turn: [r, r + rpw) of the component's nyc * nzc;
+        // every index below is the same for all lanes
+        const int rpw = combine_rows(nxc, sd.fpw);
+        const uint32_t nrows = (uint32_t)nyc * (uint32_t)nzc;
+        const uint32_t r0 = (uint32_t)lw * (uint32_t)rpw;
+        const uint32_t r1 = min(r0 + (uint32_t)rpw, nrows);
+        int J = (int)(r0 % (uint32_t)nyc), K = (int)(r0 / (uint32_t)nyc);
+        for (uint32_t r = r0; r < r1; r++) {
+            const AxisTiles ay = axis_tiles(J, sd.nby, c == 1), az = axis_tiles(K, sd.nbz, c == 2);
+            // per (z, y) brick row of the face row: the tile row it reads, and
+            // that row's occupied-brick mask (one word, loaded once for the
+            // wave, when the grid has at most 64 bricks along x)
+            size_t trow[2][2];
+            uint32_t mrow[2][2];
+            unsigned long long mw[2][2];
+#pragma unroll
+            for (int iz = 0; iz < 2; iz++)
+#pragma unroll
+                for (int iy = 0; iy < 2; iy++) {
+                    const int by = ay.b + ay.db[iy], bz = az.b + az.db[iz];
+                    const bool ok = iz < az.cnt && iy < ay.cnt;
+                    trow[iz][iy] = tile_at(tg, 0, by * sy + ay.tp[iy], bz * sz + az.tp[iz]);
+                    mrow[iz][iy] = sd.rm0 + (uint32_t)sd.rmw * ((uint32_t)by + (uint32_t)sd.nby * (uint32_t)bz);
+                    mw[iz][iy] = ok && sd.rmw == 1 ? tile_rows[mrow[iz][iy]] : 0ull;
+                }
+            for (int I = lane; I < nxc; I += 64) {
+                const AxisTiles ax = axis_tiles(I, sd.nbx, c == 0);
+                const bool two = ax.cnt == 2;
+                const int bx0 = ax.b + ax.db[0], bx1 = two ? ax.b + ax.db[1] : bx0;
+                const size_t e0 = (size_t)(bx0 * sx + ax.tp[0]), e1 = (size_t)(bx1 * sx + ax.tp[1]);
+                // the entries of the bricks that hold particles (a brick without
+                // particles wrote no tile), every load issued before any is used
+                uint32_t f0[2][2], f1[2][2];
+#pragma unroll
+                for (int iz = 0; iz < 2; iz++)
+#pragma unroll
+                    for (int iy = 0; iy < 2; iy++) {
+                        const bool ok = iz < az.cnt && iy < ay.cnt;
+                        unsigned long long m0 = mw[iz][iy], m1 = mw[iz][iy];
+                        if (sd.rmw > 1 && ok) {
+                            m0 = gld(tile_rows, (size_t)mrow[iz][iy] + (size_t)(bx0 >> 6));
+                            m1 = gld(tile_rows, (size_t)mrow[iz][iy] + (size_t)(bx1 >> 6));
+                        }
+                        f0[iz][iy] = ok ? (uint32_t)(m0 >> (bx0 & 63)) & 1u : 0u;
+                        f1[iz][iy] = ok && two ? (uint32_t)(m1 >> (bx1 & 63)) & 1u : 0u;
+                    }
+                unsigned long long v0[2][2], v1[2][2];   // (S, W) float pairs
+#pragma unroll
+                for (int iz = 0; iz < 2; iz++)
+#pragma unroll
+                    for (int iy = 0; iy < 2; iy++) {
+                        v0[iz][iy] = f0[iz][iy] ? gld(te, trow[iz][iy] + e0) : 0ull;
+                        v1[iz][iy] = f1[iz][iy] ? gld(te, trow[iz][iy] + e1) : 0ull;
+                    }
+                // the entries added lower brick first: z, then y, then x
+                float S = 0.0f, W = 0.0f;
+#pragma unroll
+                for (int iz = 0; iz < 2; iz++)
+#pragma unroll
+                    for (int iy = 0; iy < 2; iy++) {
+                        if (f0[iz][iy]) {
+                            S += __uint_as_float((uint32_t)v0[iz][iy]);
+                            W += __uint_as_float((uint32_t)(v0[iz][iy] >> 32));
+                        }
+                        if (f1[iz][iy]) {
+                            S += __uint_as_float((uint32_t)v1[iz][iy]);
+                            W += __uint_as_float((uint32_t)(v1[iz][iy] >> 32));
+                        }
+                    }
+                const int64_t f = (int64_t)I + (int64_t)nxc * ((int64_t)J + (int64_t)nyc * K);
+                float val = W > 0.0f ? S / W : S;
+                if (fo.old) gst(fo.old, (size_t)f, val);
+                if (fo.wgt) gst(fo.wgt, (size_t)f, W);
+                if (fo.grav_on) {
+                    // the cells on either side along axis c
+                    const int n = c == 0 ? I : (c == 1 ? J : K);
+                    bool fl = false;
+                    if (n < fo.nax) fl = cell_fluid(sd, fluid, I, J, K);
+                    if (n > 0)
+                        fl = fl || cell_fluid(sd, fluid, I - (c == 0), J - (c == 1), K - (c == 2));
+                    if (fl) val += fo.grav_delta;
+                }
+                gst(fo.grid, (size_t)f, val);
+            }
+            if (++J == nyc) {
+                J = 0;
+                K++;
+            }
+        }
+        return;
+    }
+    // this wave's faces: fpw of the component's, 64 at a time in array order.
+    // The first one's row by (scalar) division, a lane's by steps from it.
+    const uint32_t nf = (uint32_t)nxc * (uint32_t)nyc * (uint32_t)nzc;
+    const uint32_t fb = (uint32_t)lw * (uint32_t)sd.fpw;
+    const uint32_t fe = min(fb + (uint32_t)sd.fpw, nf);
+    const uint32_t row0 = fb / (uint32_t)nxc;
+    int J = (int)(row0 % (uint32_t)nyc), K = (int)(row0 / (uint32_t)nyc);
+    int I = (int)(fb - row0 * (uint32_t)nxc) + lane;
+    for (uint32_t f = fb + (uint32_t)lane; f < fe; f += 64u, I += 64) {
+        while (I >= nxc) {
+            I -= nxc;
+            if (++J == nyc) {
+                J = 0;
+                K++;
+            }
+        }
+        const AxisTiles ax = axis_tiles(I, sd.nbx, c == 0), ay = axis_tiles(J, sd.nby, c == 1),
+                        az = axis_tiles(K, sd.nbz, c == 2);
+        const bool two = ax.cnt == 2;
+        const int bx0 = ax.b + ax.db[0], bx1 = two ? ax.b + ax.db[1] : bx0;
+        const uint32_t e0 = (uint32_t)(bx0 * sx + ax.tp[0]), e1 = (uint32_t)(bx1 * sx + ax.tp[1]);
+        // the entries of the bricks that hold particles (a brick without
+        // particles wrote no tile), every load issued before any is used
+        uint32_t f0[2][2], f1[2][2];
         size_t trow[2][2];
-        uint32_t mrow[2][2];
-        unsigned long long mw[2][2];
 #pragma unroll
         for (int iz = 0; iz < 2; iz++)
 #pragma unroll
@@ -1156,72 +1261,52 @@ __global__ __launch_bounds__(kBlock) void k_p2g_bcombine(
                 const int by = ay.b + ay.db[iy], bz = az.b + az.db[iz];
                 const bool ok = iz < az.cnt && iy < ay.cnt;
                 trow[iz][iy] = tile_at(tg, 0, by * sy + ay.tp[iy], bz * sz + az.tp[iz]);
-                mrow[iz][iy] = sd.rm0 + (uint32_t)sd.rmw * ((uint32_t)by + (uint32_t)sd.nby * (uint32_t)bz);
-                mw[iz][iy] = ok && sd.rmw == 1 ? tile_rows[mrow[iz][iy]] : 0ull;
+                const uint32_t mrow =
+                    sd.rm0 + (uint32_t)sd.rmw * ((uint32_t)by + (uint32_t)sd.nby * (uint32_t)bz);
+                unsigned long long m0 = 0ull, m1 = 0ull;
+                if (ok) {
+                    m0 = m1 = gld(tile_rows, (size_t)mrow + (size_t)(bx0 >> 6));
+                    if (sd.rmw > 1) m1 = gld(tile_rows, (size_t)mrow + (size_t)(bx1 >> 6));
+                }
+                f0[iz][iy] = (uint32_t)(m0 >> (bx0 & 63)) & 1u;
+                f1[iz][iy] = two ? (uint32_t)(m1 >> (bx1 & 63)) & 1u : 0u;
             }
-        for (int I = lane; I < nxc; I += 64) {
-            const AxisTiles ax = axis_tiles(I, sd.nbx, c == 0);
-            const bool two = ax.cnt == 2;
-            const int bx0 = ax.b + ax.db[0], bx1 = two ? ax.b + ax.db[1] : bx0;
-            const size_t e0 = (size_t)(bx0 * sx + ax.tp[0]), e1 = (size_t)(bx1 * sx + ax.tp[1]);
-            // the entries of the bricks that hold particles (a brick without
-            // particles wrote no tile), every load issued before any is used
-            uint32_t f0[2][2], f1[2][2];
+        unsigned long long v0[2][2], v1[2][2];   // (S, W) float pairs
 #pragma unroll
-            for (int iz = 0; iz < 2; iz++)
+        for (int iz = 0; iz < 2; iz++)
 #pragma unroll
-                for (int iy = 0; iy < 2; iy++) {
-                    const bool ok = iz < az.cnt && iy < ay.cnt;
-                    unsigned long long m0 = mw[iz][iy], m1 = mw[iz][iy];
-                    if (sd.rmw > 1 && ok) {
-                        m0 = gld(tile_rows, (size_t)mrow[iz][iy] + (size_t)(bx0 >> 6));
-                        m1 = gld(tile_rows, (size_t)mrow[iz][iy] + (size_t)(bx1 >> 6));
-                    }
-                    f0[iz][iy] = ok ? (uint32_t)(m0 >> (bx0 & 63)) & 1u : 0u;
-                    f1[iz][iy] = ok && two ? (uint32_t)(m1 >> (bx1 & 63)) & 1u : 0u;
-                }
-            unsigned long long v0[2][2], v1[2][2];   // (S, W) float pairs
-#pragma unroll
-            for (int iz = 0; iz < 2; iz++)
-#pragma unroll
-                for (int iy = 0; iy < 2; iy++) {
-                    v0[iz][iy] = f0[iz][iy] ? gld(te, trow[iz][iy] + e0) : 0ull;
-                    v1[iz][iy] = f1[iz][iy] ? gld(te, trow[iz][iy] + e1) : 0ull;
-                }
-            // the entries added lower brick first: z, then y, then x
-            float S = 0.0f, W = 0.0f;
-#pragma unroll
-            for (int iz = 0; iz < 2; iz++)
-#pragma unroll
-                for (int iy = 0; iy < 2; iy++) {
-                    if (f0[iz][iy]) {
-                        S += __uint_as_float((uint32_t)v0[iz][iy]);
-                        W += __uint_as_float((uint32_t)(v0[iz][iy] >> 32));
-                    }
-                    if (f1[iz][iy]) {
-                        S += __uint_as_float((uint32_t)v1[iz][iy]);
-                        W += __uint_as_float((uint32_t)(v1[iz][iy] >> 32));
-                    }
-                }
-            const int64_t f = (int64_t)I + (int64_t)nxc * ((int64_t)J + (int64_t)nyc * K);
-            float val = W > 0.0f ? S / W : S;
-            if (fo.old) gst(fo.old, (size_t)f, val);
-            if (fo.wgt) gst(fo.wgt, (size_t)f, W);
-            if (fo.grav_on) {
-                // the cells on either side along axis c
-                const int n = c == 0 ? I : (c == 1 ? J : K);
-                bool fl = false;
-                if (n < fo.nax) fl = cell_fluid(sd, fluid, I, J, K);
-                if (n > 0)
-                    fl = fl || cell_fluid(sd, fluid, I - (c == 0), J - (c == 1), K - (c == 2));
-                if (fl) val += fo.grav_delta;
+            for (int iy = 0; iy < 2; iy++) {
+                v0[iz][iy] = f0[iz][iy] ? gld(te, trow[iz][iy] + e0) : 0ull;
+                v1[iz][iy] = f1[iz][iy] ? gld(te, trow[iz][iy] + e1) : 0ull;
             }
-            gst(fo.grid, (size_t)f, val);
+        // the entries added lower brick first: z, then y, then x
+        float S = 0.0f, W = 0.0f;
+#pragma unroll
+        for (int iz = 0; iz < 2; iz++)
+#pragma unroll
+            for (int iy = 0; iy < 2; iy++) {
+                if (f0[iz][iy]) {
+                    S += __uint_as_float((uint32_t)v0[iz][iy]);
+                    W += __uint_as_float((uint32_t)(v0[iz][iy] >> 32));
+                }
+                if (f1[iz][iy]) {
+                    S += __uint_as_float((uint32_t)v1[iz][iy]);
+                    W += __uint_as_float((uint32_t)(v1[iz][iy] >> 32));
+                }
+            }
+        float val = W > 0.0f ? S / W : S;
+        if (fo.old) gst(fo.old, (size_t)f, val);
+        if (fo.wgt) gst(fo.wgt, (size_t)f, W);
+        if (fo.grav_on) {
+            // the cells on either side along axis c
+            const int n = c == 0 ? I : (c == 1 ? J : K);
+            bool fl = false;
+            if (n < fo.nax) fl = cell_fluid(sd, fluid, I, J, K);
+            if (n > 0)
+                fl = fl || cell_fluid(sd, fluid, I - (c == 0), J - (c == 1), K - (c == 2));
+            if (fl) val += fo.grav_delta;
         }
-        if (++J == nyc) {
-            J = 0;
-            K++;
-        }
+        gst(fo.grid, (size_t)f, val);
     }
 }
 
@@ -1642,8 +1727,9 @@ void flip_step_brick(const StepBatch &s, const BrickSort &bs, hipStream_t st, hi
                        s.tile_rows, bs.fluid);
     GFSX_LAUNCH_CHECK();
     if (nsc > 1 && !s.r0s) throw Error("gfsx: the combine of several scenes needs their wave offsets");
-    hipLaunchKernelGGL(k_p2g_bcombine, dim3(grid_for(s.tot.nrow, kBlock / 64)), dim3(kBlock), 0, st,
-                       s.scenes_dev, s.r0s, nsc, s.tot.nrow, (const float2 *)s.tiles,
+    hipLaunchKernelGGL(s.tot.by_rows ? k_p2g_bcombine<true> : k_p2g_bcombine<false>,
+                       dim3(grid_for(s.tot.nrow, kBlock / 64)), dim3(kBlock), 0, st, s.scenes_dev,
+                       s.r0s, nsc, s.tot.nrow, (const float2 *)s.tiles,
                        (const unsigned long long *)s.tile_rows, (const unsigned long long *)bs.fluid);
     GFSX_LAUNCH_CHECK();
     if (s.epi) fs_epilogue(*s.epi, st);

@@ -135,7 +135,8 @@ struct SceneDesc {
     int rmw;
     int64_t f0;       // first global MAC face (faces of u, then v, then w, per scene)
     int64_t r0;       // first combine wave (over the x-rows of u, then v, then w)
-    int64_t cw[2];    // combine waves of the scene before its v rows and before its w rows
+    int64_t cw[2];    // combine waves of the scene before its v faces and before its w faces
+    int fpw;          // faces a combine wave takes (combine_faces; one value for all scenes)
     // grid and step constants
     int ni, nj, nk;
     double dx;
@@ -446,9 +447,22 @@ size_t points_workspace(int64_t n, int ni, int nj, int nk);
 void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int order, double dt,
                 int stencil, float *out, hipStream_t s);
 
-// Face rows along x that one wave of the combine takes in turn: enough for
-// about 256 faces, so that short rows share a wave's set-up.
-__host__ __device__ inline int combine_rows(int nx) { return nx < 256 ? 256 / nx : 1; }
+// Faces that one wave of the combine takes, for a step of nface faces in
+// all: 64 at a time, once in small steps, so that there are waves to fill the
+// chip (101k faces: 18 -> 4.5 us against seven rows of 33 per wave).
+inline int combine_faces(int64_t nface) {
+    return nface < ((int64_t)1 << 21) ? 64 : nface < ((int64_t)1 << 23) ? 128 : 256;
+}
+
+// Whether the combine of a step takes its faces by rows (scalar row set-up):
+// when they fill at least 9 in 10 of the lanes that cover their rows, lanes in
+// all.  50.5M faces, rows of 256 and 257 (93%): 0.36 ms by rows, 0.38 across
+// row ends; 6.3M, rows of 128 and 129 (86%): 52 and 47 us; 65.7M in rows of 32
+// to 129: 0.71 and 0.56 ms.  Choosing wave by wave inside one kernel cost both
+// (0.38, 0.61).
+inline bool combine_by_rows(int64_t nface, int64_t lanes) { return 10 * nface >= 9 * lanes; }
+// Rows per wave by rows.
+__host__ __device__ inline int combine_rows(int nx, int fpw) { return nx < fpw ? fpw / nx : 1; }
 
 // Sizes of a scene table laid out by layout_scenes.
 struct SceneTotals {
@@ -459,7 +473,8 @@ struct SceneTotals {
     int64_t ng2p = 0;    // G2P bricks
     int64_t nface = 0;   // MAC faces
     int64_t nbb = 0;     // brick sort bins, overflow bins included
-    int64_t nrow = 0;    // combine waves (face rows along x, short rows packed), all components
+    int64_t nrow = 0;    // combine waves, all components
+    bool by_rows = false;   // the combine takes whole rows (combine_by_rows)
     int64_t nrm = 0;     // occupied-brick mask words
 };
 

@@ -1865,6 +1865,17 @@ __global__ __launch_bounds__(gbrick::NT, 2) void k_flip_g2p_brick_tc(
 
 void layout_scenes(SceneDesc *sc, int nsc, SceneTotals &tot) {
     tot = SceneTotals();
+    int64_t nface = 0, lanes = 0;
+    for (int i = 0; i < nsc; i++) {
+        for (int c = 0; c < 3; c++) {
+            const int64_t nx = sc[i].ni + (c == 0);
+            const int64_t rows = (int64_t)(sc[i].nj + (c == 1)) * (sc[i].nk + (c == 2));
+            nface += nx * rows;
+            lanes += (nx + 63) / 64 * 64 * rows;
+        }
+    }
+    tot.by_rows = combine_by_rows(nface, lanes);
+    const int fpw = combine_faces(nface);
     for (int i = 0; i < nsc; i++) {
         SceneDesc &d = sc[i];
         BinGrid &bg = d.bg;
@@ -1909,19 +1920,21 @@ void layout_scenes(SceneDesc *sc, int nsc, SceneTotals &tot) {
         tot.np2g += (int64_t)d.nbx * d.nby * d.nbz;
         tot.ng2p += (int64_t)d.gbx * d.gby * d.gbz;
         tot.nbb += (int64_t)d.nbb + 1;
-        // combine waves: each takes combine_rows(nx) consecutive face rows
-        // along x
+        // combine waves: each takes fpw faces (or whole rows) of one component
+        d.fpw = fpw;
+        const int64_t nf[3] = {(int64_t)(d.ni + 1) * d.nj * d.nk, (int64_t)d.ni * (d.nj + 1) * d.nk,
+                               (int64_t)d.ni * d.nj * (d.nk + 1)};
         int64_t waves[3];
         for (int c = 0; c < 3; c++) {
-            const int64_t rows = (int64_t)(d.nj + (c == 1)) * (d.nk + (c == 2));
-            const int64_t rpw = combine_rows(d.ni + (c == 0));
-            waves[c] = (rows + rpw - 1) / rpw;
+            const int nx = d.ni + (c == 0);
+            const int64_t per = tot.by_rows ? combine_rows(nx, fpw) : fpw;
+            const int64_t what = tot.by_rows ? nf[c] / nx : nf[c];
+            waves[c] = (what + per - 1) / per;
         }
         d.cw[0] = waves[0];
         d.cw[1] = waves[0] + waves[1];
         tot.nrow += waves[0] + waves[1] + waves[2];
-        tot.nface += (int64_t)(d.ni + 1) * d.nj * d.nk + (int64_t)d.ni * (d.nj + 1) * d.nk +
-                     (int64_t)d.ni * d.nj * (d.nk + 1);
+        tot.nface += nf[0] + nf[1] + nf[2];
     }
 }
 
