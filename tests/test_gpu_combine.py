@@ -1,35 +1,36 @@
-"""The combine of the scatter P2G's tiles by rows and across row ends: grids
-whose rows fill the lanes and grids whose rows do not, one and two words of
-occupied bricks per row, against the oracle."""
+"""The combine of the scatter P2G's tiles by rows and across row ends.  A
+scene alone takes one of the two by its own rows; in a batch all scenes take
+one by the rows of all.  Either way a scene's results are the same bits."""
 import numpy as np
 import pytest
 
-from conftest import NORM_REL_TOL, norm_rel
-
 pytestmark = pytest.mark.gpu
 
+ROWS = [(250, 10, 12), (300, 6, 8)]    # fill their lanes (300: two mask words a row)
+ENDS = [(1, 3, 2), (5, 4, 63), (33, 9, 10), (129, 8, 8), (64, 200, 3), (270, 8, 9)]
 
-@pytest.mark.parametrize("dims", [
-    (1, 3, 2), (5, 4, 63), (33, 9, 10), (129, 8, 8),    # across row ends
-    (250, 10, 12), (64, 200, 3),                        # by rows; u rows of one lane past 64
-    (300, 6, 8), (270, 8, 9),                           # two mask words per row of bricks
-])
-def test_grids_match_oracle(ctx, orc, dims):
+
+def state(dims, seed, n=6000):
     import gridfluidsim3d_amd as gf
-    rng = np.random.default_rng(dims[0])
-    dx, dt, n = 0.1, 1.0 / 120.0, 6000
-    pos = (rng.uniform(-0.01, 1.01, size=(n, 3)) * np.array(dims) * dx).astype(np.float32)
+    rng = np.random.default_rng(seed)
+    pos = (rng.uniform(-0.01, 1.01, size=(n, 3)) * np.array(dims) * 0.1).astype(np.float32)
     pos[n // 2:, 0] *= 0.3      # bricks without particles along the rows
     vel = rng.normal(size=(n, 3)).astype(np.float32)
-    st = gf.FlipState(pos, vel, dims, dx, keep_old=True, keep_weights=True)
-    ctx.flip_step(st, dt, (1.0, -9.8, 0.5), 0.05, gf.TRILINEAR, gf.ORDER_KEEP)
-    exp = orc.flip_step(pos, vel, dims, dx, dt, (1.0, -9.8, 0.5), 0.05, 0)
-    for c, name in enumerate("uvw"):
-        assert norm_rel(st.grid[c].cpu().numpy(), exp[name]) <= NORM_REL_TOL
-        off = [0.5 * dx] * 3
-        off[c] = 0.0
-        nd = gf.mac_shapes(dims)[c][::-1]
-        S, W = orc.p2g(pos, vel[:, c].copy(), dx, off, dx, nd)
-        assert norm_rel(st.weights[c].cpu().numpy(), W) <= NORM_REL_TOL
-        old = np.where(W > 0, S / np.where(W > 0, W, 1), S)
-        assert norm_rel(st.grid_old[c].cpu().numpy(), old) <= NORM_REL_TOL
+    return gf.FlipState(pos, vel, dims, 0.1, keep_old=True, keep_weights=True)
+
+
+@pytest.mark.parametrize("filler,scenes", [((40, 40, 40), ROWS + ENDS), ((256, 90, 90), ENDS)])
+def test_combine_same_bits_alone_and_batched(ctx, filler, scenes):
+    """The filler's faces decide for the batch: across row ends, by rows."""
+    import torch
+    batch = [state(d, i) for i, d in enumerate(scenes)] + [state(filler, 99)]
+    kw = dict(dt=1.0 / 120.0, body_force=(1.0, -9.8, 0.5))
+    ctx.flip_step_batched(batch, **kw)
+    for i, d in enumerate(scenes):
+        one = state(d, i)
+        ctx.flip_step(one, **kw)
+        for a, b in ((one.grid, batch[i].grid), (one.grid_old, batch[i].grid_old),
+                     (one.weights, batch[i].weights), (one.cur_x, batch[i].cur_x)):
+            for p, q in zip(a, b):
+                assert torch.equal(p, q)
+        assert all(bool(w.abs().sum() > 0) for w in one.weights)
