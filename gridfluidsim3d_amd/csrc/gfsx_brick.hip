@@ -395,17 +395,14 @@ static void exclusive_scan64(const unsigned long long *in, unsigned long long *o
 }
 
 // Particle and run starts of every bin from the scanned counts.
-// Also clears the order kernels' two list counters and G2P's slow-list
-// count (zeros: three words, no separate fill launches).
+// Also clears the order kernels' list counters, those of k_step_lists and
+// G2P's slow-list count (five words, no separate fill launches).
 __global__ void k_bsort_split(const unsigned long long *__restrict__ start, uint32_t m,
                               uint32_t *__restrict__ pstart, uint32_t *__restrict__ rstart,
                               uint32_t *__restrict__ lcount, uint32_t *__restrict__ slow_count) {
     const uint32_t b = blockIdx.x * kBlock + threadIdx.x;
-    if (b == 0) {
-        lcount[0] = 0u;
-        lcount[1] = 0u;
-        *slow_count = 0u;
-    }
+    if (b < 4) lcount[b] = 0u;
+    if (b == 0) *slow_count = 0u;
     if (b >= m) return;
     const unsigned long long v = start[b];
     pstart[b] = (uint32_t)v;
@@ -672,6 +669,76 @@ __global__ __launch_bounds__(kBlock) void k_bsort_scatter(const SceneDesc *__res
     }
 }
 
+// The work lists of the scatter P2G and the brick G2P, from the bin starts:
+// bins lists every bin with particles; chunks every G2P brick (8 bins) with
+// particles, as (first bin, share), cut into equal shares of at most
+// chunk particles.  Their order follows the bins up to the order of the
+// work-groups' atomics; it decides only which work-group does what.  A
+// kernel that takes an eighth of its list on each XCD then gives every XCD
+// the same work, where an eighth of all bricks can be mostly empty space (a
+// pool with spheres in 256^3: the fullest eighth holds 1.41 times the mean),
+// and a step of few full bricks still fills the chip.  43M particles there:
+// scatter 1.47 -> 1.07 ms, G2P 0.85 -> 0.70; tricubic G2P of 1120 full bricks
+// (128^3, 4M) 0.44 -> 0.35.  Also clears the occupied-brick masks and the
+// fluid cells of the empty bins.
+__global__ __launch_bounds__(kBlock) void k_step_lists(
+    const SceneDesc *__restrict__ scenes, int nsc, uint32_t nbin, uint32_t chunk,
+    const uint32_t *__restrict__ pstart, unsigned long long *__restrict__ tile_rows, int64_t nrm,
+    unsigned long long *__restrict__ fluid, uint32_t *__restrict__ bins,
+    uint2 *__restrict__ chunks, uint32_t *__restrict__ lcount) {
+    constexpr int ITEMS = 4;   // bins per thread: a quarter of the same-address atomics
+    __shared__ uint32_t s_wsum[kBlock / 64];
+    __shared__ uint32_t s_at[2];
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t i = blockIdx.x * (int64_t)kBlock + threadIdx.x; i < nrm; i += stride) tile_rows[i] = 0ull;
+    const uint32_t first = blockIdx.x * (uint32_t)(ITEMS * kBlock);
+    // the scene of the work-group's first bin (scalar), then steps from it
+    int si = scene_of(scenes, nsc, first, [](const SceneDesc &d) { return d.kb0; });
+    uint32_t full[ITEMS], nc[ITEMS], fo[ITEMS], co[ITEMS];
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        const int64_t b = (int64_t)first + m * kBlock + threadIdx.x;
+        full[m] = nc[m] = 0;
+        if (b < (int64_t)nbin) {
+            const uint32_t q0 = pstart[b];
+            full[m] = pstart[b + 1] > q0;
+            if (!full[m]) fluid[b] = 0ull;
+            while (si + 1 < nsc && (int64_t)scenes[si + 1].kb0 <= b) si++;
+            const uint32_t lb = (uint32_t)b - scenes[si].kb0;
+            if (lb < scenes[si].nbb && (lb & 7u) == 0u)
+                nc[m] = (pstart[b + 8] - q0 + chunk - 1u) / chunk;
+        }
+    }
+    uint32_t tf = 0, tc = 0;
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        uint32_t f, c;
+        fo[m] = tf + block_exclusive_sum(full[m], s_wsum, f);
+        co[m] = tc + block_exclusive_sum(nc[m], s_wsum, c);
+        tf += f;
+        tc += c;
+    }
+    if (threadIdx.x == 0) {
+        s_at[0] = tf ? atomicAdd(&lcount[2], tf) : 0u;
+        s_at[1] = tc ? atomicAdd(&lcount[3], tc) : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        const uint32_t b = first + (uint32_t)(m * kBlock) + threadIdx.x;
+        if (full[m]) bins[s_at[0] + fo[m]] = b;
+        for (uint32_t k = 0; k < nc[m]; k++) chunks[s_at[1] + co[m] + k] = make_uint2(b, k);
+    }
+}
+
+// A work-group's entry of a work list of n entries: each XCD (blockIdx mod 8)
+// takes a contiguous eighth.  False past the end.
+__device__ __forceinline__ bool list_entry(uint32_t n, uint32_t &e) {
+    const uint32_t per = (n + 7u) / 8u, i = blockIdx.x >> 3;
+    e = (blockIdx.x & 7u) * per + i;
+    return i < per && e < n;
+}
+
 // ---------------------------------------------------------------------------
 // Scatter P2G into per-brick tiles
 // ---------------------------------------------------------------------------
@@ -800,18 +867,19 @@ __device__ __forceinline__ void bscatter_comp(unsigned long long *acc, uint32_t 
 // 32-bit byte offsets (the array addresses stay in scalar registers).
 template <bool OFF32>
 __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
-    const SceneDesc *__restrict__ scenes, int nsc, uint32_t nbin, int per_xcd,
-    const uint32_t *__restrict__ pstart, const uint32_t *__restrict__ gperm, SortedOut copy,
-    float2 *__restrict__ tiles, unsigned long long *__restrict__ tile_rows,
-    unsigned long long *__restrict__ fluid) {
+    const SceneDesc *__restrict__ scenes, int nsc, const uint32_t *__restrict__ bins,
+    const uint32_t *__restrict__ lcount, const uint32_t *__restrict__ pstart,
+    const uint32_t *__restrict__ gperm, SortedOut copy, float2 *__restrict__ tiles,
+    unsigned long long *__restrict__ tile_rows, unsigned long long *__restrict__ fluid) {
     using namespace bscat;
     __shared__ unsigned long long s_acc[NREP][3][3][TN];
     __shared__ uint32_t s_bad[(3 * TN + 7) / 8];
     __shared__ float s_red[NT / 64][3];
     __shared__ unsigned long long s_fluid;
-    // consecutive bricks on one XCD: the combine reads neighbours' tiles
-    const uint32_t gid = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
-    if (gid >= nbin) return;
+    // (consecutive bricks on one XCD: the combine reads neighbours' tiles)
+    uint32_t entry;
+    if (!list_entry(gld(lcount, 2), entry)) return;
+    const uint32_t gid = gld(bins, entry);
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const SceneDesc &sd = scenes[scene_of(scenes, nsc, gid, [](const SceneDesc &d) { return d.kb0; })];
     const uint32_t lb = gid - sd.kb0;
@@ -832,10 +900,6 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         return;
     }
     const uint32_t q0 = gld(pstart, gid), N = gld(pstart, gid + 1) - q0;
-    if (N == 0) {
-        if (t == 0) fluid[gid] = 0ull;
-        return;
-    }
     int bxi, byi, bzi;
     brick_coords(sd, lb, bxi, byi, bzi);
     const int o[3] = {4 * bxi, 4 * byi, 4 * bzi};
@@ -1527,23 +1591,34 @@ __device__ __forceinline__ void g2p_bbrick(const StepG2P &a, const MacGrid &g, i
         run(std::false_type{});
 }
 
-// One work-group per G2P brick of 8^3 cells of any scene.
+// The shares of G2P bricks that k_step_lists listed.
+struct G2PWork {
+    const uint2 *chunks;
+    const uint32_t *lcount;
+    uint32_t chunk;
+};
+
+// One work-group per listed share of a G2P brick of 8^3 cells of any scene.
 template <int ST, bool P2, bool SIMPLE>
 __device__ __forceinline__ void g2p_bb_kernel(const SceneDesc *__restrict__ scenes, int nsc,
-                                              Sorted so, int keep_order, uint32_t nbrick,
-                                              int per_xcd, const uint32_t *__restrict__ pstart,
+                                              Sorted so, int keep_order, G2PWork work,
+                                              const uint32_t *__restrict__ pstart,
                                               const uint32_t *__restrict__ perm, G2PSlow slow) {
-    // consecutive bricks share box halos: keep them on one XCD
-    const uint32_t gid = (blockIdx.x & 7u) * (uint32_t)per_xcd + (blockIdx.x >> 3);
-    if (gid >= nbrick) return;
-    const SceneDesc &sd = scenes[scene_of(scenes, nsc, gid, [](const SceneDesc &d) { return d.g0; })];
+    // (consecutive bricks share box halos: they are on one XCD)
+    uint32_t entry;
+    if (!list_entry(work.lcount[3], entry)) return;
+    const uint2 ch = work.chunks[entry];
+    const uint32_t b0 = ch.x;
+    const SceneDesc &sd = scenes[scene_of(scenes, nsc, b0, [](const SceneDesc &d) { return d.kb0; })];
     const StepG2P a = g2p_view(sd, so, keep_order);
     const MacGrid g = mac_view(sd);
-    const int lg = (int)(gid - sd.g0);
+    const int lg = (int)((b0 - sd.kb0) >> 3);
     const int gx = lg % sd.gbx, gy = (lg / sd.gbx) % sd.gby, gz = lg / (sd.gbx * sd.gby);
-    const uint32_t b0 = sd.kb0 + 8u * (uint32_t)lg;
-    g2p_bbrick<ST, 8, P2, SIMPLE>(a, g, gx * 8, gy * 8, gz * 8, pstart[b0], pstart[b0 + 8], perm,
-                                  slow);
+    const uint32_t q0 = pstart[b0], N = pstart[b0 + 8] - q0;
+    const uint32_t nc = (N + work.chunk - 1u) / work.chunk;
+    const uint32_t s0 = (uint32_t)((uint64_t)N * ch.y / nc);
+    const uint32_t s1 = (uint32_t)((uint64_t)N * (ch.y + 1u) / nc);
+    g2p_bbrick<ST, 8, P2, SIMPLE>(a, g, gx * 8, gy * 8, gz * 8, q0 + s0, q0 + s1, perm, slow);
 }
 
 // One work-group per P2G brick (4^3 cells, one bin of the sort) of any scene.
@@ -1568,20 +1643,18 @@ __device__ __forceinline__ void g2p_b4_kernel(const SceneDesc *__restrict__ scen
 // Trilinear: five work-groups per CU fit in LDS; five waves per SIMD.
 template <bool P2, bool SIMPLE>
 __global__ __launch_bounds__(gbrick::NT, 5) void k_flip_g2p_bb_tl(
-    const SceneDesc *__restrict__ scenes, int nsc, Sorted so, int keep_order, uint32_t nbrick,
-    int per_xcd, const uint32_t *__restrict__ pstart, const uint32_t *__restrict__ perm,
-    G2PSlow slow) {
-    g2p_bb_kernel<0, P2, SIMPLE>(scenes, nsc, so, keep_order, nbrick, per_xcd, pstart, perm, slow);
+    const SceneDesc *__restrict__ scenes, int nsc, Sorted so, int keep_order, G2PWork work,
+    const uint32_t *__restrict__ pstart, const uint32_t *__restrict__ perm, G2PSlow slow) {
+    g2p_bb_kernel<0, P2, SIMPLE>(scenes, nsc, so, keep_order, work, pstart, perm, slow);
 }
 
 // Tricubic: three waves per SIMD (168 VGPRs) run about 10% faster than two
 // (256) at the cost of a few bytes of spill.
 template <bool P2, bool SIMPLE>
 __global__ __launch_bounds__(gbrick::NT, 3) void k_flip_g2p_bb_tc(
-    const SceneDesc *__restrict__ scenes, int nsc, Sorted so, int keep_order, uint32_t nbrick,
-    int per_xcd, const uint32_t *__restrict__ pstart, const uint32_t *__restrict__ perm,
-    G2PSlow slow) {
-    g2p_bb_kernel<1, P2, SIMPLE>(scenes, nsc, so, keep_order, nbrick, per_xcd, pstart, perm, slow);
+    const SceneDesc *__restrict__ scenes, int nsc, Sorted so, int keep_order, G2PWork work,
+    const uint32_t *__restrict__ pstart, const uint32_t *__restrict__ perm, G2PSlow slow) {
+    g2p_bb_kernel<1, P2, SIMPLE>(scenes, nsc, so, keep_order, work, pstart, perm, slow);
 }
 
 template <bool P2, bool SIMPLE>
@@ -1712,18 +1785,30 @@ void flip_step_brick(const StepBatch &s, const BrickSort &bs, hipStream_t st, hi
     }
     if (ev) GFSX_HIP(hipEventRecord(ev[1], st));
 
-    const int per_xcd = (int)((nbin + 7) / 8);
+    // Shares of 256 to 4096 particles, about 16 per CU where the step is
+    // small: tricubic, 4M particles, the step with 8 / 16 / 32 / 64 per CU 553 /
+    // 538 / 549 / 624 us (each share stages its boxes); at 43M shares of up to
+    // 2048 / 4096 2421 / 2384 us.
+    const uint32_t chunk = (uint32_t)std::min<int64_t>(
+        std::max<int64_t>((n / ((int64_t)s.num_cu * 4 * 4) + 255) / 256 * 256, 256), 4096);
+    // the sort's lists are free now: bins with particles in mid, shares of
+    // G2P bricks (at most n / chunk + nbin / 8, 8 bytes each) in list2 or,
+    // for fewer particles than a quarter of the bins, huge
+    uint2 *chunks = reinterpret_cast<uint2 *>(4 * n >= (int64_t)nbin + n / 32 + 64 ? bs.list2 : bs.huge);
+    hipLaunchKernelGGL(k_step_lists, dim3(grid_for(nbin, 4 * kBlock)), dim3(kBlock), 0, st, s.scenes_dev,
+                       nsc, nbin, chunk, (const uint32_t *)bs.pstart, s.tile_rows,
+                       std::max<int64_t>(s.tot.nrm, 1), bs.fluid, bs.mid, chunks, bs.lcount);
+    GFSX_LAUNCH_CHECK();
     // gather with sorted copies: the P2G kernel writes them
     SortedOut p2g_copy;
     for (int c = 0; c < 3; c++) {
         p2g_copy.x[c] = s.gather && s.xs[0] ? s.xs[c] : nullptr;
         p2g_copy.v[c] = s.gather && s.xs[0] ? s.vs[c] : nullptr;
     }
-    fill_u32((uint32_t *)s.tile_rows, 0u, 2 * std::max<int64_t>(s.tot.nrm, 1), st);
     hipLaunchKernelGGL(s.tot.n < ((int64_t)1 << 30) ? k_p2g_bscatter<true> : k_p2g_bscatter<false>,
-                       dim3((unsigned)(8 * (int64_t)per_xcd)), dim3(bscat::NT), 0, st,
-                       s.scenes_dev, nsc, nbin, per_xcd, (const uint32_t *)bs.pstart,
-                       s.gather ? (const uint32_t *)bs.perm : nullptr, p2g_copy, s.tiles,
+                       dim3(8 * grid_for(std::min<int64_t>(nbin, n), 8)), dim3(bscat::NT), 0, st,
+                       s.scenes_dev, nsc, (const uint32_t *)bs.mid, (const uint32_t *)bs.lcount,
+                       (const uint32_t *)bs.pstart, s.gather ? (const uint32_t *)bs.perm : nullptr, p2g_copy, s.tiles,
                        s.tile_rows, bs.fluid);
     GFSX_LAUNCH_CHECK();
     if (nsc > 1 && !s.r0s) throw Error("gfsx: the combine of several scenes needs their wave offsets");
@@ -1752,8 +1837,6 @@ void flip_step_brick(const StepBatch &s, const BrickSort &bs, hipStream_t st, hi
     bool simple = !so.perm && !s.keep_order && s.tot.n < ((int64_t)1 << 30);
     for (const auto &d : s.scenes) simple = simple && !d.id_out;
     if (s.g2p_variant == 0) {
-        const uint32_t nbrick = (uint32_t)s.tot.ng2p;
-        const int gper = (int)((nbrick + 7) / 8);
         G2PSlow slow;
         slow.slots = bs.slow_slots;
         slow.count = bs.slow_count;
@@ -1773,8 +1856,9 @@ void flip_step_brick(const StepBatch &s, const BrickSort &bs, hipStream_t st, hi
                                      : (simple ? k_flip_g2p_bb_tl<false, true> : k_flip_g2p_bb_tl<false, false>))
                              : (s.p2 ? (simple ? k_flip_g2p_bb_tc<true, true> : k_flip_g2p_bb_tc<true, false>)
                                      : (simple ? k_flip_g2p_bb_tc<false, true> : k_flip_g2p_bb_tc<false, false>));
-            hipLaunchKernelGGL(kern, dim3((unsigned)(8 * gper)), dim3(gbrick::NT), 0, st,
-                               s.scenes_dev, nsc, so, s.keep_order, nbrick, gper,
+            const G2PWork work = {chunks, bs.lcount, chunk};
+            hipLaunchKernelGGL(kern, dim3(8 * grid_for((int64_t)s.tot.ng2p + n / chunk, 8)),
+                               dim3(gbrick::NT), 0, st, s.scenes_dev, nsc, so, s.keep_order, work,
                                (const uint32_t *)bs.pstart, (const uint32_t *)bs.perm, slow);
         }
         GFSX_LAUNCH_CHECK();

@@ -506,7 +506,7 @@ struct BrickSort {
     uint32_t *list2;             // the same ordered, for bins of many runs
     uint32_t *runbase;           // TILE per binning work-group: each chunk's first slot
     uint32_t *mid, *huge;        // bins of 17..256 runs, of more
-    uint32_t *lcount;            // 2: entries of mid and huge
+    uint32_t *lcount;            // 4: entries of mid and huge, then of the step's two work lists
     unsigned long long *scan_scratch;
     uint32_t *perm;              // nullable: sort slot -> global particle index
     unsigned long long *fluid;   // per bin: the cells of the brick that hold a particle
