@@ -863,6 +863,14 @@ __device__ __forceinline__ void bscatter_comp(unsigned long long *acc, uint32_t 
             }
 }
 
+// ilogb(2^62 / y) for a normal y > 0, without the division: 62 - e when y is
+// 2^e, else 61 - e with e its exponent (2^62 / y then lies strictly below
+// 2^(62 - e), by more than its rounding).
+__device__ __forceinline__ int scale_exp(double y) {
+    const uint64_t b = (uint64_t)__double_as_longlong(y);
+    return 61 + 1023 - (int)(b >> 52) + (int)((b & 0xFFFFFFFFFFFFFull) == 0ull);
+}
+
 // OFF32: fewer than 2^30 sort slots, so that particle arrays are indexed by
 // 32-bit byte offsets (the array addresses stay in scalar registers).
 template <bool OFF32>
@@ -872,10 +880,10 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
     const uint32_t *__restrict__ gperm, SortedOut copy, float2 *__restrict__ tiles,
     unsigned long long *__restrict__ tile_rows, unsigned long long *__restrict__ fluid) {
     using namespace bscat;
-    __shared__ unsigned long long s_acc[NREP][3][3][TN];
+    __shared__ __align__(16) unsigned long long s_acc[NREP][3][3][TN];
     __shared__ uint32_t s_bad[(3 * TN + 7) / 8];
-    __shared__ float s_red[NT / 64][3];
-    __shared__ unsigned long long s_fluid;
+    __shared__ uint32_t s_red[NT / 64][3];
+    __shared__ uint8_t s_cell[64];   // the brick's cells that hold a particle
     // (consecutive bricks on one XCD: the combine reads neighbours' tiles)
     uint32_t entry;
     if (!list_entry(gld(lcount, 2), entry)) return;
@@ -931,10 +939,15 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         for (int c = 0; c < 3; c++) st(copy.v[c], q, v[c]);
     };
     {
-        unsigned long long *z = &s_acc[0][0][0][0];
-        for (int e = t; e < NREP * 3 * 3 * TN; e += NT) z[e] = 0ull;
-        for (int e = t; e < (3 * TN + 7) / 8; e += NT) s_bad[e] = 0u;
-        if (t == 0) s_fluid = 0ull;
+        static_assert(NREP * 3 * 3 * TN % 2 == 0 && NT >= 64 + (3 * TN + 7) / 8, "the zero fill");
+        ulonglong2 *z = reinterpret_cast<ulonglong2 *>(&s_acc[0][0][0][0]);
+#pragma unroll
+        for (int m = 0; m < (NREP * 3 * 3 * TN / 2 + NT - 1) / NT; m++) {
+            const int e = t + m * NT;
+            if (e < NREP * 3 * 3 * TN / 2) z[e] = make_ulonglong2(0ull, 0ull);
+        }
+        if (t < 64) s_cell[t] = 0;
+        else if (t < 64 + (3 * TN + 7) / 8) s_bad[t - 64] = 0u;
     }
 
     // pass 1: the largest |v| below 2^90 per component; the first PRE
@@ -970,30 +983,28 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
             if (av < kBig) vm[c] = fmaxf(vm[c], av);
         }
     }
+    // (non-negative floats order like their bits)
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        float v = vm[c];
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
-        if (lane == 0) s_red[wave][c] = v;
+        const uint32_t v = wave_max_lane63(__float_as_uint(vm[c]));
+        if (lane == 63) s_red[wave][c] = v;
     }
     __syncthreads();
-    const int eW = ilogb(4611686018427387904.0 / (double)N);   // 2^62 / N
+    const int eW = scale_exp((double)N);
     int eS[3];
     float ratio[3];
 #pragma unroll
     for (int c = 0; c < 3; c++) {
-        float v = 0.0f;
+        uint32_t vb = 0u;
 #pragma unroll
-        for (int w = 0; w < NT / 64; w++) v = fmaxf(v, s_red[w][c]);
-        eS[c] = v > 0.0f ? min(ilogb(4611686018427387904.0 / ((double)N * (double)v)), eW + 100) : eW;
+        for (int w = 0; w < NT / 64; w++) vb = max(vb, s_red[w][c]);
+        eS[c] = vb ? min(scale_exp((double)N * (double)__uint_as_float(vb)), eW + 100) : eW;
         ratio[c] = ldexpf(1.0f, eS[c] - eW);
     }
     const float c0 = ldexpf(5.0f / 9.0f, eW - 32), c1 = ldexpf(4.0f / 9.0f, eW - 32);
 
     // pass 2: scatter
     const int rep = lane & (NREP - 1);
-    unsigned long long fl = 0ull;
     auto scatter = [&](float x, float y, float z, const float v[3]) {
         const AxisCoords ca[3] = {axis_coords(x, inv_dx), axis_coords(y, inv_dx),
                                   axis_coords(z, inv_dx)};
@@ -1012,16 +1023,17 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         // the particle's cell is fluid (fluidsimulation.cpp:2010-2017)
         if ((unsigned)ca[0].ia < (unsigned)ni && (unsigned)ca[1].ia < (unsigned)nj &&
             (unsigned)ca[2].ia < (unsigned)nk)
-            fl |= 1ull << ((ca[0].ia - o[0]) + 4 * (ca[1].ia - o[1]) + 16 * (ca[2].ia - o[2]));
+            s_cell[(ca[0].ia - o[0]) + 4 * (ca[1].ia - o[1]) + 16 * (ca[2].ia - o[2])] = 1;
+        // tile positions; a particle in one of the brick's own cells keeps
+        // every corner in the tiles (ib is ia or ia - 1)
         int tc[3][3];
         bool fast = true;
 #pragma unroll
-        for (int c = 0; c < 3; c++)
+        for (int a = 0; a < 3; a++) {
+            fast = fast && (unsigned)(ca[a].ia - o[a]) <= 3u;
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                tc[c][a] = a == c ? ca[a].ia - o[a] : ca[a].ib - o[a] + 1;
-                fast = fast && (unsigned)tc[c][a] <= (a == c ? 3u : 4u);
-            }
+            for (int c = 0; c < 3; c++) tc[c][a] = a == c ? ca[a].ia - o[a] : ca[a].ib - o[a] + 1;
+        }
         bool bad[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -1055,15 +1067,6 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         if (copies) put(q0 + s, x, y, z, v);
         scatter(x, y, z, v);
     }
-    {
-        uint32_t lo = (uint32_t)fl, hi = (uint32_t)(fl >> 32);
-#pragma unroll
-        for (int d = 32; d > 0; d >>= 1) {
-            lo |= __shfl_xor(lo, d, 64);
-            hi |= __shfl_xor(hi, d, 64);
-        }
-        if (lane == 0 && (lo | hi)) atomicOr(&s_fluid, ((unsigned long long)hi << 32) | lo);
-    }
     __syncthreads();
 
     // the copies summed, back to float, out to the tile grids: one
@@ -1073,6 +1076,8 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         constexpr int SX = tsx(C), SY = tsy(C), SZ = tsz(C);
         const TileGrid tg = tile_grid(sd, C);
         const int es = eS[C];
+        float2 *tile = tiles + tile_at(tg, bxi * SX, byi * SY, bzi * SZ);
+        const uint32_t ry = (uint32_t)tg.tx, rz = (uint32_t)tg.tx * (uint32_t)tg.ty;
         for (int nd = t; nd < TN; nd += NT) {
             unsigned long long Sp = 0, Sn = 0, W = 0;
 #pragma unroll
@@ -1091,18 +1096,21 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
                 else Sf = (badb & BAD_PINF) ? INFINITY : -INFINITY;
             }
             const int tz = nd / (SX * SY), ty = (nd / SX) % SY, tx = nd % SX;
-            tiles[tile_at(tg, bxi * SX + tx, byi * SY + ty, bzi * SZ + tz)] = make_float2(Sf, Wf);
+            tile[(uint32_t)tx + ry * (uint32_t)ty + rz * (uint32_t)tz] = make_float2(Sf, Wf);
         }
     };
     flush(std::integral_constant<int, 0>());
     flush(std::integral_constant<int, 1>());
     flush(std::integral_constant<int, 2>());
+    if (t < 64) {
+        const unsigned long long fl = __ballot(s_cell[t] != 0);
+        if (t == 0) fluid[gid] = fl;
+    }
     if (t == 0) {
         // the tile is written: its brick's bit in the occupied-brick mask
         atomicOr(&tile_rows[sd.rm0 + (uint32_t)sd.rmw * ((uint32_t)byi + (uint32_t)sd.nby * (uint32_t)bzi) +
                             (uint32_t)(bxi >> 6)],
                  1ull << (bxi & 63));
-        fluid[gid] = s_fluid;
     }
 }
 

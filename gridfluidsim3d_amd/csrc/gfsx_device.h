@@ -8,6 +8,7 @@
 #include "gfsx_sample.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace gfsx {
 
@@ -23,6 +24,22 @@ __device__ __forceinline__ uint32_t wave_inclusive_sum(uint32_t v) {
         uint32_t t = __shfl_up(v, d, 64);
         if (lane >= d) v += t;
     }
+    return v;
+}
+
+// The wave's largest v, valid in lane 63: row shifts, then the rows' last
+// lanes passed on (DPP operands of the maximum: no LDS, no lane addresses).
+__device__ __forceinline__ uint32_t wave_max_lane63(uint32_t v) {
+    auto step = [&](auto ctrl) {
+        v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf,
+                                                         false));
+    };
+    step(std::integral_constant<int, 0x111>());   // row_shr:1
+    step(std::integral_constant<int, 0x112>());   // row_shr:2
+    step(std::integral_constant<int, 0x114>());   // row_shr:4
+    step(std::integral_constant<int, 0x118>());   // row_shr:8
+    step(std::integral_constant<int, 0x142>());   // row_bcast:15
+    step(std::integral_constant<int, 0x143>());   // row_bcast:31
     return v;
 }
 
