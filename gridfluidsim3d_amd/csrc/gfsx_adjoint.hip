@@ -216,13 +216,13 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect(StepAdjoint a) {
 
 // The P2G bricks (4x4x4 cells) of the forward step's brick sort, one
 // work-group each, over the brick's particles (one contiguous range of
-// sorted slots).  A tile of every face index within M
-// cells of the brick's
+// sorted slots).  A tile of every face index within M cells of the brick's
 // trilinear footprint holds the grid after the body force and the
 // normalised P2G result (0 for faces outside the arrays, which is what an
-// out-of-range sample reads).  Samples whose corners leave the tile (a stage
-// moved more than M cells) use global memory.  Work-groups past the bricks
-// take the particles of the overflow bin (outside the bin grid).
+// out-of-range sample reads).  A particle with a stage whose corners leave
+// the tile (it moved more than M cells) goes to a list, which k_adj_slow
+// takes through global memory, as it does the overflow bin (particles outside
+// the bin grid).
 //
 // Every sample's adjoint is computed, dL/dx and dL/dv are written, and
 // lam * weight is added as a 64-bit fixed-point integer, scale
@@ -232,12 +232,22 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect(StepAdjoint a) {
 // sums do not depend on the order of the adds, so the grid adjoints are the
 // same on every run; no face can overflow: it receives at most 5n terms of
 // magnitude at most 2^61 / (5n).
+//
+// The P2G adjoint takes only the sum dL/dg + dL/dn of a face, so both go to
+// one accumulator: the samples of g and n at x0 share their corners and
+// weights, and their adjoints are added first (h/6 A + h/2 lq + r_pic V: the
+// two FLIP terms cancel before any rounding), 96 LDS atomics a particle
+// instead of 120 and half the sums to keep, flush and read.  The cell
+// coordinates of a stage serve its sample and its adjoint.  2M particles of
+// a 96^3 slab: 220 -> 191 us (VALU and LDS waits; 24.6 KB of LDS and 109
+// VGPRs, four work-groups a CU; 5 or 6 waves per SIMD by launch bounds: no
+// faster, and 3% slower).
 namespace abrick {
 constexpr int BX = 4, BY = 4, BZ = 4;   // the P2G bricks of the forward's brick sort
 constexpr int M = 1;
 constexpr int TX = BX + 2 + 2 * M, TY = BY + 2 + 2 * M, TZ = BZ + 2 + 2 * M;
 constexpr int TN = TX * TY * TZ;
-constexpr int NEXTRA = 16;
+constexpr int SLOW_BLOCKS = 256;
 }  // namespace abrick
 
 // An upper bound B on |lam| over every sample adjoint of adj_particle, from
@@ -285,58 +295,25 @@ __device__ __forceinline__ unsigned long long to_fixed(float v, double scale) {
     return (unsigned long long)(__double_as_longlong(y) - __double_as_longlong(kMagic));
 }
 
-__global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, AdjointSort so,
-                                                             uint32_t nbrick) {
+// A stage position in a brick's tile: the lower corner of each component's
+// stencil (tile index) and the fractions along x, y, z, unshifted (a) and
+// half-shifted (b); in: in the grid (else the sample is the constant 0).
+struct TileLoc {
+    int l[3];
+    float ta[3], tb[3];
+    bool in;
+};
+
+__global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, AdjointSort so) {
     using namespace abrick;
     __shared__ float gt[6 * TN];                 // g (0-2) and n (3-5) on the tile
-    __shared__ unsigned long long at[6 * TN];    // fixed-point dL/dg, dL/dn
+    __shared__ unsigned long long at[3 * TN];    // fixed-point dL/dg + dL/dn
     const int tid = threadIdx.x;
     const uint32_t bid = blockIdx.x;
-    const double scale = fixed_scale(so.bound, a);
-    auto fixed_sink = [&](int arr, int, int, int, uint32_t o, float v) {
-        atomicAdd(so.fx + (arr < 3 ? a.lg[arr] - a.lg[0] : a.ln[arr - 3] - a.lg[0]) + o,
-                  to_fixed(v, scale));
-    };
-    // global path of one sample (outside the tile, or an overflow particle)
-    auto global_adjoint = [&](int base, const float q[3], const float lam[3], float lq[3]) {
-        mac_adjoint(a, base == 0 ? a.g : a.old, base, q, lam, lq, fixed_sink);
-    };
-    struct GlobalFixed {
-        const GlobalPolicy &gp;
-        decltype(global_adjoint) &ga;
-        __device__ void sample(const float q[3], float out[3]) const { gp.sample(q, out); }
-        __device__ void adjoint(int base, const float q[3], const float lam[3], float lq[3]) const {
-            ga(base, q, lam, lq);
-        }
-    };
-    const GlobalPolicy gpol{a};
-    const GlobalFixed gfix{gpol, global_adjoint};
-    auto finish = [&](uint32_t q, const float lx[3], const float av[3]) {
-        const uint32_t p = so.perm[q];
-        for (int c = 0; c < 3; c++) {
-            a.gx[c][p] = lx[c];
-            a.gv[c][p] = a.r_flip * av[c];
-        }
-    };
-    if (bid >= nbrick) {
-        // overflow bin: grid-stride over its slots
-        const uint32_t q0 = so.pstart[so.nbb], q1 = so.pstart[so.nbb + 1];
-        for (uint32_t q = q0 + (bid - nbrick) * kBlock + tid; q < q1; q += NEXTRA * kBlock) {
-            const uint32_t p = so.perm[q];
-            float x0[3], ax[3], av[3], lx[3];
-            for (int c = 0; c < 3; c++) {
-                x0[c] = so.xs[c][q];
-                ax[c] = a.ax[c][p];
-                av[c] = a.av[c][p];
-            }
-            adj_particle(a, x0, ax, av, lx, gfix);
-            finish(q, lx, av);
-        }
-        return;
-    }
     // brick bid: bin bid of the sort, one contiguous range of slots
     const uint32_t q0 = so.pstart[bid], total = so.pstart[bid + 1] - q0;
     if (total == 0) return;   // uniform across the work-group
+    const double scale = fixed_scale(so.bound, a);
     const uint32_t g = bid >> 3, sub = bid & 7u;
     const int bx = (int)(2 * (g % (uint32_t)so.gbx) + (sub & 1u));
     const int by = (int)(2 * ((g / (uint32_t)so.gbx) % (uint32_t)so.gby) + ((sub >> 1) & 1u));
@@ -369,40 +346,62 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
 #pragma unroll
         for (int m = 0; m < PER; m++) {
             const int e = tid + m * kBlock;
-            if (e < 6 * TN) {
-                gt[e] = v[m];
-                at[e] = 0ull;
-            }
+            if (e < 6 * TN) gt[e] = v[m];
+            if (e < 3 * TN) at[e] = 0ull;
         }
     }
     __syncthreads();
 
-    // local flat index of lower corner (i,j,k), or -1 when a corner leaves the tile
-    auto local = [&](int i, int j, int k) -> int {
-        const int li = i - ox, lj = j - oy, lk = k - oz;
-        return ((unsigned)li < (unsigned)(TX - 1) && (unsigned)lj < (unsigned)(TY - 1) &&
-                (unsigned)lk < (unsigned)(TZ - 1)) ? li + TX * (lj + TY * lk) : -1;
-    };
-    auto in_grid = [&](const float q[3]) {
-        return q[0] >= 0.0f && q[1] >= 0.0f && q[2] >= 0.0f && q[0] < a.mac.limf[0] &&
+    // false when a corner leaves the tile
+    auto locate = [&](const float q[3], TileLoc &p) -> bool {
+        p.in = q[0] >= 0.0f && q[1] >= 0.0f && q[2] >= 0.0f && q[0] < a.mac.limf[0] &&
                q[1] < a.mac.limf[1] && q[2] < a.mac.limf[2];
+        if (!p.in) return true;
+        const AxisCoords cx = axis_coords(q[0], a.mac.inv_dx);
+        const AxisCoords cy = axis_coords(q[1], a.mac.inv_dx);
+        const AxisCoords cz = axis_coords(q[2], a.mac.inv_dx);
+        // the components' base cells span ib .. ia along each axis, their
+        // corners ib .. ia + 1
+        const int x = cx.ib - ox, y = cy.ib - oy, z = cz.ib - oz;
+        const int dx = cx.ia - cx.ib, dy = cy.ia - cy.ib, dz = cz.ia - cz.ib;
+        if ((unsigned)x >= (unsigned)(TX - 1 - dx) || (unsigned)y >= (unsigned)(TY - 1 - dy) ||
+            (unsigned)z >= (unsigned)(TZ - 1 - dz))
+            return false;
+        const int l = x + TX * (y + TY * z);
+        p.l[0] = l + dx;
+        p.l[1] = l + TX * dy;
+        p.l[2] = l + TX * TY * dz;
+        p.ta[0] = cx.ta;
+        p.ta[1] = cy.ta;
+        p.ta[2] = cz.ta;
+        p.tb[0] = cx.tb;
+        p.tb[1] = cy.tb;
+        p.tb[2] = cz.tb;
+        return true;
     };
-    // trilinear value from the tile, in the order of the forward sampler
-    auto tile_value = [&](int arr, int l, float tx, float ty, float tz) {
-        const float *f = gt + arr * TN + l;
-        const float v000 = f[0], v100 = f[1], v010 = f[TX], v110 = f[TX + 1];
-        const float v001 = f[TX * TY], v101 = f[TX * TY + 1];
-        const float v011 = f[TX * TY + TX], v111 = f[TX * TY + TX + 1];
-        const float c00 = fmaf(tx, v100 - v000, v000);
-        const float c10 = fmaf(tx, v110 - v010, v010);
-        const float c01 = fmaf(tx, v101 - v001, v001);
-        const float c11 = fmaf(tx, v111 - v011, v011);
-        const float c0 = fmaf(ty, c10 - c00, c00);
-        const float c1 = fmaf(ty, c11 - c01, c01);
-        return fmaf(tz, c1 - c0, c0);
+    auto frac = [](const TileLoc &p, int c, int ax) { return ax == c ? p.ta[ax] : p.tb[ax]; };
+    // the grid's sample, in the order of the forward sampler
+    auto sample = [&](const TileLoc &p, float out[3]) {
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            out[c] = 0.0f;
+            if (!p.in) continue;
+            const float tx = frac(p, c, 0), ty = frac(p, c, 1), tz = frac(p, c, 2);
+            const float *f = gt + c * TN + p.l[c];
+            const float v000 = f[0], v100 = f[1], v010 = f[TX], v110 = f[TX + 1];
+            const float v001 = f[TX * TY], v101 = f[TX * TY + 1];
+            const float v011 = f[TX * TY + TX], v111 = f[TX * TY + TX + 1];
+            const float c00 = fmaf(tx, v100 - v000, v000);
+            const float c10 = fmaf(tx, v110 - v010, v010);
+            const float c01 = fmaf(tx, v101 - v001, v001);
+            const float c11 = fmaf(tx, v111 - v011, v011);
+            const float c0 = fmaf(ty, c10 - c00, c00);
+            const float c1 = fmaf(ty, c11 - c01, c01);
+            out[c] = fmaf(tz, c1 - c0, c0);
+        }
     };
-    auto tile_adjoint = [&](int arr, int l, float tx, float ty, float tz, float lam, float dt[3]) {
-        if (lam == 0.0f) return;
+    // lam times the sample's derivatives along the axes
+    auto slope = [&](int arr, int l, float tx, float ty, float tz, float lam, float dt[3]) {
         const float *f = gt + arr * TN + l;
         const float v000 = f[0], v100 = f[1], v010 = f[TX], v110 = f[TX + 1];
         const float v001 = f[TX * TY], v101 = f[TX * TY + 1];
@@ -414,7 +413,11 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
                         sx * tz * (v011 - v001) + tx * tz * (v111 - v101));
         dt[2] += lam * (sx * sy * (v001 - v000) + tx * sy * (v101 - v100) +
                         sx * ty * (v011 - v010) + tx * ty * (v111 - v110));
-        unsigned long long *t = at + arr * TN + l;
+    };
+    // lam times the corner weights into component c's sums
+    auto spread = [&](int c, int l, float tx, float ty, float tz, float lam) {
+        const float sx = 1.0f - tx, sy = 1.0f - ty, sz = 1.0f - tz;
+        unsigned long long *t = at + c * TN + l;
         atomicAdd(t, to_fixed(lam * (sx * sy * sz), scale));
         atomicAdd(t + 1, to_fixed(lam * (tx * sy * sz), scale));
         atomicAdd(t + TX, to_fixed(lam * (sx * ty * sz), scale));
@@ -424,51 +427,72 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         atomicAdd(t + TX * TY + TX, to_fixed(lam * (sx * ty * tz), scale));
         atomicAdd(t + TX * TY + TX + 1, to_fixed(lam * (tx * ty * tz), scale));
     };
-    struct TilePolicy {
-        const StepAdjoint &a;
-        const GlobalFixed &gf;
-        decltype(local) &loc;
-        decltype(in_grid) &ing;
-        decltype(tile_value) &tv;
-        decltype(tile_adjoint) &tadj;
-        __device__ void sample(const float q[3], float out[3]) const {
-            if (!ing(q)) {
-                out[0] = out[1] = out[2] = 0.0f;
-                return;
-            }
-            const AxisCoords cx = axis_coords(q[0], a.mac.inv_dx);
-            const AxisCoords cy = axis_coords(q[1], a.mac.inv_dx);
-            const AxisCoords cz = axis_coords(q[2], a.mac.inv_dx);
-            const int l0 = loc(cx.ia, cy.ib, cz.ib), l1 = loc(cx.ib, cy.ia, cz.ib);
-            const int l2 = loc(cx.ib, cy.ib, cz.ia);
-            if (l0 < 0 || l1 < 0 || l2 < 0) {
-                gf.sample(q, out);
-                return;
-            }
-            out[0] = tv(0, l0, cx.ta, cy.tb, cz.tb);
-            out[1] = tv(1, l1, cx.tb, cy.ta, cz.tb);
-            out[2] = tv(2, l2, cx.tb, cy.tb, cz.ta);
+    // adjoint of the grid's sample at p
+    auto adjoint = [&](const TileLoc &p, const float lam[3], float lq[3]) {
+        if (!p.in) return;
+        float dt[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            if (lam[c] == 0.0f) continue;
+            const float tx = frac(p, c, 0), ty = frac(p, c, 1), tz = frac(p, c, 2);
+            slope(c, p.l[c], tx, ty, tz, lam[c], dt);
+            spread(c, p.l[c], tx, ty, tz, lam[c]);
         }
-        __device__ void adjoint(int base, const float q[3], const float lam[3], float lq[3]) const {
-            if (!ing(q)) return;
-            const AxisCoords cx = axis_coords(q[0], a.mac.inv_dx);
-            const AxisCoords cy = axis_coords(q[1], a.mac.inv_dx);
-            const AxisCoords cz = axis_coords(q[2], a.mac.inv_dx);
-            const int l0 = loc(cx.ia, cy.ib, cz.ib), l1 = loc(cx.ib, cy.ia, cz.ib);
-            const int l2 = loc(cx.ib, cy.ib, cz.ia);
-            if (l0 < 0 || l1 < 0 || l2 < 0) {
-                gf.adjoint(base, q, lam, lq);
-                return;
-            }
-            float dt[3] = {0.0f, 0.0f, 0.0f};
-            tadj(base + 0, l0, cx.ta, cy.tb, cz.tb, lam[0], dt);
-            tadj(base + 1, l1, cx.tb, cy.ta, cz.tb, lam[1], dt);
-            tadj(base + 2, l2, cx.tb, cy.tb, cz.ta, lam[2], dt);
-            const float inv_dx = (float)a.mac.inv_dx;
-            for (int c = 0; c < 3; c++) lq[c] += dt[c] * inv_dx;
-        }
+        // the cell fractions move by 1/dx per unit of x
+        const float inv_dx = (float)a.mac.inv_dx;
+        for (int c = 0; c < 3; c++) lq[c] += dt[c] * inv_dx;
     };
-    const TilePolicy tpol{a, gfix, local, in_grid, tile_value, tile_adjoint};
+    // the walk of adj_particle; false when a stage leaves the tile (nothing
+    // is added then)
+    auto particle = [&](const float x0[3], const float ax[3], const float av[3], float lx[3]) -> bool {
+        float k[3], q[3];
+        TileLoc p1, p2, p3, p4;
+        if (!locate(x0, p1)) return false;
+        sample(p1, k);
+        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_half * k[c];
+        if (!locate(q, p2)) return false;
+        sample(p2, k);
+        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_half * k[c];
+        if (!locate(q, p3)) return false;
+        sample(p3, k);
+        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_full * k[c];
+        if (!locate(q, p4)) return false;
+        float lk[3], lq[3];
+        for (int c = 0; c < 3; c++) {
+            lx[c] = ax[c];
+            lk[c] = a.h_sixth * ax[c];               // k4
+            lq[c] = 0.0f;
+        }
+        adjoint(p4, lk, lq);
+        for (int c = 0; c < 3; c++) {
+            lx[c] += lq[c];
+            lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_full * lq[c];    // k3
+            lq[c] = 0.0f;
+        }
+        adjoint(p3, lk, lq);
+        for (int c = 0; c < 3; c++) {
+            lx[c] += lq[c];
+            lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_half * lq[c];    // k2
+            lq[c] = 0.0f;
+        }
+        adjoint(p2, lk, lq);
+        for (int c = 0; c < 3; c++) lx[c] += lq[c];
+        if (!p1.in) return true;
+        // I(g, x0) has the adjoint k1 + (r_pic + r_flip) av, I(n, x0) -r_flip av
+        float dt[3] = {0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const float k1 = a.h_sixth * ax[c] + a.h_half * lq[c];
+            const float tx = frac(p1, c, 0), ty = frac(p1, c, 1), tz = frac(p1, c, 2);
+            slope(c, p1.l[c], tx, ty, tz, k1 + (a.r_pic + a.r_flip) * av[c], dt);
+            slope(3 + c, p1.l[c], tx, ty, tz, -a.r_flip * av[c], dt);
+            const float both = k1 + a.r_pic * av[c];
+            if (both != 0.0f) spread(c, p1.l[c], tx, ty, tz, both);
+        }
+        const float inv_dx = (float)a.mac.inv_dx;
+        for (int c = 0; c < 3; c++) lx[c] += dt[c] * inv_dx;
+        return true;
+    };
     // blocked mapping: thread t takes items [t*per, (t+1)*per), so the lanes
     // of a wave sit in different cells (fewer same-address LDS atomics)
     const uint32_t per = (total + kBlock - 1) / kBlock;
@@ -481,24 +505,65 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
             ax[c] = a.ax[c][p];
             av[c] = a.av[c][p];
         }
-        adj_particle(a, x0, ax, av, lx, tpol);
-        finish(q, lx, av);
+        if (particle(x0, ax, av, lx)) {
+            for (int c = 0; c < 3; c++) {
+                a.gx[c][p] = lx[c];
+                a.gv[c][p] = a.r_flip * av[c];
+            }
+        } else {
+            so.slow[atomicAdd(so.slow_count, 1u)] = q;
+        }
     }
     __syncthreads();
-    for (int e = tid; e < 6 * TN; e += kBlock) {
+    for (int e = tid; e < 3 * TN; e += kBlock) {
         const unsigned long long v = at[e];
         if (v == 0ull) continue;
-        const int arr = e / TN, l = e - arr * TN;
-        const int c = arr % 3;
+        const int c = e / TN, l = e - c * TN;
         const int i = ox + l % TX, j = oy + (l / TX) % TY, k = oz + l / (TX * TY);
         const int w = ni + (c == 0), h = nj + (c == 1), d = nk + (c == 2);
         // tile entries outside the arrays collect nothing that exists
         if (!((unsigned)i < (unsigned)w && (unsigned)j < (unsigned)h && (unsigned)k < (unsigned)d))
             continue;
         const uint32_t o = (uint32_t)i + (uint32_t)w * ((uint32_t)j + (uint32_t)h * (uint32_t)k);
-        const float *base = c == 0 ? (arr < 3 ? a.lg[0] : a.ln[0])
-                          : c == 1 ? (arr < 3 ? a.lg[1] : a.ln[1]) : (arr < 3 ? a.lg[2] : a.ln[2]);
+        const float *base = c == 0 ? a.lg[0] : c == 1 ? a.lg[1] : a.lg[2];
         atomicAdd(so.fx + (base - a.lg[0]) + o, v);
+    }
+}
+
+// The particles that k_adj_advect_brick left and the overflow bin's, through
+// global memory.
+struct GlobalFixed {
+    GlobalPolicy gp;
+    unsigned long long *fx;
+    double scale;
+    __device__ void sample(const float q[3], float out[3]) const { gp.sample(q, out); }
+    __device__ void adjoint(int base, const float q[3], const float lam[3], float lq[3]) const {
+        const StepAdjoint &a = gp.a;
+        mac_adjoint(a, base == 0 ? a.g : a.old, base, q, lam, lq,
+                    [&](int arr, int, int, int, uint32_t o, float v) {
+                        atomicAdd(fx + (a.lg[arr % 3] - a.lg[0]) + o, to_fixed(v, scale));
+                    });
+    }
+};
+
+__global__ __launch_bounds__(kBlock) void k_adj_slow(StepAdjoint a, AdjointSort so) {
+    const GlobalFixed pol{GlobalPolicy{a}, so.fx, fixed_scale(so.bound, a)};
+    const uint32_t ns = *so.slow_count;
+    const uint32_t o0 = so.pstart[so.nbb], no = so.pstart[so.nbb + 1] - o0;
+    for (uint32_t e = blockIdx.x * kBlock + threadIdx.x; e < ns + no; e += gridDim.x * kBlock) {
+        const uint32_t q = e < ns ? so.slow[e] : o0 + (e - ns);
+        const uint32_t p = so.perm[q];
+        float x0[3], ax[3], av[3], lx[3];
+        for (int c = 0; c < 3; c++) {
+            x0[c] = so.xs[c][q];
+            ax[c] = a.ax[c][p];
+            av[c] = a.av[c][p];
+        }
+        adj_particle(a, x0, ax, av, lx, pol);
+        for (int c = 0; c < 3; c++) {
+            a.gx[c][p] = lx[c];
+            a.gv[c][p] = a.r_flip * av[c];
+        }
     }
 }
 
@@ -525,7 +590,7 @@ __device__ __forceinline__ int face_comp(int64_t f, const int64_t nf[3], int64_t
     return c;
 }
 
-// dL/dg, dL/dn from the fixed-point sums, turned into A and B (written over
+// dL/dg + dL/dn from the fixed-point sums, turned into A and B (written to
 // lg and ln) for one thread per face.
 __global__ __launch_bounds__(kBlock) void k_fixed_to_coeffs(const unsigned long long *fx,
                                                             StepAdjoint a, FaceCount fc,
@@ -533,11 +598,10 @@ __global__ __launch_bounds__(kBlock) void k_fixed_to_coeffs(const unsigned long 
     const int64_t f = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     if (f >= fc.tot) return;
     const double scale = fixed_scale(bound, a);
-    const float lg = (float)((double)(long long)fx[f] / scale);
-    const float ln = (float)((double)(long long)fx[fc.tot + f] / scale);
+    const float both = (float)((double)(long long)fx[f] / scale);
     int64_t l;
     const int c = face_comp(f, fc.nf, l);
-    face_coeffs(lg, ln, a.w[c][l], a.old[c][l], a.lg[c][l], a.ln[c][l]);
+    face_coeffs(both, 0.0f, a.w[c][l], a.old[c][l], a.lg[c][l], a.ln[c][l]);
 }
 
 // bound[0..2] = max |dL/dx'|, max |dL/dv'| over the particles and max |g|
@@ -718,18 +782,19 @@ void flip_step_adjoint(const StepAdjoint &a, const AdjointSort *so, hipStream_t 
             a.ln[0] != a.lg[2] + nf[2] || a.ln[1] != a.ln[0] + nf[0] ||
             a.ln[2] != a.ln[1] + nf[1])
             throw Error("flip_step_adjoint: grid adjoint arrays must be contiguous");
-        fill_u32((uint32_t *)so->fx, 0u, 4 * tot, s);
-        fill_u32(so->bound, 0u, 3, s);
+        fill_u32((uint32_t *)so->fx, 0u, 2 * tot, s);
+        fill_u32(so->bound, 0u, 4, s);   // slow_count too
         // the fixed-point scale's bound, then one work-group per bin of the
-        // brick sort and the overflow bin's
+        // brick sort
         hipLaunchKernelGGL(k_adj_bound, dim3((unsigned)std::min<int64_t>(
                                blocks_for(std::max<int64_t>(a.n, tot)), 1024)),
                            dim3(kBlock), 0, s, a, fc, so->bound);
         GFSX_LAUNCH_CHECK();
         if (a.n > 0) {
             const uint32_t nbrick = so->nbb;
-            hipLaunchKernelGGL(k_adj_advect_brick, dim3(nbrick + abrick::NEXTRA), dim3(kBlock),
-                               0, s, a, *so, nbrick);
+            hipLaunchKernelGGL(k_adj_advect_brick, dim3(nbrick), dim3(kBlock), 0, s, a, *so);
+            GFSX_LAUNCH_CHECK();
+            hipLaunchKernelGGL(k_adj_slow, dim3(abrick::SLOW_BLOCKS), dim3(kBlock), 0, s, a, *so);
             GFSX_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(k_fixed_to_coeffs, dim3(blocks_for(tot)), dim3(kBlock), 0, s,
