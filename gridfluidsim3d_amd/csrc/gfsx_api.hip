@@ -502,11 +502,13 @@ gfsx::SceneDesc scene_desc(const gfsx_scene *sc, const gfsx_step_params *pr, con
 // Runs the step; returns the scenes as laid out (bin grids, offsets).  With
 // carve, every device buffer (and the scene table) comes from that region
 // and nothing is allocated: only the brick pipeline, one scene, no
-// epilogue and no timing events.
+// epilogue and no timing events.  With tape, the sort writes its permutation,
+// bin starts and sorted positions there (one scene, kept order).
 std::vector<gfsx::SceneDesc> flip_step_impl(gfsx_ctx *ctx, const gfsx_scene *scenes,
                                             const gfsx_step_params *params, int nscenes,
                                             const char *who, bool grids_only = false,
-                                            Carve *carve = nullptr) {
+                                            Carve *carve = nullptr,
+                                            const gfsx_step_tape *tape = nullptr) {
     auto ws = [&](int slot, size_t bytes) -> void * {
         return carve ? carve->take(bytes) : ctx->get(slot, bytes);
     };
@@ -557,7 +559,9 @@ std::vector<gfsx::SceneDesc> flip_step_impl(gfsx_ctx *ctx, const gfsx_scene *sce
                params[0].order == GFSX_ORDER_SORTED;
     const bool no_copies = s.gather && ctx->particle_gather == 1;
     for (int c = 0; c < 3; c++) {
-        s.xs[c] = no_copies ? nullptr : wsf(S_XS0 + c, s.tot.n);
+        float *const taped[3] = {tape ? tape->xs : nullptr, tape ? tape->ys : nullptr,
+                                 tape ? tape->zs : nullptr};
+        s.xs[c] = no_copies ? nullptr : tape ? taped[c] : wsf(S_XS0 + c, s.tot.n);
         s.vs[c] = no_copies ? nullptr : wsf(S_VS0 + c, s.tot.n);
     }
     if (ctx->p2g_variant == 4) {
@@ -635,7 +639,11 @@ std::vector<gfsx::SceneDesc> flip_step_impl(gfsx_ctx *ctx, const gfsx_scene *sce
         bool ids = false;
         for (auto &d : s.scenes) ids = ids || d.id_out != nullptr;
         gfsx::BrickSort bs = brick_sort(ws, s.tot.n, s.tot.nblk, (uint32_t)s.tot.nbb,
-                                        s.keep_order || ids || s.gather);
+                                        (s.keep_order || ids || s.gather) && !tape);
+        if (tape) {
+            bs.perm = tape->perm;
+            bs.pstart = tape->start;
+        }
         if (carve) {
             if (carve->used > carve->cap) {
                 std::ostringstream m;
@@ -687,11 +695,11 @@ void copy_out(void *dst, const void *src, size_t bytes, hipStream_t s) {
 // adjoint reads) whatever P2G variant the context has selected.
 std::vector<gfsx::SceneDesc> scatter_step(gfsx_ctx *ctx, const gfsx_scene *sc,
                                           const gfsx_step_params *pr, const char *who,
-                                          bool grids_only) {
+                                          bool grids_only, const gfsx_step_tape *tape = nullptr) {
     const int p2g_variant = ctx->p2g_variant;
     ctx->p2g_variant = 4;
     try {
-        std::vector<gfsx::SceneDesc> laid = flip_step_impl(ctx, sc, pr, 1, who, grids_only);
+        std::vector<gfsx::SceneDesc> laid = flip_step_impl(ctx, sc, pr, 1, who, grids_only, nullptr, tape);
         ctx->p2g_variant = p2g_variant;
         return laid;
     } catch (...) {
@@ -1162,20 +1170,9 @@ void gfsx_flip_step_record(gfsx_ctx *ctx, const gfsx_scene *sc, const gfsx_step_
     guarded(ctx, err, [&] {
         const char *who = "gfsx_flip_step_record";
         check_taped(who, sc, pr, tape);
-        const int64_t n = sc->n;
-        const std::vector<gfsx::SceneDesc> laid = scatter_step(ctx, sc, pr, who, false);
-        if (n > 0) {
-            const size_t b = sizeof(float) * (size_t)n;
-            GFSX_HIP(hipMemcpyAsync(tape->perm, ctx->buf[S_PERM], sizeof(uint32_t) * (size_t)n, hipMemcpyDeviceToDevice,
-                                    ctx->stream));
-            float *xs[3] = {tape->xs, tape->ys, tape->zs};
-            for (int c = 0; c < 3; c++)
-                GFSX_HIP(hipMemcpyAsync(xs[c], ctx->buf[S_XS0 + c], b, hipMemcpyDeviceToDevice,
-                                        ctx->stream));
-            GFSX_HIP(hipMemcpyAsync(tape->start, ctx->buf[S_K_PSTART],
-                                    sizeof(uint32_t) * (size_t)tape->starts,
-                                    hipMemcpyDeviceToDevice, ctx->stream));
-        }
+        // the step's sort writes the tape (tape->starts is its bin starts' count)
+        const std::vector<gfsx::SceneDesc> laid =
+            scatter_step(ctx, sc, pr, who, false, sc->n > 0 ? tape : nullptr);
         tape->gbx = laid[0].gbx;
         tape->gby = laid[0].gby;
     });
