@@ -940,17 +940,6 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
 #pragma unroll
         for (int c = 0; c < 3; c++) st(copy.v[c], q, v[c]);
     };
-    // pass 1: the largest |v| below 2^90 per component; the first PRE
-    // particles of each thread stay in registers
-    float px[PRE], py[PRE], pz[PRE], pv[PRE][3];
-    float vm[3] = {0.0f, 0.0f, 0.0f};
-    uint32_t pq[PRE];
-#pragma unroll
-    for (int m = 0; m < PRE; m++) {
-        const uint32_t s = (uint32_t)(t + m * NT);
-        pq[m] = at(q0 + (s < N ? s : 0u));
-    }
-    // (the tiles cleared while the permutation is on its way)
     {
         static_assert(NREP * 3 * 3 * TN % 2 == 0 && NT >= 64 + (3 * TN + 7) / 8, "the zero fill");
         ulonglong2 *z = reinterpret_cast<ulonglong2 *>(&s_acc[0][0][0][0]);
@@ -962,9 +951,15 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         if (t < 64) s_cell[t] = 0;
         else if (t < 64 + (3 * TN + 7) / 8) s_bad[t - 64] = 0u;
     }
+
+    // pass 1: the largest |v| below 2^90 per component; the first PRE
+    // particles of each thread stay in registers
+    float px[PRE], py[PRE], pz[PRE], pv[PRE][3];
+    float vm[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int m = 0; m < PRE; m++) {
-        const uint32_t q = pq[m];
+        const uint32_t s = (uint32_t)(t + m * NT);
+        const uint32_t q = at(q0 + (s < N ? s : 0u));
         px[m] = ld(xp, q);
         py[m] = ld(yp, q);
         pz[m] = ld(zp, q);
