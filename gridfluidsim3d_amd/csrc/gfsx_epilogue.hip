@@ -4,22 +4,23 @@
 // After the P2G gather has written the normalised values n and the weights
 // W of every face (no body force yet):
 //
-//   1. k_fs_layers_init / k_fs_dilate: the cell layer grid of
+//   1. k_fs_layers: the cell layer grid of
 //      MACVelocityField::extrapolateVelocityField (macvelocityfield.cpp:
 //      577-664): fluid cells (a particle, not solid; fluidsimulation.cpp:
 //      1990-2017) 0, then one 6-neighbour dilation per layer through
-//      non-solid cells; solid cells are marked -2 so that no test matches
-//      them.
-//   2. k_fs_fill: FluidSimulation::_advectVelocityFieldU/V/W
+//      non-solid cells, up to seven layers per launch on bit rows in LDS;
+//      solid cells are marked -2 so that no test matches them.
+//   2. k_fs_faces, the fill: FluidSimulation::_advectVelocityFieldU/V/W
 //      (fluidsimulation.cpp:2597-2730): faces bordering fluid keep n where
 //      W > 1e-9 (isValueSet, :2575-2585), else the FP64 average of their 26
 //      neighbours (|n| > 0 for U, :2630; isValueSet for V, W, :2675,2720);
 //      other faces 0.  The snapshot takes that field; the field gets the
-//      body force on faces bordering fluid (:2766-2805, 3306).
-//   3. k_fs_classify: each face's extrapolation layer (at most one) and its
-//      neighbours bordering the layer before; k_fs_extrapolate, one launch
-//      per layer L that changes the faces of layer L only: on both the
-//      snapshot and
+//      body force on faces bordering fluid (:2766-2805, 3306).  And the
+//      classification: each face's extrapolation layer (at most one) and its
+//      neighbours bordering the layer before, listed by layer per segment of
+//      SEG faces.
+//   3. k_fs_extrapolate, one launch per layer L that changes the listed faces
+//      of layer L only: on both the snapshot and
 //      the field (:3307, 3334), faces that border layer L, not layer L-1 and
 //      no solid cell take the FP64 average of their 6 same-component
 //      neighbours that border layer L-1, or 0 when that sum is 0
@@ -27,6 +28,11 @@
 //      never border layer L-1 and the faces read always do, so the launch
 //      reads only values of earlier layers, as the reference's in-place loop
 //      does.
+//
+// Bound: latency and the passes over all faces, of which one is left (the
+// fill reads two floats and writes two per face).  157x93x121, 5.3M faces,
+// seven layers: 280 us with a launch over all cells per dilation (77), a fill
+// (30), a classification (36) and a launch over all faces per layer (130).
 //
 // Everything here is integer work or a fixed-order FP64 sum per face:
 // results are bit-identical to the sequential restatement.
@@ -61,41 +67,24 @@ __device__ __forceinline__ bool face_borders(const FsEpilogue &e, int c, int i, 
     return layer_at(e, i, j, k) == v;
 }
 
-// component and index of flattened face f (u faces, then v, then w);
-// every face count is below 2^31, so 32-bit arithmetic is exact
-__device__ __forceinline__ void face_of(const FsEpilogue &e, uint32_t f, int &c, int &i, int &j,
-                                        int &k, int d[3]) {
-    const uint32_t f0 = (uint32_t)(e.ni + 1) * (uint32_t)e.nj * (uint32_t)e.nk;
-    const uint32_t f1 = (uint32_t)e.ni * (uint32_t)(e.nj + 1) * (uint32_t)e.nk;
-    c = f < f0 ? 0 : (f < f0 + f1 ? 1 : 2);
-    const uint32_t l = c == 0 ? f : (c == 1 ? f - f0 : f - f0 - f1);
-    d[0] = e.ni + (c == 0);
-    d[1] = e.nj + (c == 1);
-    d[2] = e.nk + (c == 2);
-    const uint32_t row = l / (uint32_t)d[0];
-    i = (int)(l - row * (uint32_t)d[0]);
-    j = (int)(row % (uint32_t)d[1]);
-    k = (int)(row / (uint32_t)d[1]);
-}
+// ---- the cell layers
 
-__device__ __forceinline__ void cell_of_index(const FsEpilogue &e, uint32_t t, int &i, int &j,
-                                              int &k) {
-    const uint32_t row = t / (uint32_t)e.ni;
-    i = (int)(t - row * (uint32_t)e.ni);
-    j = (int)(row % (uint32_t)e.nj);
-    k = (int)(row / (uint32_t)e.nj);
-}
+namespace lay {
+constexpr int H = 7;                       // layers per launch: the halo of a tile
+constexpr int TX = 64 - 2 * H, TY = 8, TZ = 8;   // cells of a tile: rows of 64 bits with the halo
+constexpr int RY = TY + 2 * H, RZ = TZ + 2 * H, ROWS = RY * RZ;
+constexpr int NT = 512;
+constexpr int AHEAD = 8;                   // rows a wave loads at a time
+}  // namespace lay
 
-__global__ __launch_bounds__(kBlock) void k_fs_layers_init(FsEpilogue e) {
-    const int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    const int64_t ncell = (int64_t)e.ni * e.nj * e.nk;
-    if (t >= ncell) return;
-    int i, j, k;
-    cell_of_index(e, (uint32_t)t, i, j, k);
-    int8_t v;
-    if (e.solid && e.solid[t]) {
-        v = kSolid;
-    } else if (e.fluid) {
+// The state of cell (i,j,k) before any dilation: -3 outside the grid, kSolid,
+// 0 fluid, -1 neither.
+__device__ __forceinline__ int cell_state(const FsEpilogue &e, int i, int j, int k) {
+    if ((unsigned)i >= (unsigned)e.ni || (unsigned)j >= (unsigned)e.nj || (unsigned)k >= (unsigned)e.nk)
+        return -3;
+    const uint32_t t = (uint32_t)i + (uint32_t)e.ni * ((uint32_t)j + (uint32_t)e.nj * (uint32_t)k);
+    bool fluid;
+    if (e.fluid) {
         // the cell's bit in its P2G brick's mask (brick bins: the 8 P2G
         // bricks of each G2P brick consecutive)
         const int bx = i >> 2, by = j >> 2, bz = k >> 2;
@@ -103,144 +92,245 @@ __global__ __launch_bounds__(kBlock) void k_fs_layers_init(FsEpilogue e) {
                            (uint32_t)e.gbx * ((uint32_t)(by >> 1) + (uint32_t)e.gby * (uint32_t)(bz >> 1));
         const uint32_t bin = e.kb0 + ((g << 3) | (uint32_t)((bx & 1) | ((by & 1) << 1) | ((bz & 1) << 2)));
         const int bit = (i & 3) + 4 * (j & 3) + 16 * (k & 3);
-        v = ((e.fluid[bin] >> bit) & 1ull) ? 0 : -1;
+        fluid = (e.fluid[bin] >> bit) & 1ull;
     } else {
         // the cell's bin in the sort's padded bin grid
         const uint32_t b = (uint32_t)(i + 1) + (uint32_t)e.b[0] *
                            ((uint32_t)(j + 1) + (uint32_t)e.b[1] * (uint32_t)(k + 1));
-        v = e.start[b + 1] > e.start[b] ? 0 : -1;
+        fluid = e.start[b + 1] > e.start[b];
     }
-    e.layer[t] = v;
+    if (e.solid && e.solid[t]) return kSolid;
+    return fluid ? 0 : -1;
 }
 
-__global__ __launch_bounds__(kBlock) void k_fs_dilate(FsEpilogue e, int L) {
-    const int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    const int64_t ncell = (int64_t)e.ni * e.nj * e.nk;
-    if (t >= ncell) return;
-    if (e.layer[t] != -1) return;
-    int i, j, k;
-    cell_of_index(e, (uint32_t)t, i, j, k);
-    const int8_t src = (int8_t)(L - 1);
-    // neighbours set in this launch hold L, never L - 1, whichever value is read
-    bool hit = (i > 0 && layer_at(e, i - 1, j, k) == src) ||
-               (i + 1 < e.ni && layer_at(e, i + 1, j, k) == src) ||
-               (j > 0 && layer_at(e, i, j - 1, k) == src) ||
-               (j + 1 < e.nj && layer_at(e, i, j + 1, k) == src) ||
-               (k > 0 && layer_at(e, i, j, k - 1) == src) ||
-               (k + 1 < e.nk && layer_at(e, i, j, k + 1) == src);
-    if (hit) e.layer[t] = (int8_t)L;
-}
-
-__global__ __launch_bounds__(kBlock) void k_fs_fill(FsEpilogue e, int64_t nface) {
-    const int64_t f = blockIdx.x * (int64_t)kBlock + threadIdx.x;
-    if (f >= nface) return;
-    int c, i, j, k, d[3];
-    face_of(e, (uint32_t)f, c, i, j, k, d);
-    const uint32_t o = (uint32_t)i + (uint32_t)d[0] * ((uint32_t)j + (uint32_t)d[1] * (uint32_t)k);
-    float *grid = c == 0 ? e.grid[0] : (c == 1 ? e.grid[1] : e.grid[2]);
-    float *old = c == 0 ? e.old[0] : (c == 1 ? e.old[1] : e.old[2]);
-    if (!face_borders(e, c, i, j, k, 0)) {
-        grid[o] = 0.0f;
-        old[o] = 0.0f;
-        return;
-    }
-    const float *n = c == 0 ? e.n[0] : (c == 1 ? e.n[1] : e.n[2]);
-    const float *w = c == 0 ? e.w[0] : (c == 1 ? e.w[1] : e.w[2]);
-    float val;
-    if ((double)w[o] > 1e-9) {
-        val = n[o];
-    } else {
-        double avg = 0.0, weight = 0.0;
-        for (int nk = k - 1; nk <= k + 1; nk++)
-            for (int nj = j - 1; nj <= j + 1; nj++)
-                for (int ni = i - 1; ni <= i + 1; ni++) {
-                    if (ni == i && nj == j && nk == k) continue;
-                    if ((unsigned)ni >= (unsigned)d[0] || (unsigned)nj >= (unsigned)d[1] ||
-                        (unsigned)nk >= (unsigned)d[2])
-                        continue;
-                    const uint32_t g = (uint32_t)ni + (uint32_t)d[0] * ((uint32_t)nj + (uint32_t)d[1] * (uint32_t)nk);
-                    const float nv = n[g];
-                    const bool use = c == 0 ? fabsf(nv) > 0.0f : (double)w[g] > 1e-9;
-                    if (use) {
-                        avg += (double)nv;
-                        weight += 1.0;
-                    }
-                }
-        val = weight > 0.0 ? (float)(avg / weight) : 0.0f;
-    }
-    old[o] = val;
-    const bool on = c == 0 ? e.grav_on[0] : (c == 1 ? e.grav_on[1] : e.grav_on[2]);
-    const float gd = c == 0 ? e.grav_delta[0] : (c == 1 ? e.grav_delta[1] : e.grav_delta[2]);
-    grid[o] = on ? val + gd : val;
-}
-
-// the layer L at which face (c,i,j,k) is extrapolated: L borders it, L-1
-// does not, no solid does, 1 <= L <= layers (macvelocityfield.cpp:694-706);
-// 0 when none.  A face borders at most two cells, so at most one L fits.
-__device__ __forceinline__ int face_layer(const FsEpilogue &e, int c, int i, int j, int k) {
-    const int a = c == 0 ? i : (c == 1 ? j : k);
-    const int na = c == 0 ? e.ni : (c == 1 ? e.nj : e.nk);
-    const int li = i - (c == 0), lj = j - (c == 1), lk = k - (c == 2);
-    const int hi = a < na ? layer_at(e, i, j, k) : -3;   // -3: no cell
-    const int lo = a > 0 ? layer_at(e, li, lj, lk) : -3;
-    if (hi == kSolid || lo == kSolid) return 0;
-    int L = 0;
-    if (hi >= 1 && lo != hi - 1) L = hi;
-    if (lo >= 1 && hi != lo - 1 && (L == 0 || lo < L)) L = lo;
-    return L <= e.layers ? L : 0;
-}
-
-// each face's extrapolation layer L (0: none) and, for a face that has one,
-// which of its 6 same-component neighbours (in range) border layer L-1:
-// one 16-bit word per face, L in the low byte, the mask in the high byte
-__global__ __launch_bounds__(kBlock) void k_fs_classify(FsEpilogue e, uint32_t nface) {
-    const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nface) return;
-    int c, i, j, k, d[3];
-    face_of(e, f, c, i, j, k, d);
-    const int L = face_layer(e, c, i, j, k);
-    uint32_t mask = 0;
-    if (L > 0) {
-        const int nb[6][3] = {{i - 1, j, k}, {i + 1, j, k}, {i, j - 1, k},
-                              {i, j + 1, k}, {i, j, k - 1}, {i, j, k + 1}};
-        for (int q = 0; q < 6; q++) {
-            const int a = nb[q][0], b = nb[q][1], cc = nb[q][2];
-            if ((unsigned)a >= (unsigned)d[0] || (unsigned)b >= (unsigned)d[1] ||
-                (unsigned)cc >= (unsigned)d[2])
-                continue;
-            if (face_borders(e, c, a, b, cc, L - 1)) mask |= 1u << q;
+// Layers l0 + 1 .. l0 + n (n <= H) of a tile of TX x TY x TZ cells.  A row of
+// the tile with its halo is a 64-bit word along x, so a dilation is a few word
+// operations per row; the halo is as deep as the dilations, so what is wrong
+// at its rim never reaches the tile.  FIRST (l0 = 0): the cells' states come
+// from the sort and the solid mask, and every cell is written; later launches
+// start from the layers up to l0 (another tile may already have written
+// deeper ones: such a cell counts as unreached here, as it is) and write the
+// cells they reach.
+template <bool FIRST>
+__global__ __launch_bounds__(lay::NT) void k_fs_layers(FsEpilogue e, int l0, int n) {
+    using namespace lay;
+    __shared__ uint64_t s_open[ROWS];        // neither solid nor reached before
+    __shared__ uint64_t s_r[H + 1][ROWS];    // reached after each dilation
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    const uint32_t tx = (uint32_t)(e.ni + TX - 1) / TX, ty = (uint32_t)(e.nj + TY - 1) / TY;
+    const int x0 = (int)(blockIdx.x % tx) * TX, y0 = (int)(blockIdx.x / tx % ty) * TY,
+              z0 = (int)(blockIdx.x / (tx * ty)) * TZ;
+    for (int r0 = wid; r0 < ROWS; r0 += AHEAD * (NT / 64)) {
+        int v[AHEAD];
+#pragma unroll
+        for (int m = 0; m < AHEAD; m++) {
+            const int r = r0 + m * (NT / 64);
+            const int i = x0 - H + lane, j = y0 - H + r % RY, k = z0 - H + r / RY;
+            if (FIRST) {
+                v[m] = r < ROWS ? cell_state(e, i, j, k) : -3;
+            } else {
+                const bool in = r < ROWS && (unsigned)i < (unsigned)e.ni &&
+                                (unsigned)j < (unsigned)e.nj && (unsigned)k < (unsigned)e.nk;
+                v[m] = in ? (int)layer_at(e, i, j, k) : -3;
+                if (v[m] > l0) v[m] = -1;
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < AHEAD; m++) {
+            const int r = r0 + m * (NT / 64);
+            const uint64_t in = __ballot(v[m] >= 0), open = __ballot(v[m] == -1);
+            if (lane == 0 && r < ROWS) {
+                s_r[0][r] = in;
+                s_open[r] = open;
+            }
         }
     }
-    e.fclass[f] = (uint16_t)((uint32_t)L | (mask << 8));
+    __syncthreads();
+    for (int s = 1; s <= n; s++) {
+        if (t < ROWS) {
+            const uint64_t *p = s_r[s - 1];
+            const int y = t % RY, z = t / RY;
+            const uint64_t w = p[t];
+            uint64_t near = (w << 1) | (w >> 1);
+            if (y > 0) near |= p[t - 1];
+            if (y < RY - 1) near |= p[t + 1];
+            if (z > 0) near |= p[t - RY];
+            if (z < RZ - 1) near |= p[t + RY];
+            s_r[s][t] = w | (near & s_open[t]);
+        }
+        __syncthreads();
+    }
+    for (int c = t; c < TX * TY * TZ; c += NT) {
+        const int x = c % TX, y = (c / TX) % TY, z = c / (TX * TY);
+        const int i = x0 + x, j = y0 + y, k = z0 + z;
+        if (i >= e.ni || j >= e.nj || k >= e.nk) continue;
+        const int r = (y + H) + RY * (z + H), b = x + H;
+        int v = -1;
+        if ((s_open[r] >> b) & 1ull) {
+            // the dilation that reached the cell
+            for (int s = n; s >= 1 && ((s_r[s][r] >> b) & 1ull); s--) v = l0 + s;
+            if (!FIRST && v < 0) continue;
+        } else {
+            if (!FIRST) continue;
+            v = ((s_r[0][r] >> b) & 1ull) ? 0 : kSolid;
+        }
+        e.layer[(uint32_t)i + (uint32_t)e.ni * ((uint32_t)j + (uint32_t)e.nj * (uint32_t)k)] = (int8_t)v;
+    }
+}
+
+static_assert(lay::ROWS <= lay::NT, "a thread per row");
+
+// ---- the faces
+
+constexpr int SEG = 1024;   // faces of a segment: 10 bits of an entry, 6 of its neighbours
+
+// The segment sg: its component, its first face and how many it has.
+__device__ __forceinline__ int segment(const FsEpilogue &e, uint32_t sg, uint32_t &f0, uint32_t &nf) {
+    const int c = sg < e.nseg[0] ? 0 : (sg < e.nseg[0] + e.nseg[1] ? 1 : 2);
+    f0 = (sg - (c > 0 ? e.nseg[0] : 0u) - (c > 1 ? e.nseg[1] : 0u)) * (uint32_t)SEG;
+    const uint32_t tot = (uint32_t)(e.ni + (c == 0)) * (uint32_t)(e.nj + (c == 1)) * (uint32_t)(e.nk + (c == 2));
+    nf = min(tot - f0, (uint32_t)SEG);
+    return c;
+}
+
+// The value before the forces of a face bordering fluid: n where W set it,
+// else the mean of its set neighbours.
+__device__ float fill_value(const FsEpilogue &e, int c, int i, int j, int k, const int d[3], uint32_t o) {
+    const float *n = c == 0 ? e.n[0] : (c == 1 ? e.n[1] : e.n[2]);
+    const float *w = c == 0 ? e.w[0] : (c == 1 ? e.w[1] : e.w[2]);
+    if ((double)w[o] > 1e-9) return n[o];
+    double avg = 0.0, weight = 0.0;
+    for (int nk = k - 1; nk <= k + 1; nk++)
+        for (int nj = j - 1; nj <= j + 1; nj++)
+            for (int ni = i - 1; ni <= i + 1; ni++) {
+                if (ni == i && nj == j && nk == k) continue;
+                if ((unsigned)ni >= (unsigned)d[0] || (unsigned)nj >= (unsigned)d[1] ||
+                    (unsigned)nk >= (unsigned)d[2])
+                    continue;
+                const uint32_t g = (uint32_t)ni + (uint32_t)d[0] * ((uint32_t)nj + (uint32_t)d[1] * (uint32_t)nk);
+                const float nv = n[g];
+                const bool use = c == 0 ? fabsf(nv) > 0.0f : (double)w[g] > 1e-9;
+                if (use) {
+                    avg += (double)nv;
+                    weight += 1.0;
+                }
+            }
+    return weight > 0.0 ? (float)(avg / weight) : 0.0f;
+}
+
+// One work-group per segment: the fill of its faces, and the list of those
+// with an extrapolation layer, grouped by layer (in any order inside one):
+// entry = place in the segment | mask of the neighbours that border the layer
+// before << 10; off[L - 1] .. off[L] the entries of layer L.
+//
+// The layer L at which a face is extrapolated: L borders it, L-1 does not, no
+// solid does, 1 <= L <= layers (macvelocityfield.cpp:694-706).  A face borders
+// at most two cells, so at most one L fits.
+__global__ __launch_bounds__(kBlock) void k_fs_faces(FsEpilogue e) {
+    constexpr int ITEMS = SEG / kBlock;
+    constexpr int MAXL = 100;   // layers at most
+    __shared__ uint32_t s_cnt[MAXL + 1];
+    __shared__ uint32_t s_off[MAXL + 2];
+    const int t = threadIdx.x;
+    if (t <= MAXL) s_cnt[t] = 0u;
+    uint32_t f0, nf;
+    const int c = segment(e, blockIdx.x, f0, nf);
+    const int d[3] = {e.ni + (c == 0), e.nj + (c == 1), e.nk + (c == 2)};
+    const int na = c == 0 ? e.ni : (c == 1 ? e.nj : e.nk);
+    float *grid = c == 0 ? e.grid[0] : (c == 1 ? e.grid[1] : e.grid[2]);
+    float *old = c == 0 ? e.old[0] : (c == 1 ? e.old[1] : e.old[2]);
+    const bool on = c == 0 ? e.grav_on[0] : (c == 1 ? e.grav_on[1] : e.grav_on[2]);
+    const float gd = c == 0 ? e.grav_delta[0] : (c == 1 ? e.grav_delta[1] : e.grav_delta[2]);
+    __syncthreads();
+    int L[ITEMS];
+    uint32_t ent[ITEMS], rank[ITEMS];
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        const uint32_t l = (uint32_t)(t + m * kBlock);
+        L[m] = 0;
+        if (l >= nf) continue;
+        const uint32_t o = f0 + l;
+        const uint32_t row = o / (uint32_t)d[0];
+        const int i = (int)(o - row * (uint32_t)d[0]);
+        const int j = (int)(row % (uint32_t)d[1]), k = (int)(row / (uint32_t)d[1]);
+        // the layers of the cells on either side (-3: no cell)
+        const int a = c == 0 ? i : (c == 1 ? j : k);
+        const int hi = a < na ? layer_at(e, i, j, k) : -3;
+        const int lo = a > 0 ? layer_at(e, i - (c == 0), j - (c == 1), k - (c == 2)) : -3;
+        if (hi == 0 || lo == 0) {
+            const float val = fill_value(e, c, i, j, k, d, o);
+            old[o] = val;
+            grid[o] = on ? val + gd : val;
+        } else {
+            grid[o] = 0.0f;
+            old[o] = 0.0f;
+        }
+        if (hi == kSolid || lo == kSolid) continue;
+        int f = 0;
+        if (hi >= 1 && lo != hi - 1) f = hi;
+        if (lo >= 1 && hi != lo - 1 && (f == 0 || lo < f)) f = lo;
+        if (f == 0 || f > e.layers) continue;
+        uint32_t mask = 0;
+        const int nb[6][3] = {{i - 1, j, k}, {i + 1, j, k}, {i, j - 1, k},
+                              {i, j + 1, k}, {i, j, k - 1}, {i, j, k + 1}};
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+            const int x = nb[q][0], y = nb[q][1], z = nb[q][2];
+            if ((unsigned)x >= (unsigned)d[0] || (unsigned)y >= (unsigned)d[1] ||
+                (unsigned)z >= (unsigned)d[2])
+                continue;
+            if (face_borders(e, c, x, y, z, f - 1)) mask |= 1u << q;
+        }
+        L[m] = f;
+        ent[m] = l | (mask << 10);
+        rank[m] = atomicAdd(&s_cnt[f], 1u);
+    }
+    __syncthreads();
+    if (t == 0) {
+        uint32_t at = 0;
+        for (int f = 1; f <= e.layers; f++) {
+            s_off[f] = at;
+            at += s_cnt[f];
+        }
+        s_off[e.layers + 1] = at;
+    }
+    __syncthreads();
+    if (t <= e.layers) e.foff[(size_t)blockIdx.x * (size_t)(e.layers + 1) + t] = (uint16_t)s_off[t + 1];
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++)
+        if (L[m] > 0) e.fent[(size_t)blockIdx.x * SEG + s_off[L[m]] + rank[m]] = (uint16_t)ent[m];
 }
 
 // one layer: every face of layer L takes the FP64 average of its masked
 // neighbours (in the order -x, +x, -y, +y, -z, +z), 0 when that sum is 0,
-// on both grids
-__global__ __launch_bounds__(kBlock) void k_fs_extrapolate(FsEpilogue e, uint32_t nface, int L) {
-    const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
-    if (f >= nface) return;
-    const uint32_t cl = e.fclass[f];
-    if ((cl & 0xFFu) != (uint32_t)L) return;
-    const uint32_t mask = cl >> 8;
-    const uint32_t f0 = (uint32_t)(e.ni + 1) * (uint32_t)e.nj * (uint32_t)e.nk;
-    const uint32_t f1 = (uint32_t)e.ni * (uint32_t)(e.nj + 1) * (uint32_t)e.nk;
-    const int c = f < f0 ? 0 : (f < f0 + f1 ? 1 : 2);
-    const uint32_t o = c == 0 ? f : (c == 1 ? f - f0 : f - f0 - f1);
+// on both grids; one wave per segment
+__global__ __launch_bounds__(kBlock) void k_fs_extrapolate(FsEpilogue e, uint32_t nseg, int L) {
+    const uint32_t sg = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+    if (sg >= nseg) return;
+    const uint16_t *off = e.foff + (size_t)sg * (size_t)(e.layers + 1);
+    const uint32_t e0 = off[L - 1], e1 = off[L];
+    if (e0 == e1) return;
+    uint32_t f0, nf;
+    const int c = segment(e, sg, f0, nf);
     const uint32_t d0 = (uint32_t)(e.ni + (c == 0)), d1 = (uint32_t)(e.nj + (c == 1));
     const uint32_t step[3] = {1u, d0, d0 * d1};
     float *grid = c == 0 ? e.grid[0] : (c == 1 ? e.grid[1] : e.grid[2]);
     float *old = c == 0 ? e.old[0] : (c == 1 ? e.old[1] : e.old[2]);
-    double sg = 0.0, so = 0.0, cnt = 0.0;
-    for (int q = 0; q < 6; q++) {
-        if (!(mask & (1u << q))) continue;
-        const uint32_t g = (q & 1) ? o + step[q >> 1] : o - step[q >> 1];
-        sg += (double)grid[g];
-        so += (double)old[g];
-        cnt += 1.0;
+    for (uint32_t n = e0 + (threadIdx.x & 63); n < e1; n += 64u) {
+        const uint32_t cl = e.fent[(size_t)sg * SEG + n];
+        const uint32_t o = f0 + (cl & (uint32_t)(SEG - 1)), mask = cl >> 10;
+        double sg_ = 0.0, so = 0.0, cnt = 0.0;
+#pragma unroll
+        for (int q = 0; q < 6; q++) {
+            if (!(mask & (1u << q))) continue;
+            const uint32_t g = (q & 1) ? o + step[q >> 1] : o - step[q >> 1];
+            sg_ += (double)grid[g];
+            so += (double)old[g];
+            cnt += 1.0;
+        }
+        grid[o] = sg_ == 0.0 ? 0.0f : (float)(sg_ / cnt);
+        old[o] = so == 0.0 ? 0.0f : (float)(so / cnt);
     }
-    grid[o] = sg == 0.0 ? 0.0f : (float)(sg / cnt);
-    old[o] = so == 0.0 ? 0.0f : (float)(so / cnt);
 }
 
 // ---- collision fix (fluidsimulation.cpp:3145-3207, collision.cpp:303-449)
@@ -390,26 +480,36 @@ void fs_collide(const FsEpilogue &e, hipStream_t s) {
     GFSX_LAUNCH_CHECK();
 }
 
+uint32_t fs_segments(FsEpilogue &e) {
+    uint32_t all = 0;
+    for (int c = 0; c < 3; c++) {
+        const int64_t nf = (int64_t)(e.ni + (c == 0)) * (e.nj + (c == 1)) * (e.nk + (c == 2));
+        e.nseg[c] = (uint32_t)((nf + SEG - 1) / SEG);
+        all += e.nseg[c];
+    }
+    return all;
+}
+
+size_t fs_entries(const FsEpilogue &e) {
+    return (size_t)(e.nseg[0] + e.nseg[1] + e.nseg[2]) * SEG;
+}
+
 void fs_epilogue(const FsEpilogue &e, hipStream_t s) {
-    const int64_t ncell = (int64_t)e.ni * e.nj * e.nk;
-    const int64_t nface = (int64_t)(e.ni + 1) * e.nj * e.nk + (int64_t)e.ni * (e.nj + 1) * e.nk +
-                          (int64_t)e.ni * e.nj * (e.nk + 1);
-    hipLaunchKernelGGL(k_fs_layers_init, dim3(blocks_for(ncell)), dim3(kBlock), 0, s, e);
-    GFSX_LAUNCH_CHECK();
-    for (int L = 1; L <= e.layers; L++) {
-        hipLaunchKernelGGL(k_fs_dilate, dim3(blocks_for(ncell)), dim3(kBlock), 0, s, e, L);
+    auto tiles = [](int n, int t) { return (unsigned)((n + t - 1) / t); };
+    const dim3 grid(tiles(e.ni, lay::TX) * tiles(e.nj, lay::TY) * tiles(e.nk, lay::TZ));
+    for (int l0 = 0; l0 < e.layers; l0 += lay::H) {
+        hipLaunchKernelGGL(l0 == 0 ? k_fs_layers<true> : k_fs_layers<false>, grid, dim3(lay::NT), 0, s,
+                           e, l0, std::min(e.layers - l0, lay::H));
         GFSX_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(k_fs_fill, dim3(blocks_for(nface)), dim3(kBlock), 0, s, e, nface);
+    const uint32_t nseg = e.nseg[0] + e.nseg[1] + e.nseg[2];
+    hipLaunchKernelGGL(k_fs_faces, dim3(nseg), dim3(kBlock), 0, s, e);
     GFSX_LAUNCH_CHECK();
-    // each face's layer once; a layer's launch changes only faces of that
-    // layer and reads only faces bordering the layer before
-    hipLaunchKernelGGL(k_fs_classify, dim3(blocks_for(nface)), dim3(kBlock), 0, s, e,
-                       (uint32_t)nface);
-    GFSX_LAUNCH_CHECK();
+    // a layer's launch changes only faces of that layer and reads only faces
+    // bordering the layer before
     for (int L = 1; L <= e.layers; L++) {
-        hipLaunchKernelGGL(k_fs_extrapolate, dim3(blocks_for(nface)), dim3(kBlock), 0, s, e,
-                           (uint32_t)nface, L);
+        hipLaunchKernelGGL(k_fs_extrapolate, dim3(blocks_for((int64_t)nseg * 64)), dim3(kBlock), 0, s, e,
+                           nseg, L);
         GFSX_LAUNCH_CHECK();
     }
 }

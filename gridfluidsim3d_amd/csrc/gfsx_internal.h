@@ -313,9 +313,11 @@ struct FsEpilogue {
     const float *x0[3];
     const uint32_t *x0_perm;
     float *x1[3];
-    // workspace: each face's extrapolation layer (low byte, 0: none) and
-    // neighbour mask (high byte), nface words
-    uint16_t *fclass;
+    // workspace: per component nseg segments of its faces (fs_segments), each
+    // with a list of the faces to extrapolate, by layer (fs_entries words),
+    // and layers + 1 offsets into it
+    uint32_t nseg[3];
+    uint16_t *fent, *foff;
 };
 
 // Particle removal (gfsx_remove.hip): positions/velocities in, kept ones
@@ -344,6 +346,8 @@ void fill_u32(uint32_t *p, uint32_t value, int64_t count, hipStream_t s);
 void fill_f32(float *p, float value, int64_t count, hipStream_t s);
 void fill_u8(uint8_t *p, uint8_t value, int64_t count, hipStream_t s);
 // gfsx_epilogue.hip
+uint32_t fs_segments(FsEpilogue &e);   // sets nseg, returns their sum
+size_t fs_entries(const FsEpilogue &e);
 void fs_epilogue(const FsEpilogue &e, hipStream_t s);
 void fs_collide(const FsEpilogue &e, hipStream_t s);
 // gfsx_remove.hip
