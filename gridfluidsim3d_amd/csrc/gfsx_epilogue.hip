@@ -32,7 +32,8 @@
 // Bound: latency and the passes over all faces, of which one is left (the
 // fill reads two floats and writes two per face).  157x93x121, 5.3M faces,
 // seven layers: 280 us with a launch over all cells per dilation (77), a fill
-// (30), a classification (36) and a launch over all faces per layer (130).
+// (30), a classification (36) and a launch over all faces per layer (130); now
+// 147: cell words 9, layers 16, faces 62, extrapolation 7 x 8.6.
 //
 // Everything here is integer work or a fixed-order FP64 sum per face:
 // results are bit-identical to the sequential restatement.
@@ -103,11 +104,32 @@ __device__ __forceinline__ int cell_state(const FsEpilogue &e, int i, int j, int
     return fluid ? 0 : -1;
 }
 
+// The cells as bits, 64 along x to a word (nw words a row): fluid, or open
+// (neither fluid nor solid); one wave per word, four words in flight.
+__global__ __launch_bounds__(kBlock) void k_fs_pack(FsEpilogue e, uint32_t nw, uint32_t words) {
+    constexpr int PER = 4;
+    const int lane = threadIdx.x & 63;
+    const uint32_t w0 = (blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6)) * PER;
+    int v[PER];
+#pragma unroll
+    for (int m = 0; m < PER; m++) {
+        const uint32_t w = w0 + (uint32_t)m, row = w / nw;
+        v[m] = w < words ? cell_state(e, (int)(w % nw) * 64 + lane, (int)(row % (uint32_t)e.nj),
+                                      (int)(row / (uint32_t)e.nj))
+                         : -3;
+    }
+#pragma unroll
+    for (int m = 0; m < PER; m++) {
+        const uint64_t fluid = __ballot(v[m] == 0), open = __ballot(v[m] == -1);
+        if (lane == 0 && w0 + (uint32_t)m < words) e.bits[w0 + (uint32_t)m] = make_ulonglong2(fluid, open);
+    }
+}
+
 // Layers l0 + 1 .. l0 + n (n <= H) of a tile of TX x TY x TZ cells.  A row of
 // the tile with its halo is a 64-bit word along x, so a dilation is a few word
 // operations per row; the halo is as deep as the dilations, so what is wrong
 // at its rim never reaches the tile.  FIRST (l0 = 0): the cells' states come
-// from the sort and the solid mask, and every cell is written; later launches
+// from k_fs_pack's words, and every cell is written; later launches
 // start from the layers up to l0 (another tile may already have written
 // deeper ones: such a cell counts as unreached here, as it is) and write the
 // cells they reach.
@@ -120,28 +142,39 @@ __global__ __launch_bounds__(lay::NT) void k_fs_layers(FsEpilogue e, int l0, int
     const uint32_t tx = (uint32_t)(e.ni + TX - 1) / TX, ty = (uint32_t)(e.nj + TY - 1) / TY;
     const int x0 = (int)(blockIdx.x % tx) * TX, y0 = (int)(blockIdx.x / tx % ty) * TY,
               z0 = (int)(blockIdx.x / (tx * ty)) * TZ;
-    for (int r0 = wid; r0 < ROWS; r0 += AHEAD * (NT / 64)) {
-        int v[AHEAD];
+    if (FIRST) {
+        if (t < ROWS) {
+            // the row's 64 cells from x0 - H, out of two words
+            const int j = y0 - H + t % RY, k = z0 - H + t / RY, x = x0 - H;
+            const int nw = (e.ni + 63) / 64, w = x >> 6, sh = x & 63;
+            const bool in = (unsigned)j < (unsigned)e.nj && (unsigned)k < (unsigned)e.nk;
+            const size_t row = in ? (size_t)nw * ((size_t)j + (size_t)e.nj * (size_t)k) : 0;
+            ulonglong2 lo = make_ulonglong2(0ull, 0ull), hi = lo;
+            if (in && w >= 0) lo = e.bits[row + (size_t)w];
+            if (in && w + 1 < nw && sh) hi = e.bits[row + (size_t)(w + 1)];
+            s_r[0][t] = sh ? (lo.x >> sh) | (hi.x << (64 - sh)) : lo.x;
+            s_open[t] = sh ? (lo.y >> sh) | (hi.y << (64 - sh)) : lo.y;
+        }
+    } else {
+        for (int r0 = wid; r0 < ROWS; r0 += AHEAD * (NT / 64)) {
+            int v[AHEAD];
 #pragma unroll
-        for (int m = 0; m < AHEAD; m++) {
-            const int r = r0 + m * (NT / 64);
-            const int i = x0 - H + lane, j = y0 - H + r % RY, k = z0 - H + r / RY;
-            if (FIRST) {
-                v[m] = r < ROWS ? cell_state(e, i, j, k) : -3;
-            } else {
+            for (int m = 0; m < AHEAD; m++) {
+                const int r = r0 + m * (NT / 64);
+                const int i = x0 - H + lane, j = y0 - H + r % RY, k = z0 - H + r / RY;
                 const bool in = r < ROWS && (unsigned)i < (unsigned)e.ni &&
                                 (unsigned)j < (unsigned)e.nj && (unsigned)k < (unsigned)e.nk;
                 v[m] = in ? (int)layer_at(e, i, j, k) : -3;
                 if (v[m] > l0) v[m] = -1;
             }
-        }
 #pragma unroll
-        for (int m = 0; m < AHEAD; m++) {
-            const int r = r0 + m * (NT / 64);
-            const uint64_t in = __ballot(v[m] >= 0), open = __ballot(v[m] == -1);
-            if (lane == 0 && r < ROWS) {
-                s_r[0][r] = in;
-                s_open[r] = open;
+            for (int m = 0; m < AHEAD; m++) {
+                const int r = r0 + m * (NT / 64);
+                const uint64_t in = __ballot(v[m] >= 0), open = __ballot(v[m] == -1);
+                if (lane == 0 && r < ROWS) {
+                    s_r[0][r] = in;
+                    s_open[r] = open;
+                }
             }
         }
     }
@@ -193,12 +226,11 @@ __device__ __forceinline__ int segment(const FsEpilogue &e, uint32_t sg, uint32_
     return c;
 }
 
-// The value before the forces of a face bordering fluid: n where W set it,
-// else the mean of its set neighbours.
-__device__ float fill_value(const FsEpilogue &e, int c, int i, int j, int k, const int d[3], uint32_t o) {
+// The value before the forces of a face bordering fluid that W did not set:
+// the mean of its set neighbours.
+__device__ float mean_of_set(const FsEpilogue &e, int c, int i, int j, int k, const int d[3]) {
     const float *n = c == 0 ? e.n[0] : (c == 1 ? e.n[1] : e.n[2]);
     const float *w = c == 0 ? e.w[0] : (c == 1 ? e.w[1] : e.w[2]);
-    if ((double)w[o] > 1e-9) return n[o];
     double avg = 0.0, weight = 0.0;
     for (int nk = k - 1; nk <= k + 1; nk++)
         for (int nj = j - 1; nj <= j + 1; nj++)
@@ -242,35 +274,47 @@ __global__ __launch_bounds__(kBlock) void k_fs_faces(FsEpilogue e) {
     const bool on = c == 0 ? e.grav_on[0] : (c == 1 ? e.grav_on[1] : e.grav_on[2]);
     const float gd = c == 0 ? e.grav_delta[0] : (c == 1 ? e.grav_delta[1] : e.grav_delta[2]);
     __syncthreads();
-    int L[ITEMS];
+    const float *fn = c == 0 ? e.n[0] : (c == 1 ? e.n[1] : e.n[2]);
+    const float *fw = c == 0 ? e.w[0] : (c == 1 ? e.w[1] : e.w[2]);
+    // every item's cell layers, then values, are loaded before any is used
+    int L[ITEMS], fi[ITEMS], fj[ITEMS], fk[ITEMS], lo[ITEMS], hi[ITEMS];
     uint32_t ent[ITEMS], rank[ITEMS];
+    float val[ITEMS], wgt[ITEMS];
 #pragma unroll
     for (int m = 0; m < ITEMS; m++) {
         const uint32_t l = (uint32_t)(t + m * kBlock);
-        L[m] = 0;
-        if (l >= nf) continue;
-        const uint32_t o = f0 + l;
+        const uint32_t o = f0 + min(l, nf - 1u);
         const uint32_t row = o / (uint32_t)d[0];
-        const int i = (int)(o - row * (uint32_t)d[0]);
-        const int j = (int)(row % (uint32_t)d[1]), k = (int)(row / (uint32_t)d[1]);
+        const int i = fi[m] = (int)(o - row * (uint32_t)d[0]);
+        const int j = fj[m] = (int)(row % (uint32_t)d[1]), k = fk[m] = (int)(row / (uint32_t)d[1]);
         // the layers of the cells on either side (-3: no cell)
         const int a = c == 0 ? i : (c == 1 ? j : k);
-        const int hi = a < na ? layer_at(e, i, j, k) : -3;
-        const int lo = a > 0 ? layer_at(e, i - (c == 0), j - (c == 1), k - (c == 2)) : -3;
-        if (hi == 0 || lo == 0) {
-            const float val = fill_value(e, c, i, j, k, d, o);
-            old[o] = val;
-            grid[o] = on ? val + gd : val;
-        } else {
-            grid[o] = 0.0f;
-            old[o] = 0.0f;
-        }
-        if (hi == kSolid || lo == kSolid) continue;
+        hi[m] = a < na ? layer_at(e, i, j, k) : -3;
+        lo[m] = a > 0 ? layer_at(e, i - (c == 0), j - (c == 1), k - (c == 2)) : -3;
+    }
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        const uint32_t o = f0 + min((uint32_t)(t + m * kBlock), nf - 1u);
+        const bool set = hi[m] == 0 || lo[m] == 0;
+        val[m] = set ? gld(fn, o) : 0.0f;
+        wgt[m] = set ? gld(fw, o) : 0.0f;
+    }
+#pragma unroll
+    for (int m = 0; m < ITEMS; m++) {
+        const uint32_t l = (uint32_t)(t + m * kBlock), o = f0 + l;
+        L[m] = 0;
+        if (l >= nf) continue;
+        const bool set = hi[m] == 0 || lo[m] == 0;
+        if (set && !((double)wgt[m] > 1e-9)) val[m] = mean_of_set(e, c, fi[m], fj[m], fk[m], d);
+        gst(old, (size_t)o, val[m]);
+        gst(grid, (size_t)o, set && on ? val[m] + gd : val[m]);
+        if (hi[m] == kSolid || lo[m] == kSolid) continue;
         int f = 0;
-        if (hi >= 1 && lo != hi - 1) f = hi;
-        if (lo >= 1 && hi != lo - 1 && (f == 0 || lo < f)) f = lo;
+        if (hi[m] >= 1 && lo[m] != hi[m] - 1) f = hi[m];
+        if (lo[m] >= 1 && hi[m] != lo[m] - 1 && (f == 0 || lo[m] < f)) f = lo[m];
         if (f == 0 || f > e.layers) continue;
         uint32_t mask = 0;
+        const int i = fi[m], j = fj[m], k = fk[m];
         const int nb[6][3] = {{i - 1, j, k}, {i + 1, j, k}, {i, j - 1, k},
                               {i, j + 1, k}, {i, j, k - 1}, {i, j, k + 1}};
 #pragma unroll
@@ -303,10 +347,10 @@ __global__ __launch_bounds__(kBlock) void k_fs_faces(FsEpilogue e) {
 
 // one layer: every face of layer L takes the FP64 average of its masked
 // neighbours (in the order -x, +x, -y, +y, -z, +z), 0 when that sum is 0,
-// on both grids; one wave per segment
-__global__ __launch_bounds__(kBlock) void k_fs_extrapolate(FsEpilogue e, uint32_t nseg, int L) {
-    const uint32_t sg = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
-    if (sg >= nseg) return;
+// on both grids; one work-group per segment (a segment along the fluid's
+// surface can lie in one layer whole)
+__global__ __launch_bounds__(kBlock) void k_fs_extrapolate(FsEpilogue e, int L) {
+    const uint32_t sg = blockIdx.x;
     const uint16_t *off = e.foff + (size_t)sg * (size_t)(e.layers + 1);
     const uint32_t e0 = off[L - 1], e1 = off[L];
     if (e0 == e1) return;
@@ -316,7 +360,7 @@ __global__ __launch_bounds__(kBlock) void k_fs_extrapolate(FsEpilogue e, uint32_
     const uint32_t step[3] = {1u, d0, d0 * d1};
     float *grid = c == 0 ? e.grid[0] : (c == 1 ? e.grid[1] : e.grid[2]);
     float *old = c == 0 ? e.old[0] : (c == 1 ? e.old[1] : e.old[2]);
-    for (uint32_t n = e0 + (threadIdx.x & 63); n < e1; n += 64u) {
+    for (uint32_t n = e0 + threadIdx.x; n < e1; n += kBlock) {
         const uint32_t cl = e.fent[(size_t)sg * SEG + n];
         const uint32_t o = f0 + (cl & (uint32_t)(SEG - 1)), mask = cl >> 10;
         double sg_ = 0.0, so = 0.0, cnt = 0.0;
@@ -490,6 +534,8 @@ uint32_t fs_segments(FsEpilogue &e) {
     return all;
 }
 
+size_t fs_words(const FsEpilogue &e) { return (size_t)((e.ni + 63) / 64) * (size_t)e.nj * (size_t)e.nk; }
+
 size_t fs_entries(const FsEpilogue &e) {
     return (size_t)(e.nseg[0] + e.nseg[1] + e.nseg[2]) * SEG;
 }
@@ -497,6 +543,9 @@ size_t fs_entries(const FsEpilogue &e) {
 void fs_epilogue(const FsEpilogue &e, hipStream_t s) {
     auto tiles = [](int n, int t) { return (unsigned)((n + t - 1) / t); };
     const dim3 grid(tiles(e.ni, lay::TX) * tiles(e.nj, lay::TY) * tiles(e.nk, lay::TZ));
+    const uint32_t nw = tiles(e.ni, 64), words = (uint32_t)fs_words(e);
+    hipLaunchKernelGGL(k_fs_pack, dim3(blocks_for((int64_t)words * 16)), dim3(kBlock), 0, s, e, nw, words);
+    GFSX_LAUNCH_CHECK();
     for (int l0 = 0; l0 < e.layers; l0 += lay::H) {
         hipLaunchKernelGGL(l0 == 0 ? k_fs_layers<true> : k_fs_layers<false>, grid, dim3(lay::NT), 0, s,
                            e, l0, std::min(e.layers - l0, lay::H));
@@ -508,8 +557,7 @@ void fs_epilogue(const FsEpilogue &e, hipStream_t s) {
     // a layer's launch changes only faces of that layer and reads only faces
     // bordering the layer before
     for (int L = 1; L <= e.layers; L++) {
-        hipLaunchKernelGGL(k_fs_extrapolate, dim3(blocks_for((int64_t)nseg * 64)), dim3(kBlock), 0, s, e,
-                           nseg, L);
+        hipLaunchKernelGGL(k_fs_extrapolate, dim3(nseg), dim3(kBlock), 0, s, e, L);
         GFSX_LAUNCH_CHECK();
     }
 }

@@ -318,6 +318,7 @@ struct FsEpilogue {
     // and layers + 1 offsets into it
     uint32_t nseg[3];
     uint16_t *fent, *foff;
+    ulonglong2 *bits;           // workspace: fs_words words (fluid, open) of 64 cells along x
 };
 
 // Particle removal (gfsx_remove.hip): positions/velocities in, kept ones
@@ -348,6 +349,7 @@ void fill_u8(uint8_t *p, uint8_t value, int64_t count, hipStream_t s);
 // gfsx_epilogue.hip
 uint32_t fs_segments(FsEpilogue &e);   // sets nseg, returns their sum
 size_t fs_entries(const FsEpilogue &e);
+size_t fs_words(const FsEpilogue &e);
 void fs_epilogue(const FsEpilogue &e, hipStream_t s);
 void fs_collide(const FsEpilogue &e, hipStream_t s);
 // gfsx_remove.hip
