@@ -45,7 +45,7 @@ enum Slot {
     S_B_GRID, S_B_OLD, S_B_WGT, S_B_LG, S_B_XO, S_B_VO, S_B_FX, S_B_MAX, S_B_SLOW,
     S_E_N, S_E_W, S_E_LAYER, S_E_LIST, S_E_OFF, S_E_BITS, S_R_KEEP, S_R_COUNT, S_R_DST, S_R_SCAN, S_R_N, S_R_FULL, S_R_NFULL,
     S_P_TILE, S_P_TFLAG,
-    S_K_COUNT, S_K_START, S_K_PSTART, S_K_RSTART, S_K_RUNREC, S_K_NRUNS, S_K_LIST, S_K_LIST2,
+    S_K_COUNT, S_K_PSTART, S_K_RSTART, S_K_RUNREC, S_K_NRUNS, S_K_LIST, S_K_LIST2,
     S_K_RUNBASE, S_K_MID, S_K_HUGE, S_K_LCOUNT, S_K_SCAN, S_K_FLUID, S_K_SSLOT,
     S_K_SCOUNT, S_SPLAT, S_K_JR, S_K_RLEN, S_K_NCHUNK,
     NSLOT
@@ -314,7 +314,6 @@ gfsx::BrickSort brick_sort(WS &&ws, int64_t n, int64_t nblk, uint32_t nbin, bool
     b.nwave = nwave;
     b.nbb_total = nbin;
     b.count = (unsigned long long *)ws(S_K_COUNT, u64 * nbin);
-    b.start = (unsigned long long *)ws(S_K_START, u64 * ((size_t)nbin + 1));
     b.pstart = (uint32_t *)ws(S_K_PSTART, u32 * ((size_t)nbin + 1));
     b.rstart = (uint32_t *)ws(S_K_RSTART, u32 * ((size_t)nbin + 1));
     b.runrec = (uint2 *)ws(S_K_RUNREC, sizeof(uint2) * nw * 64);

@@ -502,7 +502,6 @@ constexpr int kP2gTileNodes = 3 * 5 * 6 * 6;
 // counting sort by bin.
 struct BrickSort {
     unsigned long long *count;   // nbb_total: (runs << 32) | particles per bin
-    unsigned long long *start;   // nbb_total + 1: exclusive scan of count
     uint32_t *pstart;            // nbb_total + 1: first sort slot of each bin
     uint32_t *rstart;            // nbb_total + 1: first entry of each bin's run list
     uint2 *runrec;               // TILE per binning work-group: chunk (bin, provisional rank)
