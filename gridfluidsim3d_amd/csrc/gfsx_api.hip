@@ -328,7 +328,7 @@ gfsx::BrickSort brick_sort(WS &&ws, int64_t n, int64_t nblk, uint32_t nbin, bool
     b.huge = (uint32_t *)ws(S_K_HUGE, u32 * nbin);
     b.lcount = (uint32_t *)ws(S_K_LCOUNT, u32 * 4);
     b.scan_scratch = (unsigned long long *)ws(
-        S_K_SCAN, u64 * (size_t)std::max<int64_t>(gfsx::scan64_scratch_words(nbin), 1));
+        S_K_SCAN, u64 * (size_t)std::max<int64_t>(gfsx::bin_scan_words(nbin), 1));
     b.perm = want_perm ? (uint32_t *)ws(S_PERM, u32 * nn) : nullptr;
     b.fluid = (unsigned long long *)ws(S_K_FLUID, u64 * nbin);
     b.slow_slots = (uint32_t *)ws(S_K_SSLOT, u32 * nn);

@@ -526,7 +526,7 @@ struct BrickSort {
     uint32_t nbb_total;
 };
 constexpr uint32_t kBrickBinBits = 26;   // global bins below 2^26
-int64_t scan64_scratch_words(int64_t m);
+int64_t bin_scan_words(int64_t m);
 
 // A fused step over one or more scenes.
 struct StepBatch {
