@@ -86,7 +86,7 @@ def flops_per_particle(stencil):
 # The kernels each stage of gfsx_flip_step launches (HIP events bracket the
 # stage on the library's stream).
 STAGE_KERNELS = {
-    "sort": "brick sort: k_bsort_bin, k_tile_scan64, k_bsort_list, k_bsort_order_*, "
+    "sort": "brick sort: k_bsort_bin, k_bin_starts, k_bsort_list, k_bsort_order_*, "
             "k_bsort_scatter",
     "p2g": "k_p2g_bscatter + k_p2g_bcombine",
     "g2p": "k_flip_g2p_bb_tl (trilinear) / k_flip_g2p_bb_tc (tricubic)",
