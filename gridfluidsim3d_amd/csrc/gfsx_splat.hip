@@ -16,7 +16,8 @@
 //      the next entry).
 //   3. k_sp_gather: every node sums the records of its candidate cells, rows
 //      in (k, j) order, then cell order, then index order: a fixed order, so
-//      results are bit-identical run to run.
+//      results are bit-identical run to run.  k_sp_gather_sparse does the
+//      same where no brick holds more than two points per cell on average.
 //
 // Bound: the gather by L2 reads (a lane's records are 16 bytes apart, a
 // wave's spread over a cache line per cell), the passes before it by
@@ -24,7 +25,7 @@
 // read 16 bytes from a random place per candidate (64-odd per node at 8
 // points per cell).  3.85M shuffled points with values on 131x97x113, R = dx,
 // with weights, per component: 1.44 -> 0.33 ms (gather 1.14 -> 0.10, sort
-// 0.30 -> 0.20); 0.73M points on 160x121x144, R = 2.5 dx: 0.94 -> 0.41 ms.
+// 0.30 -> 0.20); 0.73M points on 160x121x144, R = 2.5 dx: 0.94 -> 0.32 ms.
 
 #include "gfsx_internal.h"
 #include "gfsx_device.h"
@@ -40,6 +41,7 @@ constexpr int SITEMS = 16;            // most points per thread there
 constexpr uint32_t kMaxBricks = 40000;   // histogram words that fit a CU's 160 KB of LDS
 constexpr uint32_t CAP = 6144;        // points of a brick ordered in LDS
 constexpr int CELLS = 512;            // cells of a brick
+constexpr uint32_t kSparse = 2 * CELLS;   // most points of a brick for k_sp_gather_sparse
 
 struct SplatGrid {
     BinGrid bg;
@@ -84,17 +86,21 @@ __global__ __launch_bounds__(SNT) void k_sp_count(SplatGrid g, const float *__re
     }
 }
 
-// One work-group: first[b] (b = 0..nbrick+1) and the placing cursors.
+// One work-group: first[b] (b = 0..nbrick+1), the placing cursors, and in
+// first[nbrick+2] the points of the fullest brick.
 __global__ __launch_bounds__(SNT) void k_sp_starts(uint32_t nbrick, const uint32_t *__restrict__ count,
                                                    uint32_t *__restrict__ first,
                                                    uint32_t *__restrict__ cursor) {
     __shared__ uint32_t s_w[SNT / 64];
+    __shared__ uint32_t s_most;
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-    uint32_t at = 0;
+    uint32_t at = 0, most = 0;
+    if (t == 0) s_most = 0u;
     for (uint32_t b0 = 0; b0 <= nbrick; b0 += SNT) {
         const uint32_t b = b0 + (uint32_t)t;
         const uint32_t c = b <= nbrick ? count[b] : 0u;
         const uint32_t inc = wave_inclusive_sum(c);
+        if (b < nbrick) most = max(most, c);
         if (lane == 63) s_w[wid] = inc;
         __syncthreads();
         uint32_t s = at + inc - c;
@@ -109,7 +115,14 @@ __global__ __launch_bounds__(SNT) void k_sp_starts(uint32_t nbrick, const uint32
         }
         __syncthreads();
     }
-    if (t == 0) first[nbrick + 1] = at;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d, 64));
+    if (lane == 0) atomicMax(&s_most, most);
+    __syncthreads();
+    if (t == 0) {
+        first[nbrick + 1] = at;
+        first[nbrick + 2] = s_most;
+    }
 }
 
 __global__ __launch_bounds__(SNT) void k_sp_place(SplatGrid g, const float *__restrict__ pos,
@@ -245,10 +258,12 @@ __global__ __launch_bounds__(CELLS) void k_sp_cells(SplatGrid g, const uint32_t 
 template <bool HAS_VAL, int D>
 __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, double dx,
                                                       float inv_r2, int kseg,
+                                                      const uint32_t *__restrict__ most,
                                                       const uint32_t *__restrict__ start,
                                                       const float4 *__restrict__ rec,
                                                       float *__restrict__ S, float *__restrict__ W) {
     constexpr int AHEAD = 2;
+    if (most && *most <= kSparse) return;   // k_sp_gather_sparse does it
     const int64_t col = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     const int64_t ncol = (int64_t)ng.n[0] * ng.n[1];
     if (col >= ncol) return;
@@ -326,6 +341,117 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, 
     }
 }
 
+// The same sums in the same order where cells hold few points.  A row is then
+// mostly a wait for its two starts and for the wave's longest lane (0.26 points
+// per cell: 1.6 records in a row of 6 cells, 5 to 6 in the longest of 64 lanes):
+// all of a plane's starts are loaded together, its ranges that are not empty
+// kept in LDS, and a thread goes through them as one sequence, so a wave waits
+// for its longest lane once a plane.  A row's cells (at most 8) lie in at most
+// two bricks.  0.73M points on 160x121x144, R = 2.5 dx: the call 410 -> 317 us.
+// Where cells are full, lanes on different rows no longer share cache
+// lines: splats of evenly spread points by rows / as one sequence at 1, 2, 4
+// and 8 points per cell, R = dx: 189/177, 282/277, 266/284, 670/888 us; R = 2.5
+// dx: 750/524, 1189/1005, 1611/2129, 3981/8717 us.  Hence kSparse, two points
+// per cell in the fullest brick.
+template <bool HAS_VAL, int D>
+__global__ __launch_bounds__(kBlock) void k_sp_gather_sparse(SplatGrid g, NodeGrid ng, double dx,
+                                                      float inv_r2, int kseg,
+                                                      const uint32_t *__restrict__ most,
+                                                      const uint32_t *__restrict__ start,
+                                                      const float4 *__restrict__ rec,
+                                                      float *__restrict__ S, float *__restrict__ W) {
+    // the calling thread's own column only: no barrier
+    __shared__ uint2 s_range[2 * D][kBlock];
+    if (*most > kSparse) return;   // k_sp_gather does it
+    const int64_t col = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    const int64_t ncol = (int64_t)ng.n[0] * ng.n[1];
+    if (col >= ncol) return;
+    const int i = (int)(col % ng.n[0]), j = (int)(col / ng.n[0]);
+    const int k0 = (int)blockIdx.y * kseg, k1 = min(k0 + kseg, ng.n[2]);
+    // node position in the shifted frame, rounded as
+    // Grid3d::GridIndexToPosition does (grid3d.h:79-81)
+    const float gx = (float)((float)i * dx);
+    const float gy = (float)((float)j * dx);
+    const int ilo = max(i + ng.dlo[0], 0), ihi = min(i + ng.dhi[0], g.bg.b[0] - 1);
+    const int jlo = max(j + ng.dlo[1], 0), jhi = min(j + ng.dhi[1], g.bg.b[1] - 1);
+    const size_t stride = (size_t)ng.n[0] * ng.n[1];
+    float s[D], w[D], gz[D];
+#pragma unroll
+    for (int m = 0; m < D; m++) s[m] = w[m] = 0.0f;
+    for (int bk = k0 + ng.dlo[2]; bk <= k1 - 1 + ng.dhi[2]; bk++) {
+        const int kk = bk - ng.dhi[2];   // the node of slot 0
+        if (bk >= 0 && bk < g.bg.b[2]) {
+#pragma unroll
+            for (int m = 0; m < D; m++) gz[m] = (float)((float)(kk + m) * dx);
+            // the plane's ranges of records, every start loaded before any is used
+            uint32_t q0[2 * D], q1[2 * D];
+#pragma unroll
+            for (int y = 0; y < D; y++) {
+                const int bj = jlo + y;
+                const uint32_t row = (uint32_t)g.gb[0] *
+                                     ((uint32_t)(bj >> 3) + (uint32_t)g.gb[1] * (uint32_t)(bk >> 3));
+                const uint32_t cjk = (uint32_t)((bj & 7) << 3) | (uint32_t)((bk & 7) << 6);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int a = h ? (ilo | 7) + 1 : ilo, e = h ? ihi : min(ihi, ilo | 7);
+                    const bool some = bj <= jhi && a <= e;
+                    const uint32_t id = ((row + (uint32_t)(a >> 3)) << 9) | cjk | (uint32_t)(a & 7);
+                    q0[2 * y + h] = start[some ? id : 0u];
+                    q1[2 * y + h] = start[some ? id + (uint32_t)(e - a) + 1u : 0u];
+                }
+            }
+            int nr = 0;
+#pragma unroll
+            for (int c = 0; c < 2 * D; c++) {
+                if (q0[c] < q1[c]) s_range[nr++][threadIdx.x] = make_uint2(q0[c], q1[c]);
+            }
+            bool live = nr > 0;
+            uint2 at = make_uint2(0u, 0u);
+            if (live) at = s_range[0][threadIdx.x];
+            float4 r = rec[at.x];
+            for (int c = 0; live;) {
+                // the next record, loaded ahead of this one's sums
+                bool more = true;
+                if (++at.x >= at.y) {
+                    more = ++c < nr;
+                    if (more) at = s_range[c][threadIdx.x];
+                }
+                const float4 rn = rec[more ? at.x : 0u];
+                const float vx = gx - (r.x - ng.off[0]);
+                const float vy = gy - (r.y - ng.off[1]);
+                const float pz = r.z - ng.off[2];
+                const float dxy = vx * vx + vy * vy;
+#pragma unroll
+                for (int m = 0; m < D; m++) {
+                    if (kk + m < k0 || kk + m >= k1) continue;
+                    const float vz = gz[m] - pz;
+                    const float d2 = dxy + vz * vz;
+                    const float t = d2 * inv_r2;
+                    const float K = wyvill(t);
+                    if (HAS_VAL) s[m] = fmaf(K, t < 1.0f ? r.w : 0.0f, s[m]);
+                    else s[m] += K;
+                    w[m] += K;
+                }
+                r = rn;
+                live = more;
+            }
+        }
+        // the node of slot 0 has all its planes: accumulate into the caller's
+        // arrays (clscalarfield.cpp:1448-1449)
+        if (kk >= k0) {
+            const size_t f = (size_t)col + stride * (size_t)kk;
+            S[f] += s[0];
+            if (W) W[f] += w[0];
+        }
+#pragma unroll
+        for (int m = 0; m + 1 < D; m++) {
+            s[m] = s[m + 1];
+            w[m] = w[m + 1];
+        }
+        s[D - 1] = w[D - 1] = 0.0f;
+    }
+}
+
 int64_t bricks(const BinGrid &bg) {
     int64_t b = 1;
     for (int a = 0; a < 3; a++) b *= (bg.b[a] + 7) / 8;
@@ -341,7 +467,7 @@ bool splat_by_brick(int64_t n, const BinGrid &bg, double reach) {
 size_t splat_workspace(int64_t n, const BinGrid &bg) {
     const size_t nb = (size_t)bricks(bg);
     // records twice, indices, crowded bricks' groups; counts, starts, cursors, cell starts
-    return (16 + 16 + 8 + 4) * (size_t)n + 3 * 4 * (nb + 2) + 4 * (nb * CELLS + 1) + 8 * 256;
+    return (16 + 16 + 8 + 4) * (size_t)n + 3 * 4 * (nb + 3) + 4 * (nb * CELLS + 1) + 8 * 256;
 }
 
 void splat_run(void *work, const float *pos, const float *val, int64_t n, const BinGrid &bins,
@@ -363,7 +489,7 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
     uint2 *spill = (uint2 *)take(8 * nn);
     uint32_t *idx = (uint32_t *)take(4 * nn);
     uint32_t *count = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
-    uint32_t *first = (uint32_t *)take(4 * (size_t)(g.nbrick + 2));
+    uint32_t *first = (uint32_t *)take(4 * (size_t)(g.nbrick + 3));
     uint32_t *cursor = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
     uint32_t *start = (uint32_t *)take(4 * ((size_t)g.nbrick * CELLS + 1));
     fill_u32(count, 0u, (int64_t)g.nbrick + 1, st);
@@ -390,17 +516,29 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
                  : D == 4 ? (val ? k_sp_gather<true, 4> : k_sp_gather<false, 4>)
                  : D == 6 ? (val ? k_sp_gather<true, 6> : k_sp_gather<false, 6>)
                           : (val ? k_sp_gather<true, 8> : k_sp_gather<false, 8>);
+    auto *sparse = D == 2   ? (val ? k_sp_gather_sparse<true, 2> : k_sp_gather_sparse<false, 2>)
+                   : D == 4 ? (val ? k_sp_gather_sparse<true, 4> : k_sp_gather_sparse<false, 4>)
+                   : D == 6 ? (val ? k_sp_gather_sparse<true, 6> : k_sp_gather_sparse<false, 6>)
+                            : (val ? k_sp_gather_sparse<true, 8> : k_sp_gather_sparse<false, 8>);
     // Columns of 1 to 16 nodes, about 8192 waves of them (and no more
     // segments than a grid's y extent holds): longer columns read less,
     // shorter ones fill the chip.  0.27M nodes, columns of 1 / 4: 22 / 52 us
     // of gather; 2.8M nodes at R = 2.5 dx, the whole call with columns of
-    // 1 / 3 / 5 / 8: 644 / 442 / 410 / 427 us.
+    // 1 / 3 / 5 / 8: 644 / 442 / 410 / 427 us by rows.
     const int kseg = (int)std::max<int64_t>(
         std::min<int64_t>(std::max<int64_t>(nnode / (64 * 8192), 1), 16), nodes.n[2] / 65535 + 1);
-    hipLaunchKernelGGL(kern, dim3(grid_for((int64_t)nodes.n[0] * nodes.n[1], kBlock),
-                                  grid_for(nodes.n[2], kseg)),
-                       dim3(kBlock), 0, st, g, nodes, dx, inv_r2, kseg, (const uint32_t *)start,
-                       (const float4 *)out, S, W);
+    const dim3 grid(grid_for((int64_t)nodes.n[0] * nodes.n[1], kBlock), grid_for(nodes.n[2], kseg));
+    // the fullest brick, known on the device, decides which of the two works;
+    // where the points' mean exceeds the line the rows do it anyway (3.85M
+    // points in 3315 bricks: an empty launch saved)
+    const uint32_t *most = n <= (int64_t)kSparse * g.nbrick ? first + g.nbrick + 2 : nullptr;
+    if (most) {
+        hipLaunchKernelGGL(sparse, grid, dim3(kBlock), 0, st, g, nodes, dx, inv_r2, kseg, most,
+                           (const uint32_t *)start, (const float4 *)out, S, W);
+        GFSX_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(kBlock), 0, st, g, nodes, dx, inv_r2, kseg, most,
+                       (const uint32_t *)start, (const float4 *)out, S, W);
     GFSX_LAUNCH_CHECK();
 }
 
