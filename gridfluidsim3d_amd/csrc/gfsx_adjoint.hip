@@ -233,15 +233,14 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect(StepAdjoint a) {
 // same on every run; no face can overflow: it receives at most 5n terms of
 // magnitude at most 2^61 / (5n).
 //
-// The P2G adjoint takes only the sum dL/dg + dL/dn of a face, so both go to
-// one accumulator: the samples of g and n at x0 share their corners and
-// weights, and their adjoints are added first (h/6 A + h/2 lq + r_pic V: the
-// two FLIP terms cancel before any rounding), 96 LDS atomics a particle
-// instead of 120 and half the sums to keep, flush and read.  The cell
-// coordinates of a stage serve its sample and its adjoint.  2M particles of
-// a 96^3 slab: 220 -> 191 us (VALU and LDS waits; 24.6 KB of LDS and 109
-// VGPRs, four work-groups a CU; 5 or 6 waves per SIMD by launch bounds: no
-// faster, and 3% slower).
+// dL/dg and dL/dn keep sums of their own, each rounded to float before
+// face_coeffs adds them, although the P2G adjoint takes only their sum: one
+// sum for both would round 1/W times smaller differences another way, and a
+// face that particles touch only at the rim of the kernel (W of 1e-10) turns
+// that into other gradients (2M particles of a 96^3 slab: 192 us with one
+// sum, 216 with two, and the rollout's gradient up to 1.7e-4 away).  The cell
+// coordinates of a stage serve its sample and its adjoint (225 us before).
+// Bound by VALU and LDS waits.
 namespace abrick {
 constexpr int BX = 4, BY = 4, BZ = 4;   // the P2G bricks of the forward's brick sort
 constexpr int M = 1;
@@ -307,7 +306,7 @@ struct TileLoc {
 __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, AdjointSort so) {
     using namespace abrick;
     __shared__ float gt[6 * TN];                 // g (0-2) and n (3-5) on the tile
-    __shared__ unsigned long long at[3 * TN];    // fixed-point dL/dg + dL/dn
+    __shared__ unsigned long long at[6 * TN];    // fixed-point dL/dg, dL/dn
     const int tid = threadIdx.x;
     const uint32_t bid = blockIdx.x;
     // brick bid: bin bid of the sort, one contiguous range of slots
@@ -346,8 +345,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
 #pragma unroll
         for (int m = 0; m < PER; m++) {
             const int e = tid + m * kBlock;
-            if (e < 6 * TN) gt[e] = v[m];
-            if (e < 3 * TN) at[e] = 0ull;
+            if (e < 6 * TN) {
+                gt[e] = v[m];
+                at[e] = 0ull;
+            }
         }
     }
     __syncthreads();
@@ -414,10 +415,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         dt[2] += lam * (sx * sy * (v001 - v000) + tx * sy * (v101 - v100) +
                         sx * ty * (v011 - v010) + tx * ty * (v111 - v110));
     };
-    // lam times the corner weights into component c's sums
-    auto spread = [&](int c, int l, float tx, float ty, float tz, float lam) {
+    // lam times the corner weights into array arr's sums
+    auto spread = [&](int arr, int l, float tx, float ty, float tz, float lam) {
         const float sx = 1.0f - tx, sy = 1.0f - ty, sz = 1.0f - tz;
-        unsigned long long *t = at + c * TN + l;
+        unsigned long long *t = at + arr * TN + l;
         atomicAdd(t, to_fixed(lam * (sx * sy * sz), scale));
         atomicAdd(t + 1, to_fixed(lam * (tx * sy * sz), scale));
         atomicAdd(t + TX, to_fixed(lam * (sx * ty * sz), scale));
@@ -427,16 +428,16 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         atomicAdd(t + TX * TY + TX, to_fixed(lam * (sx * ty * tz), scale));
         atomicAdd(t + TX * TY + TX + 1, to_fixed(lam * (tx * ty * tz), scale));
     };
-    // adjoint of the grid's sample at p
-    auto adjoint = [&](const TileLoc &p, const float lam[3], float lq[3]) {
+    // adjoint of the sample at p, of g (base 0) or n (base 3)
+    auto adjoint = [&](int base, const TileLoc &p, const float lam[3], float lq[3]) {
         if (!p.in) return;
         float dt[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             if (lam[c] == 0.0f) continue;
             const float tx = frac(p, c, 0), ty = frac(p, c, 1), tz = frac(p, c, 2);
-            slope(c, p.l[c], tx, ty, tz, lam[c], dt);
-            spread(c, p.l[c], tx, ty, tz, lam[c]);
+            slope(base + c, p.l[c], tx, ty, tz, lam[c], dt);
+            spread(base + c, p.l[c], tx, ty, tz, lam[c]);
         }
         // the cell fractions move by 1/dx per unit of x
         const float inv_dx = (float)a.mac.inv_dx;
@@ -463,34 +464,27 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
             lk[c] = a.h_sixth * ax[c];               // k4
             lq[c] = 0.0f;
         }
-        adjoint(p4, lk, lq);
+        adjoint(0, p4, lk, lq);
         for (int c = 0; c < 3; c++) {
             lx[c] += lq[c];
             lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_full * lq[c];    // k3
             lq[c] = 0.0f;
         }
-        adjoint(p3, lk, lq);
+        adjoint(0, p3, lk, lq);
         for (int c = 0; c < 3; c++) {
             lx[c] += lq[c];
             lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_half * lq[c];    // k2
             lq[c] = 0.0f;
         }
-        adjoint(p2, lk, lq);
-        for (int c = 0; c < 3; c++) lx[c] += lq[c];
-        if (!p1.in) return true;
-        // I(g, x0) has the adjoint k1 + (r_pic + r_flip) av, I(n, x0) -r_flip av
-        float dt[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll
+        adjoint(0, p2, lk, lq);
+        float lgx[3], lnx[3];
         for (int c = 0; c < 3; c++) {
-            const float k1 = a.h_sixth * ax[c] + a.h_half * lq[c];
-            const float tx = frac(p1, c, 0), ty = frac(p1, c, 1), tz = frac(p1, c, 2);
-            slope(c, p1.l[c], tx, ty, tz, k1 + (a.r_pic + a.r_flip) * av[c], dt);
-            slope(3 + c, p1.l[c], tx, ty, tz, -a.r_flip * av[c], dt);
-            const float both = k1 + a.r_pic * av[c];
-            if (both != 0.0f) spread(c, p1.l[c], tx, ty, tz, both);
+            lx[c] += lq[c];
+            lgx[c] = a.h_sixth * ax[c] + a.h_half * lq[c] + (a.r_pic + a.r_flip) * av[c];
+            lnx[c] = -a.r_flip * av[c];
         }
-        const float inv_dx = (float)a.mac.inv_dx;
-        for (int c = 0; c < 3; c++) lx[c] += dt[c] * inv_dx;
+        adjoint(0, p1, lgx, lx);
+        adjoint(3, p1, lnx, lx);
         return true;
     };
     // blocked mapping: thread t takes items [t*per, (t+1)*per), so the lanes
@@ -515,17 +509,19 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         }
     }
     __syncthreads();
-    for (int e = tid; e < 3 * TN; e += kBlock) {
+    for (int e = tid; e < 6 * TN; e += kBlock) {
         const unsigned long long v = at[e];
         if (v == 0ull) continue;
-        const int c = e / TN, l = e - c * TN;
+        const int arr = e / TN, l = e - arr * TN;
+        const int c = arr % 3;
         const int i = ox + l % TX, j = oy + (l / TX) % TY, k = oz + l / (TX * TY);
         const int w = ni + (c == 0), h = nj + (c == 1), d = nk + (c == 2);
         // tile entries outside the arrays collect nothing that exists
         if (!((unsigned)i < (unsigned)w && (unsigned)j < (unsigned)h && (unsigned)k < (unsigned)d))
             continue;
         const uint32_t o = (uint32_t)i + (uint32_t)w * ((uint32_t)j + (uint32_t)h * (uint32_t)k);
-        const float *base = c == 0 ? a.lg[0] : c == 1 ? a.lg[1] : a.lg[2];
+        const float *base = c == 0 ? (arr < 3 ? a.lg[0] : a.ln[0])
+                          : c == 1 ? (arr < 3 ? a.lg[1] : a.ln[1]) : (arr < 3 ? a.lg[2] : a.ln[2]);
         atomicAdd(so.fx + (base - a.lg[0]) + o, v);
     }
 }
@@ -541,7 +537,8 @@ struct GlobalFixed {
         const StepAdjoint &a = gp.a;
         mac_adjoint(a, base == 0 ? a.g : a.old, base, q, lam, lq,
                     [&](int arr, int, int, int, uint32_t o, float v) {
-                        atomicAdd(fx + (a.lg[arr % 3] - a.lg[0]) + o, to_fixed(v, scale));
+                        atomicAdd(fx + ((arr < 3 ? a.lg[arr] : a.ln[arr - 3]) - a.lg[0]) + o,
+                                  to_fixed(v, scale));
                     });
     }
 };
@@ -590,7 +587,7 @@ __device__ __forceinline__ int face_comp(int64_t f, const int64_t nf[3], int64_t
     return c;
 }
 
-// dL/dg + dL/dn from the fixed-point sums, turned into A and B (written to
+// dL/dg, dL/dn from the fixed-point sums, turned into A and B (written over
 // lg and ln) for one thread per face.
 __global__ __launch_bounds__(kBlock) void k_fixed_to_coeffs(const unsigned long long *fx,
                                                             StepAdjoint a, FaceCount fc,
@@ -598,10 +595,11 @@ __global__ __launch_bounds__(kBlock) void k_fixed_to_coeffs(const unsigned long 
     const int64_t f = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     if (f >= fc.tot) return;
     const double scale = fixed_scale(bound, a);
-    const float both = (float)((double)(long long)fx[f] / scale);
+    const float lg = (float)((double)(long long)fx[f] / scale);
+    const float ln = (float)((double)(long long)fx[fc.tot + f] / scale);
     int64_t l;
     const int c = face_comp(f, fc.nf, l);
-    face_coeffs(both, 0.0f, a.w[c][l], a.old[c][l], a.lg[c][l], a.ln[c][l]);
+    face_coeffs(lg, ln, a.w[c][l], a.old[c][l], a.lg[c][l], a.ln[c][l]);
 }
 
 // bound[0..2] = max |dL/dx'|, max |dL/dv'| over the particles and max |g|
@@ -659,18 +657,33 @@ __global__ __launch_bounds__(kBlock) void k_face_coeffs(StepAdjoint a, FaceCount
 // floor(s) + 1, 2x2x2 candidates per component; the kernel's support
 // decides which of them take weight.  The offsets and their squares are
 // formed once per axis and the two faces of a row read together (2M
-// particles: 73 us with a loop over the faces, 52 now; VALU bound).
+// particles: 74 us with a loop over the faces, 57 now; VALU bound).
+//
+// The roundings are written out: near t = 1 the slope of K over its value
+// grows without bound, a face that took little weight has a large A, and
+// v A - B cancels, so another rounding of the squared distance or of the sums
+// is another gradient there.
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+// x^2 + y2 + z2, x^2 unrounded
+__device__ __forceinline__ float dist2(float x, float y2, float z2) {
+#pragma clang fp contract(off)
+    return fmaf(x, x, y2) + z2;
+}
+
 __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
     typedef float Row __attribute__((ext_vector_type(2), aligned(4)));
     typedef const __attribute__((address_space(1))) Row GRow;
     const int64_t p = blockIdx.x * (int64_t)kBlock + threadIdx.x;
     if (p >= a.n) return;
-    float lx[3], lv[3], xp[3], vp[3];
+    float lx[3] = {0.0f, 0.0f, 0.0f};
+    float lv[3] = {0.0f, 0.0f, 0.0f};
+    float xp[3], vp[3];
     for (int c = 0; c < 3; c++) {
         xp[c] = a.x[c][p];
         vp[c] = a.v[c][p];
-        lx[c] = a.gx[c][p];
-        lv[c] = a.gv[c][p];
     }
     const double dx = a.mac.dx;
 #pragma unroll
@@ -678,7 +691,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
         const int dims[3] = {a.mac.ni + (c == 0), a.mac.nj + (c == 1), a.mac.nk + (c == 2)};
         int lo[3];
         bool any = true, all = true;
-        float d[3][2], q[3][2];    // node - p, and its square over R^2
+        float d[3][2], q[3][2];    // node - p, and its square
 #pragma unroll
         for (int ax = 0; ax < 3; ax++) {
             // p -= offset (scalarfield.cpp:168)
@@ -695,7 +708,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
 #pragma unroll
             for (int m = 0; m < 2; m++) {
                 d[ax][m] = (float)((float)(lo[ax] + m) * dx) - ps;
-                q[ax][m] = d[ax][m] * d[ax][m];
+                q[ax][m] = rounded_product(d[ax][m], d[ax][m]);
             }
         }
         if (!any) continue;
@@ -729,23 +742,23 @@ __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
                 }
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    const float t = (q[0][i] + q[1][j] + q[2][k]) * a.inv_r2;
-                    // only inside the radius: a factor that is not finite must
-                    // not reach the particles beyond it
+                    const float t = rounded_product(dist2(d[0][i], q[1][j], q[2][k]), a.inv_r2);
+                    // only inside the radius: a factor or a velocity that is
+                    // not finite must not reach past it
                     const bool on = t < 1.0f;
-                    const float fa = on ? af[i] : 0.0f, fb = on ? bf[i] : 0.0f;
-                    lv[c] += wyvill(t) * fa;
+                    lv[c] = fmaf(wyvill(t), on ? af[i] : 0.0f, lv[c]);
                     // d(d2)/dx_p = -2 (g - p); lam (v_p - n_f) / W_f = v_p A - B
-                    const float coef = fmaf(vp[c], fa, -fb) * wyvill_dt(t) * a.inv_r2 * -2.0f;
-                    lx[0] += coef * d[0][i];
-                    lx[1] += coef * d[1][j];
-                    lx[2] += coef * d[2][k];
+                    const float slope = fmaf(vp[c], af[i], -bf[i]) * wyvill_dt(t) * a.inv_r2 * -2.0f;
+                    const float coef = on ? slope : 0.0f;
+                    lx[0] = fmaf(coef, d[0][i], lx[0]);
+                    lx[1] = fmaf(coef, d[1][j], lx[1]);
+                    lx[2] = fmaf(coef, d[2][k], lx[2]);
                 }
             }
     }
     for (int c = 0; c < 3; c++) {
-        a.gx[c][p] = lx[c];
-        a.gv[c][p] = lv[c];
+        a.gx[c][p] += lx[c];
+        a.gv[c][p] += lv[c];
     }
 }
 
@@ -823,7 +836,7 @@ void flip_step_adjoint(const StepAdjoint &a, const AdjointSort *so, hipStream_t 
             a.ln[0] != a.lg[2] + nf[2] || a.ln[1] != a.ln[0] + nf[0] ||
             a.ln[2] != a.ln[1] + nf[1])
             throw Error("flip_step_adjoint: grid adjoint arrays must be contiguous");
-        fill_u32((uint32_t *)so->fx, 0u, 2 * tot, s);
+        fill_u32((uint32_t *)so->fx, 0u, 4 * tot, s);
         fill_u32(so->bound, 0u, 4, s);   // slow_count too
         // the fixed-point scale's bound, then one work-group per bin of the
         // brick sort

@@ -790,9 +790,9 @@ void run_adjoint(gfsx_ctx *ctx, const gfsx_scene *sc, const gfsx_step_params *pr
     for (int c = 0; c < 3; c++) tot += (nf[c] = mac_count(c, ni, nj, nk));
     const int64_t at[3] = {0, nf[0], nf[0] + nf[1]};
     // dL/dg then dL/dn, one block (the LDS-brick adjoint turns its
-    // fixed-point sums into the P2G adjoint's two factors there in one pass)
+    // fixed-point sums into the P2G adjoint's two factors in it in one pass)
     float *lg = ctx->f32(S_B_LG, 2 * tot), *ln = lg + tot;
-    so.fx = (unsigned long long *)ctx->get(S_B_FX, sizeof(unsigned long long) * (size_t)tot);
+    so.fx = (unsigned long long *)ctx->get(S_B_FX, sizeof(unsigned long long) * 2 * (size_t)tot);
     so.bound = ctx->u32(S_B_MAX, 4);
     so.slow = ctx->u32(S_B_SLOW, sc->n);
     so.slow_count = so.bound + 3;

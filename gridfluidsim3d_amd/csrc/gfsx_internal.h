@@ -272,11 +272,11 @@ struct StepAdjoint {
 // per z layer), bin nbb the particles beyond the padded grid; its particles
 // are slots [pstart[lb], pstart[lb + 1]) of the sorted positions xs, and
 // perm maps a slot to its input index.  fx: fixed-point accumulators for
-// the grid adjoints (int64, dL/dg + dL/dn on the face arrays u, v, w back to
-// back); bound: three words for the fixed-point scale's bound (max |dL/dx'|,
-// max |dL/dv'|, max |g|, float bits); slow: slots of particles left to the
-// global-memory kernel (at most n), slow_count their number, the word after
-// bound's three.
+// the grid adjoints (int64, the face arrays of dL/dg u,v,w then dL/dn u,v,w
+// back to back); bound: three words for the fixed-point scale's bound
+// (max |dL/dx'|, max |dL/dv'|, max |g|, float bits); slow: slots of particles
+// left to the global-memory kernel (at most n), slow_count their number, the
+// word after bound's three.
 struct AdjointSort {
     const uint32_t *pstart, *perm;
     const float *xs[3];
