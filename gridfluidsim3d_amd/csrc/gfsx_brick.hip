@@ -29,6 +29,7 @@
 #include "gfsx_internal.h"
 #include "gfsx_sample.h"
 #include "gfsx_device.h"
+#include "gfsx_tiles.h"
 
 #include <type_traits>
 
@@ -822,17 +823,9 @@ __host__ __device__ constexpr int tsz(int c) { return c == 2 ? 5 : 6; }
 }  // namespace bscat
 static_assert(3 * bscat::TN == kP2gTileNodes, "tile buffer size");
 
-// Tile entries of a scene in HBM: per component one array of
-// (nbx*SX) x (nby*SY) x (nbz*SZ) entries (x fastest), brick (bx,by,bz)'s
-// tile at (bx*SX, by*SY, bz*SZ), so that the tiles of neighbouring bricks
-// along x sit side by side and a face row reads them in sequence.  A scene
-// owns the entries from kb0 * kP2gTileNodes on (it has at least
-// nbx*nby*nbz <= nbb bins), component c at c * nbx*nby*nbz * TN after that.
-struct TileGrid {
-    size_t base;          // first entry of component c
-    int tx, ty;           // entries along x and y
-};
-
+// A scene owns the tile entries (gfsx_tiles.h) from kb0 * kP2gTileNodes on (it
+// has at least nbx*nby*nbz <= nbb bins), component c at c * nbx*nby*nbz * TN
+// after that.
 __device__ __forceinline__ TileGrid tile_grid(const SceneDesc &sd, int c) {
     using namespace bscat;
     TileGrid t;
@@ -841,10 +834,6 @@ __device__ __forceinline__ TileGrid tile_grid(const SceneDesc &sd, int c) {
     t.tx = sd.nbx * tsx(c);
     t.ty = sd.nby * tsy(c);
     return t;
-}
-
-__device__ __forceinline__ size_t tile_at(const TileGrid &t, int ex, int ey, int ez) {
-    return t.base + (size_t)ex + (size_t)t.tx * ((size_t)ey + (size_t)t.ty * (size_t)ez);
 }
 
 // floor(y * 2^32) of y in [0, 2^31) as 64 bits: the integer part is the
@@ -1123,7 +1112,6 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
         const TileGrid tg = tile_grid(sd, C);
         const int es = eS[C];
         float2 *tile = tiles + tile_at(tg, bxi * SX, byi * SY, bzi * SZ);
-        const uint32_t ry = (uint32_t)tg.tx, rz = (uint32_t)tg.tx * (uint32_t)tg.ty;
         for (int nd = t; nd < TN; nd += NT) {
             unsigned long long Sp = 0, Sn = 0, W = 0;
 #pragma unroll
@@ -1142,7 +1130,7 @@ __global__ __launch_bounds__(bscat::NT) void k_p2g_bscatter(
                 else Sf = (badb & BAD_PINF) ? INFINITY : -INFINITY;
             }
             const int tz = nd / (SX * SY), ty = (nd / SX) % SY, tx = nd % SX;
-            tile[(uint32_t)tx + ry * (uint32_t)ty + rz * (uint32_t)tz] = make_float2(Sf, Wf);
+            tile[tile_entry(tg, (uint32_t)tx, (uint32_t)ty, (uint32_t)tz)] = make_float2(Sf, Wf);
         }
     };
     flush(std::integral_constant<int, 0>());
