@@ -13,7 +13,9 @@
 //   2. k_sp_cells: one work-group per brick counts its cells in LDS, and
 //      writes each record to its cell at the rank of its index there; the
 //      512 cell starts go to a table (brick * 512 + cell, so a cell's end is
-//      the next entry).
+//      the next entry).  A brick of more than CAP points is only grouped by
+//      cell there; k_sp_rank gives its records their places, RANK_TILE of
+//      them per work-group.
 //   3. k_sp_gather: every node sums the records of its candidate cells, rows
 //      in (k, j) order, then cell order, then index order: a fixed order, so
 //      results are bit-identical run to run.  k_sp_gather_sparse does the
@@ -41,6 +43,8 @@ constexpr int SITEMS = 16;            // most points per thread there
 constexpr uint32_t kMaxBricks = 40000;   // histogram words that fit a CU's 160 KB of LDS
 constexpr uint32_t CAP = 6144;        // points of a brick ordered in LDS
 constexpr int CELLS = 512;            // cells of a brick
+constexpr uint32_t RANK_TILE = 256;   // points of a crowded brick that a work-group ranks
+constexpr size_t RANK_BLOCKS = 2048;  // its work-groups
 constexpr uint32_t kSparse = 2 * CELLS;   // most points of a brick for k_sp_gather_sparse
 
 struct SplatGrid {
@@ -86,8 +90,9 @@ __global__ __launch_bounds__(SNT) void k_sp_count(SplatGrid g, const float *__re
     }
 }
 
-// One work-group: first[b] (b = 0..nbrick+1), the placing cursors, and in
-// first[nbrick+2] the points of the fullest brick.
+// One work-group: first[b] (b = 0..nbrick+1), the placing cursors, in
+// first[nbrick+2] the points of the fullest brick, and in first[nbrick+3] the
+// count of k_sp_rank's tiles, cleared.
 __global__ __launch_bounds__(SNT) void k_sp_starts(uint32_t nbrick, const uint32_t *__restrict__ count,
                                                    uint32_t *__restrict__ first,
                                                    uint32_t *__restrict__ cursor) {
@@ -122,6 +127,7 @@ __global__ __launch_bounds__(SNT) void k_sp_starts(uint32_t nbrick, const uint32
     if (t == 0) {
         first[nbrick + 1] = at;
         first[nbrick + 2] = s_most;
+        first[nbrick + 3] = 0u;
     }
 }
 
@@ -165,11 +171,16 @@ __global__ __launch_bounds__(SNT) void k_sp_place(SplatGrid g, const float *__re
 
 // One work-group per brick: its records from rec (any order) to out (by
 // cell, then point index), and its cells' starts.  Ranks inside a cell come
-// from counting the cell's smaller indices, 8 at 8 points per cell.
+// from counting the cell's smaller indices, 8 at 8 points per cell.  A brick
+// of more than CAP points leaves that count, which grows as the square, to
+// k_sp_rank: its points grouped by cell (index and place in rec) in spill, and
+// their tiles appended to tiles (brick, tile), *ntile of them.
 __global__ __launch_bounds__(CELLS) void k_sp_cells(SplatGrid g, const uint32_t *__restrict__ first,
                                                      const float4 *__restrict__ rec,
                                                      const uint32_t *__restrict__ idx,
                                                      uint2 *__restrict__ spill,
+                                                     uint2 *__restrict__ tiles,
+                                                     uint32_t *__restrict__ ntile,
                                                      float4 *__restrict__ out,
                                                      uint32_t *__restrict__ start) {
     __shared__ uint32_t s_cell[CELLS + 1];    // points per cell, then the cell's first place
@@ -227,23 +238,49 @@ __global__ __launch_bounds__(CELLS) void k_sp_cells(SplatGrid g, const uint32_t 
         }
         return;
     }
-    // a crowded brick: the same with the groups in memory
     for (uint32_t e = t; e < N; e += CELLS) {
         const float4 r = rec[q0 + e];
         uint32_t cell;
         brick_of(g, r.x, r.y, r.z, cell);
         spill[q0 + atomicAdd(&s_cur[cell], 1u)] = make_uint2(idx[q0 + e], e);
     }
-    __syncthreads();   // (the groups are read back below)
-    for (uint32_t e = t; e < N; e += CELLS) {
-        const uint2 me = spill[q0 + e];
+    const uint32_t nt = (N + RANK_TILE - 1u) / RANK_TILE;
+    if (t == 0) s_wsum[0] = atomicAdd(ntile, nt);
+    __syncthreads();
+    for (uint32_t k = t; k < nt; k += CELLS) tiles[s_wsum[0] + k] = make_uint2(b, k);
+}
+
+// The records of the crowded bricks to their places, a tile of RANK_TILE
+// grouped points at a time (grid-stride over the tiles): as in k_sp_cells, a
+// point's rank is the number of smaller indices in its cell.  A cell's points
+// lie together, so a wave reads the same few words; a cell's tiles are spread
+// over the chip.  Whole calls on a 48^3 grid, R = dx, as measured with the
+// brick's one work-group ranking them / now: 1M points in one brick 329 / 8.2
+// ms (5 of it the gather of the crowded nodes, 0.3 this kernel), 0.2M 16.6 /
+// 1.6, 16 points in every cell 251 / 196 us, 32 573 / 371; 20 thousand points
+// in one cell 5.5 ms.
+__global__ __launch_bounds__(RANK_TILE) void k_sp_rank(SplatGrid g, const uint32_t *__restrict__ first,
+                                                       const uint32_t *__restrict__ start,
+                                                       const float4 *__restrict__ rec,
+                                                       const uint2 *__restrict__ spill,
+                                                       const uint2 *__restrict__ tiles,
+                                                       const uint32_t *__restrict__ ntile,
+                                                       float4 *__restrict__ out) {
+    const uint32_t nt = *ntile;
+    for (uint32_t n = blockIdx.x; n < nt; n += gridDim.x) {
+        const uint2 tile = tiles[n];
+        const uint32_t q0 = first[tile.x], q1 = first[tile.x + 1u];
+        const uint32_t p = q0 + tile.y * RANK_TILE + threadIdx.x;
+        if (p >= q1) continue;
+        const uint2 me = spill[p];
         const float4 r = rec[q0 + me.y];
         uint32_t cell;
-        brick_of(g, r.x, r.y, r.z, cell);
-        const uint32_t c0 = s_cell[cell], c1 = s_cell[cell + 1];
+        const uint32_t id = brick_of(g, r.x, r.y, r.z, cell) * (uint32_t)CELLS + cell;
+        const uint32_t c0 = start[id], c1 = start[id + 1u];
         uint32_t rank = 0;
-        for (uint32_t k = c0; k < c1; k++) rank += spill[q0 + k].x < me.x;
-        out[q0 + c0 + rank] = r;
+#pragma unroll 8
+        for (uint32_t k = c0; k < c1; k++) rank += spill[k].x < me.x;
+        out[c0 + rank] = r;
     }
 }
 
@@ -464,10 +501,17 @@ bool splat_by_brick(int64_t n, const BinGrid &bg, double reach) {
     return reach <= 4.0 && n < ((int64_t)1 << 31) && bricks(bg) < (int64_t)kMaxBricks;
 }
 
+// Most tiles of crowded bricks: a brick's last one may hold a single point,
+// but a crowded brick holds more than CAP.
+static size_t rank_tiles(int64_t n) {
+    return (size_t)n / RANK_TILE + (size_t)n / CAP + 1;
+}
+
 size_t splat_workspace(int64_t n, const BinGrid &bg) {
     const size_t nb = (size_t)bricks(bg);
-    // records twice, indices, crowded bricks' groups; counts, starts, cursors, cell starts
-    return (16 + 16 + 8 + 4) * (size_t)n + 3 * 4 * (nb + 3) + 4 * (nb * CELLS + 1) + 8 * 256;
+    // records twice, indices, crowded bricks' groups and tiles; counts, starts, cursors, cell starts
+    return (16 + 16 + 8 + 4) * (size_t)n + 8 * rank_tiles(n) + 3 * 4 * (nb + 4) +
+           4 * (nb * CELLS + 1) + 9 * 256;
 }
 
 void splat_run(void *work, const float *pos, const float *val, int64_t n, const BinGrid &bins,
@@ -487,9 +531,10 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
     const size_t nn = (size_t)n;
     float4 *rec = (float4 *)take(16 * nn), *out = (float4 *)take(16 * nn);
     uint2 *spill = (uint2 *)take(8 * nn);
+    uint2 *tiles = (uint2 *)take(8 * rank_tiles(n));
     uint32_t *idx = (uint32_t *)take(4 * nn);
     uint32_t *count = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
-    uint32_t *first = (uint32_t *)take(4 * (size_t)(g.nbrick + 3));
+    uint32_t *first = (uint32_t *)take(4 * (size_t)(g.nbrick + 4));
     uint32_t *cursor = (uint32_t *)take(4 * (size_t)(g.nbrick + 1));
     uint32_t *start = (uint32_t *)take(4 * ((size_t)g.nbrick * CELLS + 1));
     fill_u32(count, 0u, (int64_t)g.nbrick + 1, st);
@@ -508,8 +553,16 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
                        rec, idx);
     GFSX_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_sp_cells, dim3(g.nbrick), dim3(CELLS), 0, st, g, (const uint32_t *)first,
-                       (const float4 *)rec, (const uint32_t *)idx, spill, out, start);
+                       (const float4 *)rec, (const uint32_t *)idx, spill, tiles,
+                       first + g.nbrick + 3, out, start);
     GFSX_LAUNCH_CHECK();
+    if (n > (int64_t)CAP) {
+        hipLaunchKernelGGL(k_sp_rank, dim3((unsigned)std::min<size_t>(rank_tiles(n), RANK_BLOCKS)),
+                           dim3(RANK_TILE), 0, st, g, (const uint32_t *)first,
+                           (const uint32_t *)start, (const float4 *)rec, (const uint2 *)spill,
+                           (const uint2 *)tiles, (const uint32_t *)(first + g.nbrick + 3), out);
+        GFSX_LAUNCH_CHECK();
+    }
     const float inv_r2 = (float)(1.0 / (radius * radius));
     const int D = nodes.dhi[2] - nodes.dlo[2] + 1;
     auto *kern = D == 2   ? (val ? k_sp_gather<true, 2> : k_sp_gather<false, 2>)
