@@ -368,7 +368,7 @@ __global__ __launch_bounds__(kBlock) void k_pt_slow(PointJob j, const float4 *__
         const float x0[3] = {r.x, r.y, r.z};
         float k1[3], o[3], unused[3];
         sample_mac<ST, false>(j.g, nullptr, nullptr, nullptr, x0[0], x0[1], x0[2], k1, unused);
-        if (j.order > 0) {
+        if (ST == 0 || j.order > 0) {
             rk_step<ST>(j.g, j.order, j.c, x0, k1, o);
             store_point(j, r, o);
         } else {
@@ -442,12 +442,11 @@ void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int o
     GFSX_LAUNCH_CHECK();
     int e = 0;
     const bool p2 = std::frexp(g.inv_dx, &e) == 0.5 && e > -100 && e < 100;
-    const bool rk = order > 0;
-    auto *kern = stencil == 0
-        ? (rk ? (p2 ? k_pt_brick<0, true, true> : k_pt_brick<0, true, false>)
-              : (p2 ? k_pt_brick<0, false, true> : k_pt_brick<0, false, false>))
-        : (rk ? (p2 ? k_pt_brick<1, true, true> : k_pt_brick<1, true, false>)
-              : (p2 ? k_pt_brick<1, false, true> : k_pt_brick<1, false, false>));
+    // (a trilinear sample is not taken here: points_by_brick)
+    if (stencil == 0 && order == 0) throw Error("points_run: no trilinear sample by bricks");
+    auto *kern = stencil == 0 ? (p2 ? k_pt_brick<0, true, true> : k_pt_brick<0, true, false>)
+               : order > 0    ? (p2 ? k_pt_brick<1, true, true> : k_pt_brick<1, true, false>)
+                              : (p2 ? k_pt_brick<1, false, true> : k_pt_brick<1, false, false>);
     hipLaunchKernelGGL(kern, dim3((unsigned)(8 * ((nchunk + 7) / 8))), dim3(gbrick::NT), 0, s, pg, j,
                        (const float4 *)rec, (const uint4 *)chunks, slow, meta);
     GFSX_LAUNCH_CHECK();
