@@ -43,7 +43,7 @@ enum Slot {
     S_OLD0, S_XS0, S_XS1, S_XS2, S_VS0, S_VS1, S_VS2, S_DENSE, S_DENSEN,
     S_D_POS, S_D_VAL, S_D_S, S_D_W, S_D_U, S_D_V, S_D_WW, S_D_OUT,
     S_B_GRID, S_B_OLD, S_B_WGT, S_B_LG, S_B_XO, S_B_VO, S_B_FX, S_B_MAX, S_B_SLOW,
-    S_E_N, S_E_W, S_E_LAYER, S_E_LIST, S_E_OFF, S_E_BITS, S_R_KEEP, S_R_COUNT, S_R_DST, S_R_SCAN, S_R_N, S_R_FULL, S_R_NFULL,
+    S_E_N, S_E_W, S_E_LAYER, S_E_LIST, S_E_OFF, S_R_KEEP, S_R_COUNT, S_R_DST, S_R_SCAN, S_R_N, S_R_FULL, S_R_NFULL,
     S_P_TILE, S_P_TFLAG,
     S_K_COUNT, S_K_PSTART, S_K_RSTART, S_K_RUNREC, S_K_NRUNS, S_K_LIST, S_K_LIST2,
     S_K_RUNBASE, S_K_MID, S_K_HUGE, S_K_LCOUNT, S_K_SCAN, S_K_FLUID, S_K_SSLOT,
@@ -596,8 +596,11 @@ std::vector<gfsx::SceneDesc> flip_step_impl(gfsx_ctx *ctx, const gfsx_scene *sce
         epi.layer = (int8_t *)ctx->get(S_E_LAYER, (size_t)d.ni * d.nj * d.nk);
         epi.layers = params[0].extrapolation_layers > 0 ? params[0].extrapolation_layers : 7;
         const size_t nseg = gfsx::fs_segments(epi);
-        epi.fent = (uint16_t *)ctx->get(S_E_LIST, sizeof(uint16_t) * gfsx::fs_entries(epi));
-        epi.bits = (ulonglong2 *)ctx->get(S_E_BITS, sizeof(ulonglong2) * gfsx::fs_words(epi));
+        // the cell words are read before the face lists are written: one buffer
+        // (the lists are the larger where a row holds more than two cells)
+        epi.bits = (ulonglong2 *)ctx->get(S_E_LIST, std::max(sizeof(uint16_t) * gfsx::fs_entries(epi),
+                                                             sizeof(ulonglong2) * gfsx::fs_words(epi)));
+        epi.fent = (uint16_t *)epi.bits;
         epi.foff = (uint16_t *)ctx->get(S_E_OFF, sizeof(uint16_t) * nseg * (size_t)(epi.layers + 1));
         epi.dx = d.dx;
         epi.np = d.n;

@@ -318,7 +318,8 @@ struct FsEpilogue {
     // and layers + 1 offsets into it
     uint32_t nseg[3];
     uint16_t *fent, *foff;
-    ulonglong2 *bits;           // workspace: fs_words words (fluid, open) of 64 cells along x
+    ulonglong2 *bits;           // workspace: fs_words words (fluid, open) of 64 cells along x, in
+                                // fent's place (last read before fent is written)
 };
 
 // Particle removal (gfsx_remove.hip): positions/velocities in, kept ones
