@@ -400,7 +400,8 @@ __global__ __launch_bounds__(kBlock) void k_bin_starts(
         hi[e] = (uint32_t)(at >> 32);
         at += v[e];
     }
-    if (i + 4 <= m) {
+    // (a recorded step's pstart is the caller's array, on any 4-byte address)
+    if (i + 4 <= m && (reinterpret_cast<uintptr_t>(pstart) & 15u) == 0) {
         *reinterpret_cast<uint4 *>(pstart + i) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
         *reinterpret_cast<uint4 *>(rstart + i) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
     } else {
