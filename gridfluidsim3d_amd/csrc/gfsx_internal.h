@@ -442,14 +442,17 @@ void advect(const float *pos, int64_t n, const MacGrid &g, int order,
 // Where the line lies (us per call, direct / bricked, particles 8 per cell in
 // cell order, and shuffled): tricubic RK4 268k points 122 / 95 and 216 / 105
 // (131k: 74 / 83 and 85 / 89); tricubic sample 1M 69 / 74 and 204 / 87
-// (268k: 30 / 50 and 59 / 56); trilinear RK4 1M 58 / 73 and 196 / 85 (268k:
-// 20 / 52 and 54 / 60); a trilinear sample or a one- or two-sample step gains
-// only when shuffled (8M: 104 / 241 and 1260 / 458) and stays direct.  Below
+// (268k: 30 / 50 and 59 / 56); trilinear RK4 2.1M 125 / 93 and 399 / 123, RK3
+// 99 / 87 and 306 / 124 (RK4 1.06M: 52 / 84 and 208 / 94: only shuffled points
+// would gain); with steps of five cells, whose stages leave the boxes, RK4
+// 2.1M 106 / 123 and 384 / 164.  A trilinear sample or a one- or two-sample
+// step gains only when shuffled (8M: 104 / 241 and 1260 / 458) and stays
+// direct.  Below
 // about a hundred points per brick of the grid the histograms and the boxes
 // cost more than they save (256^3, 1M points spread over it, tricubic RK4:
 // 734 / 989).
 constexpr int64_t kPointsPerBrick = 96;
-constexpr int64_t kPointsMinLinear = (int64_t)1 << 20;
+constexpr int64_t kPointsMinLinear = (int64_t)1 << 21;
 constexpr int64_t kPointsMinCubicRk = 200000;
 constexpr int64_t kPointsMinCubic = (int64_t)1 << 19;
 bool points_by_brick(int64_t n, int ni, int nj, int nk, int order, int stencil);

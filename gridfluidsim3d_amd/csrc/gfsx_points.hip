@@ -19,8 +19,10 @@
 //      atomic per brick met reserving the work-group's range; the points are
 //      written there with their index (16 bytes each).
 //   4. k_pt_brick: one work-group per chunk stages the u, v, w boxes and
-//      samples them; a point with a stage that leaves the boxes, and the
-//      points of nearly empty chunks, go to a list.
+//      samples them.  A stage that leaves the boxes is sampled from global
+//      memory (trilinear), or its point goes to a list (tricubic: 192 loads
+//      in the kernel's loop would take its registers); so do the points of
+//      nearly empty chunks.
 //   5. k_pt_slow: the listed points, sampled from global memory.
 //
 // Bound: the tricubic brick kernel by LDS reads and VALU (64 taps and 84 FMAs
@@ -265,6 +267,10 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
     __shared__ uint32_t s_cell[CELLS];       // points per cell, then their first place
     __shared__ uint16_t s_ord[CHUNK];        // the chunk's points in cell order
     __shared__ uint32_t s_wsum[gbrick::NT / 64];
+    // the points to list, a bit each: a wave's 64 points of a pass share a word
+    constexpr int WORDS = (int)CHUNK / 64;
+    __shared__ uint64_t s_slow[ST == 0 ? 1 : WORDS];
+    __shared__ uint32_t s_slow_at[ST == 0 ? 1 : WORDS];
     const uint32_t nchunk = gld(meta, 0);
     const uint32_t per = (nchunk + 7u) / 8u;
     // consecutive bricks share box halos: keep them on one XCD
@@ -273,18 +279,14 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
     const uint4 ch = chunks[c];
     const int t = threadIdx.x, lane = t & 63;
     const bool outside = ch.x == pg.nbin - 1u;
-    // points for the global-memory pass: one atomic per wave
-    auto defer = [&](bool mine, uint32_t q) {
-        const uint64_t mk = __ballot(mine);
-        if (!mk) return;
-        const int lead = __ffsll((unsigned long long)mk) - 1;
-        uint32_t at = 0;
-        if (lane == lead) at = atomicAdd(&meta[1], (uint32_t)__popcll(mk));
-        at = __shfl(at, lead, 64);
-        if (mine) slow[at + (uint32_t)__popcll(mk & ((1ull << lane) - 1ull))] = q;
-    };
     if (ch.z < SPARSE && !outside) {
-        defer((uint32_t)t < ch.z, ch.y + (uint32_t)t);
+        static_assert(SPARSE <= 64, "one wave lists a sparse chunk");
+        if (t < 64) {
+            uint32_t at = 0;
+            if (t == 0) at = atomicAdd(&meta[1], ch.z);
+            at = __shfl(at, 0, 64);
+            if ((uint32_t)t < ch.z) slow[at + (uint32_t)t] = ch.y + (uint32_t)t;
+        }
         return;
     }
     const int gx = (int)(ch.x % (uint32_t)pg.gbx), gy = (int)(ch.x / (uint32_t)pg.gbx % (uint32_t)pg.gby),
@@ -301,6 +303,7 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
     static_assert(CELLS == 2 * gbrick::NT, "two cells per thread in the scan");
     s_cell[t] = 0u;
     s_cell[t + gbrick::NT] = 0u;
+    if (ST != 0 && t < WORDS) s_slow[t] = 0ull;
     __syncthreads();
     uint32_t cr[PER];   // cell << 16 | rank in it
 #pragma unroll
@@ -331,7 +334,11 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
     }
     __syncthreads();
     auto smp = [&](const float q[3], float out[3]) {
-        return box_sample<ST, B::E, P2>(j.g, s_box[0], s_box[1], s_box[2], lx, ly, lz, q, out);
+        const bool in = box_sample<ST, B::E, P2>(j.g, s_box[0], s_box[1], s_box[2], lx, ly, lz, q, out);
+        if (ST != 0 || in) return in;
+        float unused[3];
+        sample_mac<0, false>(j.g, nullptr, nullptr, nullptr, q[0], q[1], q[2], out, unused);
+        return true;
     };
     for (uint32_t e = (uint32_t)t; e < ch.z; e += gbrick::NT) {
         const uint32_t q = ch.y + s_ord[e];
@@ -347,7 +354,28 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
             for (int a = 0; a < 3; a++) o[a] = k1[a];
         }
         if (done) store_point(j, r, o);
-        defer(!done, q);
+        if (ST != 0) {
+            const uint64_t mk = __ballot(!done);
+            if (mk && lane == 0) s_slow[e >> 6] = mk;
+        }
+    }
+    if (ST == 0) return;
+    // the chunk's listed points: one atomic for all of them
+    __syncthreads();
+    if (t < 64) {
+        const uint32_t n = t < WORDS ? (uint32_t)__popcll(s_slow[t]) : 0u;
+        const uint32_t inc = wave_inclusive_sum(n), tot = __shfl(inc, 63, 64);
+        uint32_t at = 0;
+        if (tot && t == 0) at = atomicAdd(&meta[1], tot);
+        at = __shfl(at, 0, 64);
+        if (t < WORDS) s_slow_at[t] = at + inc - n;
+    }
+    __syncthreads();
+    for (int w = t >> 6; w < WORDS; w += gbrick::NT / 64) {
+        const uint64_t mk = s_slow[w];
+        if ((mk >> lane) & 1ull)
+            slow[s_slow_at[w] + (uint32_t)__popcll(mk & ((1ull << lane) - 1ull))] =
+                ch.y + s_ord[64 * w + lane];
     }
 }
 

@@ -1,4 +1,4 @@
-"""The trilinear Runge-Kutta steps by bricks (orders 3 and 4 from 2^20 points
+"""The trilinear Runge-Kutta steps by bricks (orders 3 and 4 from 2^21 points
 on), in FP64 cells as well as where 1/dx is a power of two, on either side of
 that line: the same bits as the direct kernels, which a call of few points
 takes."""
@@ -12,10 +12,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("order", [3, 4])
 @pytest.mark.parametrize("dims,dx,n,speed", [
-    ((40, 33, 27), 0.1, 1 << 20, 1.0),
-    ((40, 33, 27), 0.1, (1 << 20) - 1, 1.0),
-    ((40, 33, 27), 0.1, 1100003, 20.0),      # stages that leave the boxes
-    ((33, 40, 9), 0.125, 1 << 20, 2.0),
+    ((40, 33, 27), 0.1, 1 << 21, 1.0),
+    ((40, 33, 27), 0.1, (1 << 21) - 1, 1.0),
+    ((40, 33, 27), 0.1, 2100003, 20.0),      # stages that leave the boxes
+    ((33, 40, 9), 0.125, 1 << 21, 2.0),
 ])
 def test_linear_steps_same_bits_as_direct(ctx, dims, dx, n, speed, order):
     import torch
