@@ -220,9 +220,9 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect(StepAdjoint a) {
 // trilinear footprint holds the grid after the body force and the
 // normalised P2G result (0 for faces outside the arrays, which is what an
 // out-of-range sample reads).  A particle with a stage whose corners leave
-// the tile (it moved more than M cells) goes to a list, which k_adj_slow
-// takes through global memory, as it does the overflow bin (particles outside
-// the bin grid).
+// the tile (it moved more than M cells) takes that stage through global
+// memory.  k_adj_overflow takes the overflow bin (particles outside the bin
+// grid).
 //
 // Every sample's adjoint is computed, dL/dx and dL/dv are written, and
 // lam * weight is added as a 64-bit fixed-point integer, scale
@@ -246,7 +246,7 @@ constexpr int BX = 4, BY = 4, BZ = 4;   // the P2G bricks of the forward's brick
 constexpr int M = 1;
 constexpr int TX = BX + 2 + 2 * M, TY = BY + 2 + 2 * M, TZ = BZ + 2 + 2 * M;
 constexpr int TN = TX * TY * TZ;
-constexpr int SLOW_BLOCKS = 256;
+constexpr int OVERFLOW_BLOCKS = 64;
 }  // namespace abrick
 
 // An upper bound B on |lam| over every sample adjoint of adj_particle, from
@@ -293,6 +293,22 @@ __device__ __forceinline__ unsigned long long to_fixed(float v, double scale) {
     const double y = fma((double)v, scale, kMagic);
     return (unsigned long long)(__double_as_longlong(y) - __double_as_longlong(kMagic));
 }
+
+// Samples from global memory, adjoints added there in fixed point.
+struct GlobalFixed {
+    GlobalPolicy gp;
+    unsigned long long *fx;
+    double scale;
+    __device__ void sample(const float q[3], float out[3]) const { gp.sample(q, out); }
+    __device__ void adjoint(int base, const float q[3], const float lam[3], float lq[3]) const {
+        const StepAdjoint &a = gp.a;
+        mac_adjoint(a, base == 0 ? a.g : a.old, base, q, lam, lq,
+                    [&](int arr, int, int, int, uint32_t o, float v) {
+                        atomicAdd(fx + ((arr < 3 ? a.lg[arr] : a.ln[arr - 3]) - a.lg[0]) + o,
+                                  to_fixed(v, scale));
+                    });
+    }
+};
 
 // A stage position in a brick's tile: the lower corner of each component's
 // stencil (tile index) and the fractions along x, y, z, unshifted (a) and
@@ -443,49 +459,60 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         const float inv_dx = (float)a.mac.inv_dx;
         for (int c = 0; c < 3; c++) lq[c] += dt[c] * inv_dx;
     };
-    // the walk of adj_particle; false when a stage leaves the tile (nothing
-    // is added then)
-    auto particle = [&](const float x0[3], const float ax[3], const float av[3], float lx[3]) -> bool {
-        float k[3], q[3];
+    // the walk of adj_particle; a stage that leaves the tile goes through
+    // global memory
+    const GlobalFixed gfix{GlobalPolicy{a}, so.fx, scale};
+    auto particle = [&](const float x0[3], const float ax[3], const float av[3], float lx[3]) {
+        float k[3], q2[3], q3[3], q4[3];
         TileLoc p1, p2, p3, p4;
-        if (!locate(x0, p1)) return false;
-        sample(p1, k);
-        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_half * k[c];
-        if (!locate(q, p2)) return false;
-        sample(p2, k);
-        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_half * k[c];
-        if (!locate(q, p3)) return false;
-        sample(p3, k);
-        for (int c = 0; c < 3; c++) q[c] = x0[c] + a.h_full * k[c];
-        if (!locate(q, p4)) return false;
+        const bool t1 = locate(x0, p1);
+        if (t1) sample(p1, k);
+        else gfix.sample(x0, k);
+        for (int c = 0; c < 3; c++) q2[c] = x0[c] + a.h_half * k[c];
+        const bool t2 = locate(q2, p2);
+        if (t2) sample(p2, k);
+        else gfix.sample(q2, k);
+        for (int c = 0; c < 3; c++) q3[c] = x0[c] + a.h_half * k[c];
+        const bool t3 = locate(q3, p3);
+        if (t3) sample(p3, k);
+        else gfix.sample(q3, k);
+        for (int c = 0; c < 3; c++) q4[c] = x0[c] + a.h_full * k[c];
+        const bool t4 = locate(q4, p4);
         float lk[3], lq[3];
         for (int c = 0; c < 3; c++) {
             lx[c] = ax[c];
             lk[c] = a.h_sixth * ax[c];               // k4
             lq[c] = 0.0f;
         }
-        adjoint(0, p4, lk, lq);
+        if (t4) adjoint(0, p4, lk, lq);
+        else gfix.adjoint(0, q4, lk, lq);
         for (int c = 0; c < 3; c++) {
             lx[c] += lq[c];
             lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_full * lq[c];    // k3
             lq[c] = 0.0f;
         }
-        adjoint(0, p3, lk, lq);
+        if (t3) adjoint(0, p3, lk, lq);
+        else gfix.adjoint(0, q3, lk, lq);
         for (int c = 0; c < 3; c++) {
             lx[c] += lq[c];
             lk[c] = 2.0f * a.h_sixth * ax[c] + a.h_half * lq[c];    // k2
             lq[c] = 0.0f;
         }
-        adjoint(0, p2, lk, lq);
+        if (t2) adjoint(0, p2, lk, lq);
+        else gfix.adjoint(0, q2, lk, lq);
         float lgx[3], lnx[3];
         for (int c = 0; c < 3; c++) {
             lx[c] += lq[c];
             lgx[c] = a.h_sixth * ax[c] + a.h_half * lq[c] + (a.r_pic + a.r_flip) * av[c];
             lnx[c] = -a.r_flip * av[c];
         }
-        adjoint(0, p1, lgx, lx);
-        adjoint(3, p1, lnx, lx);
-        return true;
+        if (t1) {
+            adjoint(0, p1, lgx, lx);
+            adjoint(3, p1, lnx, lx);
+        } else {
+            gfix.adjoint(0, x0, lgx, lx);
+            gfix.adjoint(3, x0, lnx, lx);
+        }
     };
     // blocked mapping: thread t takes items [t*per, (t+1)*per), so the lanes
     // of a wave sit in different cells (fewer same-address LDS atomics)
@@ -499,13 +526,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
             ax[c] = a.ax[c][p];
             av[c] = a.av[c][p];
         }
-        if (particle(x0, ax, av, lx)) {
-            for (int c = 0; c < 3; c++) {
-                a.gx[c][p] = lx[c];
-                a.gv[c][p] = a.r_flip * av[c];
-            }
-        } else {
-            so.slow[atomicAdd(so.slow_count, 1u)] = q;
+        particle(x0, ax, av, lx);
+        for (int c = 0; c < 3; c++) {
+            a.gx[c][p] = lx[c];
+            a.gv[c][p] = a.r_flip * av[c];
         }
     }
     __syncthreads();
@@ -526,29 +550,12 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
     }
 }
 
-// The particles that k_adj_advect_brick left and the overflow bin's, through
-// global memory.
-struct GlobalFixed {
-    GlobalPolicy gp;
-    unsigned long long *fx;
-    double scale;
-    __device__ void sample(const float q[3], float out[3]) const { gp.sample(q, out); }
-    __device__ void adjoint(int base, const float q[3], const float lam[3], float lq[3]) const {
-        const StepAdjoint &a = gp.a;
-        mac_adjoint(a, base == 0 ? a.g : a.old, base, q, lam, lq,
-                    [&](int arr, int, int, int, uint32_t o, float v) {
-                        atomicAdd(fx + ((arr < 3 ? a.lg[arr] : a.ln[arr - 3]) - a.lg[0]) + o,
-                                  to_fixed(v, scale));
-                    });
-    }
-};
-
-__global__ __launch_bounds__(kBlock) void k_adj_slow(StepAdjoint a, AdjointSort so) {
+// The overflow bin's particles.
+__global__ __launch_bounds__(kBlock) void k_adj_overflow(StepAdjoint a, AdjointSort so) {
+    const uint32_t q0 = so.pstart[so.nbb], q1 = so.pstart[so.nbb + 1];
+    if (q0 == q1) return;
     const GlobalFixed pol{GlobalPolicy{a}, so.fx, fixed_scale(so.bound, a)};
-    const uint32_t ns = *so.slow_count;
-    const uint32_t o0 = so.pstart[so.nbb], no = so.pstart[so.nbb + 1] - o0;
-    for (uint32_t e = blockIdx.x * kBlock + threadIdx.x; e < ns + no; e += gridDim.x * kBlock) {
-        const uint32_t q = e < ns ? so.slow[e] : o0 + (e - ns);
+    for (uint32_t q = q0 + blockIdx.x * kBlock + threadIdx.x; q < q1; q += gridDim.x * kBlock) {
         const uint32_t p = so.perm[q];
         float x0[3], ax[3], av[3], lx[3];
         for (int c = 0; c < 3; c++) {
@@ -837,7 +844,7 @@ void flip_step_adjoint(const StepAdjoint &a, const AdjointSort *so, hipStream_t 
             a.ln[2] != a.ln[1] + nf[1])
             throw Error("flip_step_adjoint: grid adjoint arrays must be contiguous");
         fill_u32((uint32_t *)so->fx, 0u, 4 * tot, s);
-        fill_u32(so->bound, 0u, 4, s);   // slow_count too
+        fill_u32(so->bound, 0u, 3, s);
         // the fixed-point scale's bound, then one work-group per bin of the
         // brick sort
         hipLaunchKernelGGL(k_adj_bound, dim3((unsigned)std::min<int64_t>(
@@ -848,7 +855,7 @@ void flip_step_adjoint(const StepAdjoint &a, const AdjointSort *so, hipStream_t 
             const uint32_t nbrick = so->nbb;
             hipLaunchKernelGGL(k_adj_advect_brick, dim3(nbrick), dim3(kBlock), 0, s, a, *so);
             GFSX_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_adj_slow, dim3(abrick::SLOW_BLOCKS), dim3(kBlock), 0, s, a, *so);
+            hipLaunchKernelGGL(k_adj_overflow, dim3(abrick::OVERFLOW_BLOCKS), dim3(kBlock), 0, s, a, *so);
             GFSX_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(k_fixed_to_coeffs, dim3(blocks_for(tot)), dim3(kBlock), 0, s,

@@ -42,7 +42,7 @@ enum Slot {
     S_BOUT, S_BOUTS, S_SCAN, S_OCT, S_POCT,
     S_OLD0, S_XS0, S_XS1, S_XS2, S_VS0, S_VS1, S_VS2, S_DENSE, S_DENSEN,
     S_D_POS, S_D_VAL, S_D_S, S_D_W, S_D_U, S_D_V, S_D_WW, S_D_OUT,
-    S_B_GRID, S_B_OLD, S_B_WGT, S_B_LG, S_B_XO, S_B_VO, S_B_FX, S_B_MAX, S_B_SLOW,
+    S_B_GRID, S_B_OLD, S_B_WGT, S_B_LG, S_B_XO, S_B_VO, S_B_FX, S_B_MAX,
     S_E_N, S_E_W, S_E_LAYER, S_E_LIST, S_E_OFF, S_R_KEEP, S_R_COUNT, S_R_DST, S_R_SCAN, S_R_N, S_R_FULL, S_R_NFULL,
     S_P_TILE, S_P_TFLAG,
     S_K_COUNT, S_K_PSTART, S_K_RSTART, S_K_RUNREC, S_K_NRUNS, S_K_LIST, S_K_LIST2,
@@ -796,9 +796,7 @@ void run_adjoint(gfsx_ctx *ctx, const gfsx_scene *sc, const gfsx_step_params *pr
     // fixed-point sums into the P2G adjoint's two factors in it in one pass)
     float *lg = ctx->f32(S_B_LG, 2 * tot), *ln = lg + tot;
     so.fx = (unsigned long long *)ctx->get(S_B_FX, sizeof(unsigned long long) * 2 * (size_t)tot);
-    so.bound = ctx->u32(S_B_MAX, 4);
-    so.slow = ctx->u32(S_B_SLOW, sc->n);
-    so.slow_count = so.bound + 3;
+    so.bound = ctx->u32(S_B_MAX, 3);
     const float *g[3] = {grids.u, grids.v, grids.w};
     const float *old[3] = {grids.u_old, grids.v_old, grids.w_old};
     const float *wgt[3] = {grids.wu, grids.wv, grids.ww};

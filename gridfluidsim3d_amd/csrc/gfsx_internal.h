@@ -274,9 +274,7 @@ struct StepAdjoint {
 // perm maps a slot to its input index.  fx: fixed-point accumulators for
 // the grid adjoints (int64, the face arrays of dL/dg u,v,w then dL/dn u,v,w
 // back to back); bound: three words for the fixed-point scale's bound
-// (max |dL/dx'|, max |dL/dv'|, max |g|, float bits); slow: slots of particles
-// left to the global-memory kernel (at most n), slow_count their number, the
-// word after bound's three.
+// (max |dL/dx'|, max |dL/dv'|, max |g|, float bits).
 struct AdjointSort {
     const uint32_t *pstart, *perm;
     const float *xs[3];
@@ -284,7 +282,6 @@ struct AdjointSort {
     int gbx, gby;
     unsigned long long *fx;
     uint32_t *bound;
-    uint32_t *slow, *slow_count;
 };
 
 // FluidSimulation's face fill and extrapolation around the transfer (one
