@@ -442,14 +442,18 @@ void advect(const float *pos, int64_t n, const MacGrid &g, int order,
 // (268k: 30 / 50 and 59 / 56); trilinear RK4 2.1M 125 / 93 and 399 / 123, RK3
 // 99 / 87 and 306 / 124 (RK4 1.06M: 52 / 84 and 208 / 94: only shuffled points
 // would gain); with steps of five cells, whose stages leave the boxes, RK4
-// 2.1M 106 / 123 and 384 / 164.  A trilinear sample or a one- or two-sample
-// step gains only when shuffled (8M: 104 / 241 and 1260 / 458) and stays
-// direct.  Below
+// 2.1M 106 / 123 and 384 / 164.  Where the points lie unevenly the bricks do
+// less for trilinear steps: 2.3M on 100^3, a tenth of them spread over it and
+// the rest in a sixth of it, in cell order RK4 148 / 147, RK3 115 / 134 (hence
+// its own line); 2.2M on 200x100x100, 520 a brick, 148 / 165 and 113 / 150.  A
+// trilinear sample or a one- or two-sample step gains only when shuffled (8M:
+// 104 / 241 and 1260 / 458) and stays direct.  Below
 // about a hundred points per brick of the grid the histograms and the boxes
 // cost more than they save (256^3, 1M points spread over it, tricubic RK4:
 // 734 / 989).
 constexpr int64_t kPointsPerBrick = 96;
-constexpr int64_t kPointsMinLinear = (int64_t)1 << 21;
+constexpr int64_t kPointsPerBrickLinear = 1024;
+constexpr int64_t kPointsMinLinear = (int64_t)1 << 21;   // RK4; twice for RK3
 constexpr int64_t kPointsMinCubicRk = 200000;
 constexpr int64_t kPointsMinCubic = (int64_t)1 << 19;
 bool points_by_brick(int64_t n, int ni, int nj, int nk, int order, int stencil);

@@ -14,16 +14,17 @@
 //      (one word per brick), added to the global counts with one atomic per
 //      brick the work-group met.
 //   2. k_pt_scan: brick starts, and the work list: bricks cut into chunks of
-//      at most CHUNK points.
+//      at most CHUNK points.  Bricks of fewer than SPARSE points are in no
+//      chunk; their points lie together behind all others.
 //   3. k_pt_place: the histogram again, each point's rank in it kept, one
 //      atomic per brick met reserving the work-group's range; the points are
 //      written there with their index (16 bytes each).
 //   4. k_pt_brick: one work-group per chunk stages the u, v, w boxes and
 //      samples them.  A stage that leaves the boxes is sampled from global
 //      memory (trilinear), or its point goes to a list (tricubic: 192 loads
-//      in the kernel's loop would take its registers); so do the points of
-//      nearly empty chunks.
-//   5. k_pt_slow: the listed points, sampled from global memory.
+//      in the kernel's loop would take its registers).
+//   5. k_pt_slow: the listed points and the sparse bricks', sampled from
+//      global memory.
 //
 // Bound: the tricubic brick kernel by LDS reads and VALU (64 taps and 84 FMAs
 // a component), the passes around it by memory (12 B read twice, 16 B written
@@ -45,7 +46,7 @@ namespace {
 constexpr int PNT = 1024;            // threads of the count and place kernels
 constexpr int PITEMS = 16;           // most points per thread there
 constexpr uint32_t CHUNK = 2048;     // most points of one brick work-group
-constexpr uint32_t SPARSE = 32;      // chunks below this size are not staged
+constexpr uint32_t SPARSE = 32;      // bricks below this size are not staged
 constexpr int SLOW_BLOCKS = 1024;
 constexpr uint32_t kMaxBins = 40000; // histogram words that fit a CU's 160 KB of LDS
 
@@ -94,37 +95,45 @@ __global__ __launch_bounds__(PNT) void k_pt_count(PointGrid g, const float *__re
     }
 }
 
-// One work-group: cursor[b] = first slot of bin b, and the chunk list
-// (bin, first slot, points); meta[0] = chunks, meta[1] (the slow list's
-// count) = 0.
-__global__ __launch_bounds__(PNT) void k_pt_scan(uint32_t nbin, const uint32_t *__restrict__ count,
+// One work-group: cursor[b] = first slot of bin b, the sparse ones' from the
+// end of the n points down, and the chunk list (bin, first slot, points);
+// meta[0] = chunks, meta[1] (the slow list's count) = 0, meta[2] = points of
+// the sparse bins.
+__global__ __launch_bounds__(PNT) void k_pt_scan(uint32_t nbin, uint32_t n,
+                                                 const uint32_t *__restrict__ count,
                                                  uint32_t *__restrict__ cursor,
                                                  uint4 *__restrict__ chunks,
                                                  uint32_t *__restrict__ meta) {
-    __shared__ uint32_t s_p[PNT / 64], s_c[PNT / 64];
+    __shared__ uint32_t s_p[PNT / 64], s_c[PNT / 64], s_s[PNT / 64];
     const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-    uint32_t p0 = 0, c0 = 0;
+    uint32_t p0 = 0, c0 = 0, s0 = 0;
     for (uint32_t b0 = 0; b0 < nbin; b0 += PNT) {
         const uint32_t b = b0 + (uint32_t)t;
-        const uint32_t np = b < nbin ? count[b] : 0u;
+        const uint32_t all = b < nbin ? count[b] : 0u;
+        const bool sparse = all < SPARSE && b != nbin - 1u;
+        const uint32_t np = sparse ? 0u : all, ns = sparse ? all : 0u;
         const uint32_t nc = (np + CHUNK - 1u) / CHUNK;
-        const uint32_t ip = wave_inclusive_sum(np), ic = wave_inclusive_sum(nc);
+        const uint32_t ip = wave_inclusive_sum(np), ic = wave_inclusive_sum(nc),
+                       is = wave_inclusive_sum(ns);
         if (lane == 63) {
             s_p[wid] = ip;
             s_c[wid] = ic;
+            s_s[wid] = is;
         }
         __syncthreads();
-        uint32_t ps = p0 + ip - np, cs = c0 + ic - nc, pt = 0, ct = 0;
+        uint32_t ps = p0 + ip - np, cs = c0 + ic - nc, ss = s0 + is, pt = 0, ct = 0, st = 0;
         for (int w = 0; w < PNT / 64; w++) {
-            const uint32_t a = s_p[w], c = s_c[w];
+            const uint32_t a = s_p[w], c = s_c[w], d = s_s[w];
             if (w < wid) {
                 ps += a;
                 cs += c;
+                ss += d;
             }
             pt += a;
             ct += c;
+            st += d;
         }
-        if (b < nbin) cursor[b] = ps;
+        if (b < nbin) cursor[b] = sparse ? n - ss : ps;
         // equal shares of the bin's points
         for (uint32_t k = 0; k < nc; k++) {
             const uint32_t f = (uint32_t)((uint64_t)np * k / nc), e = (uint32_t)((uint64_t)np * (k + 1) / nc);
@@ -132,11 +141,13 @@ __global__ __launch_bounds__(PNT) void k_pt_scan(uint32_t nbin, const uint32_t *
         }
         p0 += pt;
         c0 += ct;
+        s0 += st;
         __syncthreads();
     }
     if (t == 0) {
         meta[0] = c0;
         meta[1] = 0u;
+        meta[2] = s0;
     }
 }
 
@@ -279,16 +290,6 @@ __device__ __forceinline__ void point_brick(const PointGrid &pg, const PointJob 
     const uint4 ch = chunks[c];
     const int t = threadIdx.x, lane = t & 63;
     const bool outside = ch.x == pg.nbin - 1u;
-    if (ch.z < SPARSE && !outside) {
-        static_assert(SPARSE <= 64, "one wave lists a sparse chunk");
-        if (t < 64) {
-            uint32_t at = 0;
-            if (t == 0) at = atomicAdd(&meta[1], ch.z);
-            at = __shfl(at, 0, 64);
-            if ((uint32_t)t < ch.z) slow[at + (uint32_t)t] = ch.y + (uint32_t)t;
-        }
-        return;
-    }
     const int gx = (int)(ch.x % (uint32_t)pg.gbx), gy = (int)(ch.x / (uint32_t)pg.gbx % (uint32_t)pg.gby),
               gz = (int)(ch.x / ((uint32_t)pg.gbx * (uint32_t)pg.gby));
     const int lx = 8 * gx - B::LO, ly = 8 * gy - B::LO, lz = 8 * gz - B::LO;
@@ -387,12 +388,13 @@ __global__ __launch_bounds__(gbrick::NT, ST == 0 ? 6 : 4) void k_pt_brick(
 }
 
 template <int ST>
-__global__ __launch_bounds__(kBlock) void k_pt_slow(PointJob j, const float4 *__restrict__ rec,
+__global__ __launch_bounds__(kBlock) void k_pt_slow(PointJob j, uint32_t n,
+                                                   const float4 *__restrict__ rec,
                                                    const uint32_t *__restrict__ slow,
                                                    const uint32_t *__restrict__ meta) {
-    const uint32_t ns = meta[1];
-    for (uint32_t e = blockIdx.x * kBlock + threadIdx.x; e < ns; e += gridDim.x * kBlock) {
-        const float4 r = rec[slow[e]];
+    const uint32_t ns = meta[1], all = ns + meta[2];
+    for (uint32_t e = blockIdx.x * kBlock + threadIdx.x; e < all; e += gridDim.x * kBlock) {
+        const float4 r = rec[e < ns ? slow[e] : n - (all - e)];
         const float x0[3] = {r.x, r.y, r.z};
         float k1[3], o[3], unused[3];
         sample_mac<ST, false>(j.g, nullptr, nullptr, nullptr, x0[0], x0[1], x0[2], k1, unused);
@@ -416,7 +418,9 @@ bool points_by_brick(int64_t n, int ni, int nj, int nk, int order, int stencil) 
     const int64_t bins = points_bins(ni, nj, nk);
     if (bins > (int64_t)kMaxBins || n >= ((int64_t)1 << 31) || n < kPointsPerBrick * (bins - 1))
         return false;
-    if (stencil == 0) return order >= 3 && n >= kPointsMinLinear;
+    if (stencil == 0)
+        return order >= 3 && n >= (order == 3 ? 2 : 1) * kPointsMinLinear &&
+               n >= kPointsPerBrickLinear * (bins - 1);
     return n >= (order >= 2 ? kPointsMinCubicRk : kPointsMinCubic);
 }
 
@@ -448,7 +452,7 @@ void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int o
     uint32_t *slow = (uint32_t *)take(4 * (size_t)n);
     uint32_t *count = (uint32_t *)take(4 * (size_t)pg.nbin);
     uint32_t *cursor = (uint32_t *)take(4 * (size_t)pg.nbin);
-    uint32_t *meta = (uint32_t *)take(8);
+    uint32_t *meta = (uint32_t *)take(12);
     PointJob j;
     j.g = g;
     j.c = rk_consts(dt);
@@ -463,8 +467,8 @@ void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int o
     const size_t lds = 4 * (size_t)pg.nbin;
     hipLaunchKernelGGL(k_pt_count, dim3(nblk), dim3(PNT), lds, s, pg, pos, n, items, count);
     GFSX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_pt_scan, dim3(1), dim3(PNT), 0, s, pg.nbin, (const uint32_t *)count, cursor,
-                       chunks, meta);
+    hipLaunchKernelGGL(k_pt_scan, dim3(1), dim3(PNT), 0, s, pg.nbin, (uint32_t)n,
+                       (const uint32_t *)count, cursor, chunks, meta);
     GFSX_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_pt_place, dim3(nblk), dim3(PNT), lds, s, pg, pos, n, items, cursor, rec);
     GFSX_LAUNCH_CHECK();
@@ -479,8 +483,8 @@ void points_run(void *work, const float *pos, int64_t n, const MacGrid &g, int o
                        (const float4 *)rec, (const uint4 *)chunks, slow, meta);
     GFSX_LAUNCH_CHECK();
     auto *slowk = stencil == 0 ? k_pt_slow<0> : k_pt_slow<1>;
-    hipLaunchKernelGGL(slowk, dim3(SLOW_BLOCKS), dim3(kBlock), 0, s, j, (const float4 *)rec,
-                       (const uint32_t *)slow, (const uint32_t *)meta);
+    hipLaunchKernelGGL(slowk, dim3(SLOW_BLOCKS), dim3(kBlock), 0, s, j, (uint32_t)n,
+                       (const float4 *)rec, (const uint32_t *)slow, (const uint32_t *)meta);
     GFSX_LAUNCH_CHECK();
 }
 

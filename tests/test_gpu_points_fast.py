@@ -19,7 +19,7 @@ def flow(dims, dx, cells):
 
 
 @pytest.mark.parametrize("cells", [1.0, 2.0, 3.5, 6.0])
-@pytest.mark.parametrize("stencil,n", [(0, 1 << 21), (1, 300001)])
+@pytest.mark.parametrize("stencil,n", [(0, 1 << 22), (1, 300001)])
 def test_stages_outside_the_boxes_same_bits(ctx, stencil, n, cells):
     import torch
     dims, dx = (33, 40, 30), 0.1
