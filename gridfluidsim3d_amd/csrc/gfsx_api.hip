@@ -415,7 +415,7 @@ void p2g_device_impl(gfsx_ctx *c, const float *pos, const float *val,
     bg.inv_dx = 1.0 / dx;
     bg.nbin = (uint32_t)nbin;
     ng.dx_f = (float)dx;
-    if (gfsx::splat_by_brick(n, bg, r)) {
+    if (gfsx::splat_by_brick(n, bg, r, (int64_t)ni * nj * nk)) {
         gfsx::splat_run(c->get(S_SPLAT, gfsx::splat_workspace(n, bg)), pos, val, n, bg, ng, radius,
                         dx, S, W, c->stream);
         return;

@@ -414,10 +414,10 @@ void p2g_gather(const float *aos, const float *val, int64_t n,
                 hipStream_t s);
 
 // The same sums over points sorted by bricks of 8^3 bin cells in LDS
-// (gfsx_splat.hip), for bin grids of fewer than 40000 bricks and radii of up
-// to 4 cells (reach = radius / dx); work holds splat_workspace bytes of
-// device memory.
-bool splat_by_brick(int64_t n, const BinGrid &bins, double reach);
+// (gfsx_splat.hip; the same bits), for bin grids of fewer than 40000 bricks,
+// radii of up to 4 cells (reach = radius / dx) and, with radii of up to one on
+// large grids, not too few points for the nnode nodes; work holds splat_workspace bytes of device memory.
+bool splat_by_brick(int64_t n, const BinGrid &bins, double reach, int64_t nnode);
 size_t splat_workspace(int64_t n, const BinGrid &bins);
 void splat_run(void *work, const float *pos, const float *val, int64_t n, const BinGrid &bins,
                const NodeGrid &nodes, double radius, double dx, float *S, float *W,

@@ -284,6 +284,26 @@ __global__ __launch_bounds__(RANK_TILE) void k_sp_rank(SplatGrid g, const uint32
     }
 }
 
+// A record's terms of one node: K (and K val) at squared distance dxy + vz^2,
+// dxy = vx^2 + vy^2.  The roundings are written out, so that a node's sums do
+// not depend on which gather takes it; they are those of the cell sort's
+// gather.  in false: the record adds nothing.
+__device__ __forceinline__ float square_xy(float vx, float vy) { return fmaf(vx, vx, vy * vy); }
+
+template <bool HAS_VAL>
+__device__ __forceinline__ void add_record(float dxy, float vz, float inv_r2, float val, bool in,
+                                           float &s, float &w) {
+    const float d2 = fmaf(vz, vz, dxy);
+    const float b = fmaxf(fmaf(-d2, inv_r2, 1.0f), 0.0f);
+    const float a = in ? b : 0.0f, a2 = a * a;
+    const float q = fmaf(4.0f / 9.0f, a, 5.0f / 9.0f);
+    // only inside the radius (scalarfield.cpp:191-196): a value that is not
+    // finite must not reach the nodes beyond it
+    if (HAS_VAL) s = fmaf(a2 * q, in && d2 * inv_r2 < 1.0f ? val : 0.0f, s);
+    else s = fmaf(a2, q, s);
+    w = fmaf(a2, q, w);
+}
+
 // One thread per column of kseg nodes along z.  A node's candidate cells
 // along an axis are D consecutive ones (dhi - dlo + 1), so the cells of one
 // plane reach D nodes of the column: the thread walks the planes upwards,
@@ -292,7 +312,8 @@ __global__ __launch_bounds__(RANK_TILE) void k_sp_rank(SplatGrid g, const uint32
 // plane - dhi + m.  A node's own terms still come plane by plane, row by row
 // and in cell order.  A row's cells are one range per brick they lie in; two
 // records are loaded ahead of the sums, and one past the range adds K = 0.
-template <bool HAS_VAL, int D>
+// COLUMN false: kseg is 1, one slot.
+template <bool HAS_VAL, int D, bool COLUMN>
 __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, double dx,
                                                       float inv_r2, int kseg,
                                                       const uint32_t *__restrict__ most,
@@ -313,14 +334,15 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, 
     const int ilo = max(i + ng.dlo[0], 0), ihi = min(i + ng.dhi[0], g.bg.b[0] - 1);
     const int jlo = max(j + ng.dlo[1], 0), jhi = min(j + ng.dhi[1], g.bg.b[1] - 1);
     const size_t stride = (size_t)ng.n[0] * ng.n[1];
-    float s[D], w[D], gz[D];
+    constexpr int M = COLUMN ? D : 1;
+    float s[M], w[M], gz[M];
 #pragma unroll
-    for (int m = 0; m < D; m++) s[m] = w[m] = 0.0f;
+    for (int m = 0; m < M; m++) s[m] = w[m] = 0.0f;
     for (int bk = k0 + ng.dlo[2]; bk <= k1 - 1 + ng.dhi[2]; bk++) {
-        const int kk = bk - ng.dhi[2];   // the node of slot 0
+        const int kk = COLUMN ? bk - ng.dhi[2] : k0;   // the node of slot 0
         if (bk >= 0 && bk < g.bg.b[2]) {
 #pragma unroll
-            for (int m = 0; m < D; m++) gz[m] = (float)((float)(kk + m) * dx);
+            for (int m = 0; m < M; m++) gz[m] = (float)((float)(kk + m) * dx);
             for (int bj = jlo; bj <= jhi; bj++) {
                 const uint32_t row = (uint32_t)g.gb[0] *
                                      ((uint32_t)(bj >> 3) + (uint32_t)g.gb[1] * (uint32_t)(bk >> 3));
@@ -339,22 +361,13 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, 
                             const float vx = gx - (r[u].x - ng.off[0]);
                             const float vy = gy - (r[u].y - ng.off[1]);
                             const float pz = r[u].z - ng.off[2];
-                            const float dxy = vx * vx + vy * vy;
+                            const float dxy = square_xy(vx, vy);
                             const bool in = q + (uint32_t)u < q1;
 #pragma unroll
-                            for (int m = 0; m < D; m++) {
+                            for (int m = 0; m < M; m++) {
                                 // (the same for all lanes)
-                                if (kk + m < k0 || kk + m >= k1) continue;
-                                const float vz = gz[m] - pz;
-                                const float d2 = dxy + vz * vz;
-                                const float t = in ? d2 * inv_r2 : 1.0f;
-                                const float K = wyvill(t);
-                                // only inside the radius (scalarfield.cpp:191-196):
-                                // a value that is not finite must not reach the
-                                // nodes beyond it
-                                if (HAS_VAL) s[m] = fmaf(K, t < 1.0f ? r[u].w : 0.0f, s[m]);
-                                else s[m] += K;
-                                w[m] += K;
+                                if (COLUMN && (kk + m < k0 || kk + m >= k1)) continue;
+                                add_record<HAS_VAL>(dxy, gz[m] - pz, inv_r2, r[u].w, in, s[m], w[m]);
                             }
                         }
                     }
@@ -364,17 +377,17 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, 
         }
         // the node of slot 0 has all its planes: accumulate into the caller's
         // arrays (clscalarfield.cpp:1448-1449)
-        if (kk >= k0) {
+        if (COLUMN ? kk >= k0 : bk == k0 + ng.dhi[2]) {
             const size_t f = (size_t)col + stride * (size_t)kk;
             S[f] += s[0];
             if (W) W[f] += w[0];
         }
 #pragma unroll
-        for (int m = 0; m + 1 < D; m++) {
+        for (int m = 0; m + 1 < M; m++) {
             s[m] = s[m + 1];
             w[m] = w[m + 1];
         }
-        s[D - 1] = w[D - 1] = 0.0f;
+        if (COLUMN) s[M - 1] = w[M - 1] = 0.0f;
     }
 }
 
@@ -390,7 +403,7 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather(SplatGrid g, NodeGrid ng, 
 // and 8 points per cell, R = dx: 189/177, 282/277, 266/284, 670/888 us; R = 2.5
 // dx: 750/524, 1189/1005, 1611/2129, 3981/8717 us.  Hence kSparse, two points
 // per cell in the fullest brick.
-template <bool HAS_VAL, int D>
+template <bool HAS_VAL, int D, bool COLUMN>
 __global__ __launch_bounds__(kBlock) void k_sp_gather_sparse(SplatGrid g, NodeGrid ng, double dx,
                                                       float inv_r2, int kseg,
                                                       const uint32_t *__restrict__ most,
@@ -412,14 +425,15 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather_sparse(SplatGrid g, NodeGr
     const int ilo = max(i + ng.dlo[0], 0), ihi = min(i + ng.dhi[0], g.bg.b[0] - 1);
     const int jlo = max(j + ng.dlo[1], 0), jhi = min(j + ng.dhi[1], g.bg.b[1] - 1);
     const size_t stride = (size_t)ng.n[0] * ng.n[1];
-    float s[D], w[D], gz[D];
+    constexpr int M = COLUMN ? D : 1;
+    float s[M], w[M], gz[M];
 #pragma unroll
-    for (int m = 0; m < D; m++) s[m] = w[m] = 0.0f;
+    for (int m = 0; m < M; m++) s[m] = w[m] = 0.0f;
     for (int bk = k0 + ng.dlo[2]; bk <= k1 - 1 + ng.dhi[2]; bk++) {
-        const int kk = bk - ng.dhi[2];   // the node of slot 0
+        const int kk = COLUMN ? bk - ng.dhi[2] : k0;   // the node of slot 0
         if (bk >= 0 && bk < g.bg.b[2]) {
 #pragma unroll
-            for (int m = 0; m < D; m++) gz[m] = (float)((float)(kk + m) * dx);
+            for (int m = 0; m < M; m++) gz[m] = (float)((float)(kk + m) * dx);
             // the plane's ranges of records, every start loaded before any is used
             uint32_t q0[2 * D], q1[2 * D];
 #pragma unroll
@@ -457,17 +471,11 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather_sparse(SplatGrid g, NodeGr
                 const float vx = gx - (r.x - ng.off[0]);
                 const float vy = gy - (r.y - ng.off[1]);
                 const float pz = r.z - ng.off[2];
-                const float dxy = vx * vx + vy * vy;
+                const float dxy = square_xy(vx, vy);
 #pragma unroll
-                for (int m = 0; m < D; m++) {
-                    if (kk + m < k0 || kk + m >= k1) continue;
-                    const float vz = gz[m] - pz;
-                    const float d2 = dxy + vz * vz;
-                    const float t = d2 * inv_r2;
-                    const float K = wyvill(t);
-                    if (HAS_VAL) s[m] = fmaf(K, t < 1.0f ? r.w : 0.0f, s[m]);
-                    else s[m] += K;
-                    w[m] += K;
+                for (int m = 0; m < M; m++) {
+                    if (COLUMN && (kk + m < k0 || kk + m >= k1)) continue;
+                    add_record<HAS_VAL>(dxy, gz[m] - pz, inv_r2, r.w, true, s[m], w[m]);
                 }
                 r = rn;
                 live = more;
@@ -475,18 +483,30 @@ __global__ __launch_bounds__(kBlock) void k_sp_gather_sparse(SplatGrid g, NodeGr
         }
         // the node of slot 0 has all its planes: accumulate into the caller's
         // arrays (clscalarfield.cpp:1448-1449)
-        if (kk >= k0) {
+        if (COLUMN ? kk >= k0 : bk == k0 + ng.dhi[2]) {
             const size_t f = (size_t)col + stride * (size_t)kk;
             S[f] += s[0];
             if (W) W[f] += w[0];
         }
 #pragma unroll
-        for (int m = 0; m + 1 < D; m++) {
+        for (int m = 0; m + 1 < M; m++) {
             s[m] = s[m + 1];
             w[m] = w[m + 1];
         }
-        s[D - 1] = w[D - 1] = 0.0f;
+        if (COLUMN) s[M - 1] = w[M - 1] = 0.0f;
     }
+}
+
+using Gather = void (*)(SplatGrid, NodeGrid, double, float, int, const uint32_t *, const uint32_t *,
+                        const float4 *, float *, float *);
+
+template <int D>
+Gather gather_kernel(bool val, bool column, bool sparse) {
+    if (sparse)
+        return column ? (val ? k_sp_gather_sparse<true, D, true> : k_sp_gather_sparse<false, D, true>)
+                      : (val ? k_sp_gather_sparse<true, D, false> : k_sp_gather_sparse<false, D, false>);
+    return column ? (val ? k_sp_gather<true, D, true> : k_sp_gather<false, D, true>)
+                  : (val ? k_sp_gather<true, D, false> : k_sp_gather<false, D, false>);
 }
 
 int64_t bricks(const BinGrid &bg) {
@@ -497,8 +517,14 @@ int64_t bricks(const BinGrid &bg) {
 
 }  // namespace
 
-bool splat_by_brick(int64_t n, const BinGrid &bg, double reach) {
-    return reach <= 4.0 && n < ((int64_t)1 << 31) && bricks(bg) < (int64_t)kMaxBricks;
+// The gather of few points with a radius of one cell on a large grid is short,
+// and the bricks' passes before it take longer than the cell sort's.  Cell sort /
+// bricks, us per call, R = dx: 128^3 nodes, 3 thousand points 73 / 59, 100
+// thousand 93 / 77; 160^3 89 / 90, 117 / 120; 200^3 122 / 124, 160 / 191, 250
+// thousand 192 / 190; R = 1.7 dx: 200^3 191 / 172 and 300 / 238.
+bool splat_by_brick(int64_t n, const BinGrid &bg, double reach, int64_t nnode) {
+    const int64_t few = reach <= 1.0 && nnode > ((int64_t)3 << 20) ? nnode / 32 : 0;
+    return reach <= 4.0 && n >= few && n < ((int64_t)1 << 31) && bricks(bg) < (int64_t)kMaxBricks;
 }
 
 // Most tiles of crowded bricks: a brick's last one may hold a single point,
@@ -564,15 +590,6 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
         GFSX_LAUNCH_CHECK();
     }
     const float inv_r2 = (float)(1.0 / (radius * radius));
-    const int D = nodes.dhi[2] - nodes.dlo[2] + 1;
-    auto *kern = D == 2   ? (val ? k_sp_gather<true, 2> : k_sp_gather<false, 2>)
-                 : D == 4 ? (val ? k_sp_gather<true, 4> : k_sp_gather<false, 4>)
-                 : D == 6 ? (val ? k_sp_gather<true, 6> : k_sp_gather<false, 6>)
-                          : (val ? k_sp_gather<true, 8> : k_sp_gather<false, 8>);
-    auto *sparse = D == 2   ? (val ? k_sp_gather_sparse<true, 2> : k_sp_gather_sparse<false, 2>)
-                   : D == 4 ? (val ? k_sp_gather_sparse<true, 4> : k_sp_gather_sparse<false, 4>)
-                   : D == 6 ? (val ? k_sp_gather_sparse<true, 6> : k_sp_gather_sparse<false, 6>)
-                            : (val ? k_sp_gather_sparse<true, 8> : k_sp_gather_sparse<false, 8>);
     // Columns of 1 to 16 nodes, about 8192 waves of them (and no more
     // segments than a grid's y extent holds): longer columns read less,
     // shorter ones fill the chip.  0.27M nodes, columns of 1 / 4: 22 / 52 us
@@ -581,12 +598,31 @@ void splat_run(void *work, const float *pos, const float *val, int64_t n, const 
     const int kseg = (int)std::max<int64_t>(
         std::min<int64_t>(std::max<int64_t>(nnode / (64 * 8192), 1), 16), nodes.n[2] / 65535 + 1);
     const dim3 grid(grid_for((int64_t)nodes.n[0] * nodes.n[1], kBlock), grid_for(nodes.n[2], kseg));
+    const int D = nodes.dhi[2] - nodes.dlo[2] + 1;
+    const Gather kern = D == 2   ? gather_kernel<2>(val, kseg > 1, false)
+                        : D == 4 ? gather_kernel<4>(val, kseg > 1, false)
+                        : D == 6 ? gather_kernel<6>(val, kseg > 1, false)
+                                 : gather_kernel<8>(val, kseg > 1, false);
+    // The sparse gather's starts cost it more than its sums: past a radius of
+    // one cell, columns of up to 3 nodes where the above gives fewer, and with
+    // few points for the nodes 2048 waves of them.  100^3 nodes, columns of 1 / 3
+    // / 7, us per call: R = 4 dx, 100 points 188 / 110 / 91, 62 thousand evenly
+    // spread 243 / 151 / 128, in a ball 321 / 288 / 373; R = 1.7 dx 89 / 73 / 76
+    // and 89 / 88 / 115; R = dx (128^3, columns of 4 / 8, 30 thousand) 75 / 87.
+    const bool few = 32 * n < nnode;
+    const int ksp = D == 2 ? kseg : (int)std::max<int64_t>(
+        kseg, std::min<int64_t>(nnode / (64 * (few ? 2048 : 4096)), few ? 16 : 3));
+    const Gather sparse = D == 2   ? gather_kernel<2>(val, ksp > 1, true)
+                          : D == 4 ? gather_kernel<4>(val, ksp > 1, true)
+                          : D == 6 ? gather_kernel<6>(val, ksp > 1, true)
+                                   : gather_kernel<8>(val, ksp > 1, true);
     // the fullest brick, known on the device, decides which of the two works;
     // where the points' mean exceeds the line the rows do it anyway (3.85M
     // points in 3315 bricks: an empty launch saved)
     const uint32_t *most = n <= (int64_t)kSparse * g.nbrick ? first + g.nbrick + 2 : nullptr;
     if (most) {
-        hipLaunchKernelGGL(sparse, grid, dim3(kBlock), 0, st, g, nodes, dx, inv_r2, kseg, most,
+        hipLaunchKernelGGL(sparse, dim3(grid.x, grid_for(nodes.n[2], ksp)), dim3(kBlock), 0, st, g,
+                           nodes, dx, inv_r2, ksp, most,
                            (const uint32_t *)start, (const float4 *)out, S, W);
         GFSX_LAUNCH_CHECK();
     }
