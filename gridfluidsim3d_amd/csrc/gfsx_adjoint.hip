@@ -221,8 +221,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect(StepAdjoint a) {
 // normalised P2G result (0 for faces outside the arrays, which is what an
 // out-of-range sample reads).  A particle with a stage whose corners leave
 // the tile (it moved more than M cells) takes that stage through global
-// memory.  k_adj_overflow takes the overflow bin (particles outside the bin
-// grid).
+// memory.  Work-groups past the bricks take the particles of the overflow bin
+// (outside the bin grid; a launch of their own costs 5 us).
 //
 // Every sample's adjoint is computed, dL/dx and dL/dv are written, and
 // lam * weight is added as a 64-bit fixed-point integer, scale
@@ -246,7 +246,7 @@ constexpr int BX = 4, BY = 4, BZ = 4;   // the P2G bricks of the forward's brick
 constexpr int M = 1;
 constexpr int TX = BX + 2 + 2 * M, TY = BY + 2 + 2 * M, TZ = BZ + 2 + 2 * M;
 constexpr int TN = TX * TY * TZ;
-constexpr int OVERFLOW_BLOCKS = 64;
+constexpr int NEXTRA = 16;
 }  // namespace abrick
 
 // An upper bound B on |lam| over every sample adjoint of adj_particle, from
@@ -326,9 +326,28 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
     const int tid = threadIdx.x;
     const uint32_t bid = blockIdx.x;
     // brick bid: bin bid of the sort, one contiguous range of slots
-    const uint32_t q0 = so.pstart[bid], total = so.pstart[bid + 1] - q0;
+    const uint32_t bin = min(bid, so.nbb);
+    const uint32_t q0 = so.pstart[bin], total = so.pstart[bin + 1] - q0;
     if (total == 0) return;   // uniform across the work-group
     const double scale = fixed_scale(so.bound, a);
+    const GlobalFixed gfix{GlobalPolicy{a}, so.fx, scale};
+    if (bid >= so.nbb) {
+        for (uint32_t e = (bid - so.nbb) * kBlock + tid; e < total; e += NEXTRA * kBlock) {
+            const uint32_t q = q0 + e, p = so.perm[q];
+            float x0[3], ax[3], av[3], lx[3];
+            for (int c = 0; c < 3; c++) {
+                x0[c] = so.xs[c][q];
+                ax[c] = a.ax[c][p];
+                av[c] = a.av[c][p];
+            }
+            adj_particle(a, x0, ax, av, lx, gfix);
+            for (int c = 0; c < 3; c++) {
+                a.gx[c][p] = lx[c];
+                a.gv[c][p] = a.r_flip * av[c];
+            }
+        }
+        return;
+    }
     const uint32_t g = bid >> 3, sub = bid & 7u;
     const int bx = (int)(2 * (g % (uint32_t)so.gbx) + (sub & 1u));
     const int by = (int)(2 * ((g / (uint32_t)so.gbx) % (uint32_t)so.gby) + ((sub >> 1) & 1u));
@@ -461,7 +480,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
     };
     // the walk of adj_particle; a stage that leaves the tile goes through
     // global memory
-    const GlobalFixed gfix{GlobalPolicy{a}, so.fx, scale};
     auto particle = [&](const float x0[3], const float ax[3], const float av[3], float lx[3]) {
         float k[3], q2[3], q3[3], q4[3];
         TileLoc p1, p2, p3, p4;
@@ -547,27 +565,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_advect_brick(StepAdjoint a, Adjo
         const float *base = c == 0 ? (arr < 3 ? a.lg[0] : a.ln[0])
                           : c == 1 ? (arr < 3 ? a.lg[1] : a.ln[1]) : (arr < 3 ? a.lg[2] : a.ln[2]);
         atomicAdd(so.fx + (base - a.lg[0]) + o, v);
-    }
-}
-
-// The overflow bin's particles.
-__global__ __launch_bounds__(kBlock) void k_adj_overflow(StepAdjoint a, AdjointSort so) {
-    const uint32_t q0 = so.pstart[so.nbb], q1 = so.pstart[so.nbb + 1];
-    if (q0 == q1) return;
-    const GlobalFixed pol{GlobalPolicy{a}, so.fx, fixed_scale(so.bound, a)};
-    for (uint32_t q = q0 + blockIdx.x * kBlock + threadIdx.x; q < q1; q += gridDim.x * kBlock) {
-        const uint32_t p = so.perm[q];
-        float x0[3], ax[3], av[3], lx[3];
-        for (int c = 0; c < 3; c++) {
-            x0[c] = so.xs[c][q];
-            ax[c] = a.ax[c][p];
-            av[c] = a.av[c][p];
-        }
-        adj_particle(a, x0, ax, av, lx, pol);
-        for (int c = 0; c < 3; c++) {
-            a.gx[c][p] = lx[c];
-            a.gv[c][p] = a.r_flip * av[c];
-        }
     }
 }
 
@@ -664,7 +661,8 @@ __global__ __launch_bounds__(kBlock) void k_face_coeffs(StepAdjoint a, FaceCount
 // floor(s) + 1, 2x2x2 candidates per component; the kernel's support
 // decides which of them take weight.  The offsets and their squares are
 // formed once per axis and the two faces of a row read together (2M
-// particles: 74 us with a loop over the faces, 57 now; VALU bound).
+// particles in cell order: 74 us with a loop over the faces, 59 now; VALU
+// bound).
 //
 // The roundings are written out: near t = 1 the slope of K over its value
 // grows without bound, a face that took little weight has a large A, and
@@ -725,7 +723,14 @@ __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
         for (int k = 0; k < 2; k++)
 #pragma unroll
             for (int j = 0; j < 2; j++) {
-                float af[2], bf[2];
+                float t[2], af[2], bf[2];
+#pragma unroll
+                for (int i = 0; i < 2; i++)
+                    t[i] = rounded_product(dist2(d[0][i], q[1][j], q[2][k]), a.inv_r2);
+                // rows outside the radius are not read: where the particles
+                // come in no order the reads bound it (1M shuffled: 160 us with
+                // every row, 118 without)
+                if (!(t[0] < 1.0f) && !(t[1] < 1.0f)) continue;
                 if (all) {
                     const uint32_t f = (uint32_t)lo[0] + (uint32_t)dims[0] *
                         ((uint32_t)(lo[1] + j) + (uint32_t)dims[1] * (uint32_t)(lo[2] + k));
@@ -749,13 +754,13 @@ __global__ __launch_bounds__(kBlock) void k_adj_p2g_step(StepAdjoint a) {
                 }
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    const float t = rounded_product(dist2(d[0][i], q[1][j], q[2][k]), a.inv_r2);
                     // only inside the radius: a factor or a velocity that is
                     // not finite must not reach past it
-                    const bool on = t < 1.0f;
-                    lv[c] = fmaf(wyvill(t), on ? af[i] : 0.0f, lv[c]);
+                    const bool on = t[i] < 1.0f;
+                    lv[c] = fmaf(wyvill(t[i]), on ? af[i] : 0.0f, lv[c]);
                     // d(d2)/dx_p = -2 (g - p); lam (v_p - n_f) / W_f = v_p A - B
-                    const float slope = fmaf(vp[c], af[i], -bf[i]) * wyvill_dt(t) * a.inv_r2 * -2.0f;
+                    const float slope =
+                        fmaf(vp[c], af[i], -bf[i]) * wyvill_dt(t[i]) * a.inv_r2 * -2.0f;
                     const float coef = on ? slope : 0.0f;
                     lx[0] = fmaf(coef, d[0][i], lx[0]);
                     lx[1] = fmaf(coef, d[1][j], lx[1]);
@@ -853,9 +858,8 @@ void flip_step_adjoint(const StepAdjoint &a, const AdjointSort *so, hipStream_t 
         GFSX_LAUNCH_CHECK();
         if (a.n > 0) {
             const uint32_t nbrick = so->nbb;
-            hipLaunchKernelGGL(k_adj_advect_brick, dim3(nbrick), dim3(kBlock), 0, s, a, *so);
-            GFSX_LAUNCH_CHECK();
-            hipLaunchKernelGGL(k_adj_overflow, dim3(abrick::OVERFLOW_BLOCKS), dim3(kBlock), 0, s, a, *so);
+            hipLaunchKernelGGL(k_adj_advect_brick, dim3(nbrick + abrick::NEXTRA), dim3(kBlock), 0, s,
+                               a, *so);
             GFSX_LAUNCH_CHECK();
         }
         hipLaunchKernelGGL(k_fixed_to_coeffs, dim3(blocks_for(tot)), dim3(kBlock), 0, s,
