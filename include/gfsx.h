@@ -78,6 +78,8 @@ const char *gfsx_get_device_info(gfsx_ctx *ctx, int *err);
  * clscalarfield.cpp:68-122, scalarfield.cl:79-138).  Accumulates into S/W
  * like the reference (clscalarfield.cpp:1448-1449); the sum for each node is
  * taken in a fixed order, so results are bit-identical run to run.
+ * The context keeps the sort's workspace (23 to 45 bytes a point and up to
+ * 12 a node), sized by its largest call so far.
  * Replaces CLScalarField::addPointValues (clscalarfield.cpp:143-301). */
 void gfsx_p2g(gfsx_ctx *ctx, const float *pos, const float *val, int64_t n,
               double radius, const float offset[3], double dx, int ni, int nj,
@@ -98,6 +100,14 @@ void gfsx_apply_weight_device(gfsx_ctx *ctx, float *S, const float *W,
  * dx) at pos[p]; (0,0,0) outside [0,ni*dx)x[0,nj*dx)x[0,nk*dx); NaN/Inf
  * results are zeroed (particleadvector.cpp:1139-1149).  out may alias pos
  * (the reference's in-place overload, particleadvector.cpp:457-465).
+ * Large device calls (from 200 thousand points on, a hundred or more per
+ * 8^3 cells) sort the points by brick of the grid in a workspace that the
+ * context keeps (20 bytes a point), here and in gfsx_advect_device: the first
+ * one allocates it, and one of more points than any before it waits for the
+ * call before to finish and allocates it anew, so a program that must do
+ * neither in its loop makes one call of its largest size beforehand.  Calls
+ * being captured into a graph, and calls for which there is no memory, sample
+ * straight from the grid: the same bits, no workspace.
  * Replaces ParticleAdvector::tricubicInterpolate (particleadvector.cpp:
  * 401-455). */
 void gfsx_g2p(gfsx_ctx *ctx, const float *pos, int64_t n, const float *u,
